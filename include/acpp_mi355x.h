@@ -429,7 +429,8 @@ acpp_status acpp_transform_exclusive_scan_f64(acpp_allocation_group *scratch, ac
 
 /* Histogram: bins[keys[i]] += 1 for every keys[i] < num_bins (other keys are
    ignored); the counts are added to the existing bin values.  The
-   privatized strategy supports up to 65536 bins. */
+   privatized strategy supports up to 65536 bins; the automatic choice
+   privatizes up to 2^22. */
 acpp_status acpp_histogram_u32(acpp_allocation_group *scratch, acpp_stream_t stream, const uint32_t *keys, uint64_t n, uint32_t *bins, uint32_t num_bins, int strategy, const acpp_launch_config *config);
 
 /* Strided fetch ops: target[i % num_slots] = op(target[i % num_slots], values[i]). */

@@ -10,15 +10,15 @@
 //
 // MI355X design:
 //   - strategy "privatized": every work-group keeps private counters in LDS
-//     and only the group totals reach global memory.  Up to 32768 bins the
-//     counters are 32-bit; up to 65536 bins two 16-bit counters share one
-//     32-bit LDS word (65536 bins = 128 KiB of the 160 KiB LDS).  A 16-bit
-//     counter that reaches 0x8000 is drained by the one work-item that saw
-//     it cross: it subtracts 0x8000 in LDS and adds 0x8000 to the global
-//     bin, so a field never carries into its neighbour.  Group totals are
-//     written as per-group partial histograms (coalesced, no atomics) and a
-//     second kernel adds their column sums to the bins, which keeps global
-//     atomics off the hot path entirely.
+//     and only the group totals reach global memory.  Up to 8192 bins the
+//     counters are 32-bit; above, two 16-bit counters share one 32-bit LDS
+//     word (65536 bins = 128 KiB of the 160 KiB LDS).  A 16-bit counter that
+//     has reached 0x8000 is drained by the one work-item that clears its top
+//     bit: it adds 0x8000 to the global bin, so a field never carries into
+//     its neighbour.  Up to 2^22 bins are cut into slices, one per group.
+//     Group totals go straight to the bins where that takes few atomics, else
+//     they are written as per-group partial histograms (coalesced, no
+//     atomics) and a second kernel adds their column sums to the bins;
 //   - keys are streamed with 128-bit loads, several per work-item in flight;
 //   - strided fetch_min / fetch_max / fetch_add (slot = i mod num_slots):
 //     the grid is sized so that num_slots divides the grid stride whenever
@@ -28,6 +28,8 @@
 //     tracked incrementally;
 //   - strategy "global": one device-scope atomic per element, the
 //     reference's pattern, kept for comparison.
+#include <algorithm>
+#include <cmath>
 #include <numeric>
 
 #include "launch_util.hpp"
@@ -69,47 +71,170 @@ __device__ __forceinline__ uint64_t scalar_index(const geom &g, uint64_t s) {
 // --------------------------------------------------------------------------
 // Histogram
 // --------------------------------------------------------------------------
-// copies_log2 (32-bit counters only): the group keeps 2^copies_log2 copies
-// of the histogram, word (bin << copies_log2) + copy, and work-item t counts
-// into copy t mod 2^copies_log2.  Lanes that meet the same hot bin then hit
-// adjacent words in different banks instead of one address.
-template <bool PACKED, bool GLOBAL, int UNROLL>
-__global__ __launch_bounds__(1024) void histogram_kernel(const uint32_t *__restrict__ keys,
-                                                         geom gm, uint32_t num_bins,
-                                                         uint32_t *partials, uint32_t *bins,
-                                                         uint32_t copies_log2) {
-  extern __shared__ uint32_t lds[];
-  const uint32_t my_copy = threadIdx.x & ((1u << copies_log2) - 1u);
-  // Packed counters: bin b < half in the low 16 bits of word b, bin
-  // half + b in the high 16 bits, so the low (under skewed keys, hot) bins
-  // sit in consecutive words and banks; adjacent bins sharing a word put
-  // the two hottest Zipf bins on one address.
-  const uint32_t half = (num_bins + 1) / 2;
-  if constexpr (!GLOBAL) {
-    const uint32_t words = PACKED ? half : (num_bins << copies_log2);
-    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) lds[i] = 0;
-    __syncthreads();
-  }
+struct hist_params {
+  const uint32_t *keys;
+  geom gm;
+  uint32_t *bins;
+  uint32_t num_bins;
+  uint32_t local_bins;   // bins of one slice (num_bins without slices)
+  uint32_t slices_log2;  // SLICED: 2^slices_log2 slices of the bins
+  uint32_t copies_log2;  // 32-bit counters: LDS copies of the histogram
+  uint32_t chunks;       // work-groups per slice; each takes one part of the keys
+  int xcd_map;           // SLICED: a chunk's slices share an XCD
+  uint32_t *partials;    // NULL: the counts go straight to the bins
+};
 
-  auto count = [&](uint32_t k) {
-    if (k >= num_bins) return;
-    if constexpr (GLOBAL) {
-      __hip_atomic_fetch_add(&bins[k], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else if constexpr (PACKED) {
-      const bool hi = k >= half;
-      const uint32_t word = hi ? k - half : k;
-      const uint32_t shift = hi ? 16u : 0u;
-      const uint32_t old = atomicAdd(&lds[word], 1u << shift);
-      if (((old >> shift) & 0xffffu) == 0x7fffu) {
-        // This work-item moved the field to 0x8000: drain it.
-        atomicAdd(&lds[word], 0u - (0x8000u << shift));
-        __hip_atomic_fetch_add(&bins[k], 0x8000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A slice holds the bins k with (k ^ (k >> s)) mod 2^s == slice, as its
+// local bins k >> s (s = slices_log2): hot neighbouring bins, and bins a power
+// of two apart, fall into different slices.
+__device__ __forceinline__ uint32_t slice_bin(uint32_t local, uint32_t slice, uint32_t s) {
+  return (local << s) | ((local ^ slice) & ((1u << s) - 1u));
+}
+
+// 32-bit counters: the group keeps 2^copies_log2 copies of the histogram,
+// word (bin << copies_log2) + copy, and work-item t counts into copy
+// t mod 2^copies_log2.  Lanes that meet the same hot bin then hit adjacent
+// words in different banks instead of one address.
+//
+// PACKED: bin b < half in the low 16 bits of word b, bin half + b in the
+// high 16 bits, so the low (under skewed keys, hot) bins sit in consecutive
+// words and banks; adjacent bins sharing a word put the two hottest Zipf
+// bins on one address.
+//
+// SLICED (packed, more than 65536 bins): every group counts the keys of one
+// slice of the bins and skips the others, so each key is read once per slice,
+// but only once from memory: the groups of one part of the keys run on one
+// XCD and meet in its L2.  Bound by the instructions per visited key (four
+// keys per clock and CU).  One device atomic per key, the form before,
+// serialises on hot bins and reaches 26 G keys/s on uniform ones: 2^25
+// Zipf(1.1) keys into 200,000 bins 48.7 ms -> 76 us, 2^24 uniform keys
+// 640 -> 48 us, 2^25 Zipf keys into 1,000,000 bins 46 ms -> 249 us.  (32-bit
+// counters without a returned value, in twice the slices: 120 and 399 us.)
+template <bool PACKED, bool SLICED, int UNROLL>
+__global__ __launch_bounds__(1024) void histogram_kernel(hist_params p) {
+  static_assert(PACKED || !SLICED, "slices use packed counters");
+  extern __shared__ uint32_t lds[];
+  const uint32_t my_copy = threadIdx.x & ((1u << p.copies_log2) - 1u);
+  const uint32_t half = (p.local_bins + 1) / 2;
+  const uint32_t s = p.slices_log2;
+  const uint32_t mask = (1u << s) - 1u;
+  uint32_t slice = 0, chunk = blockIdx.x;
+  if constexpr (SLICED) {
+    // Work-groups go to the eight XCDs in turn.
+    const uint32_t i = p.xcd_map ? blockIdx.x >> 3 : blockIdx.x;
+    slice = i & mask;
+    chunk = p.xcd_map ? ((i >> s) << 3) + (blockIdx.x & 7u) : i >> s;
+  }
+  const uint32_t slice_top = SLICED ? slice << (32 - s) : 0;
+  // the slice's local bins: the last one only if its bin exists
+  const uint32_t slice_end =
+      SLICED ? p.local_bins - (slice_bin(p.local_bins - 1, slice, s) >= p.num_bins ? 1u : 0u) : p.num_bins;
+  auto bin_of = [&](uint32_t local) { return SLICED ? slice_bin(local, slice, s) : local; };
+  auto add_bin = [&](uint32_t b, uint32_t v) {
+    if (v && b < p.num_bins) __hip_atomic_fetch_add(&p.bins[b], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const uint32_t words = PACKED ? half : (p.num_bins << p.copies_log2);
+  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) lds[i] = 0;
+  __syncthreads();
+
+  // The counts of a batch of keys: all LDS atomics are issued before the
+  // first returned word is looked at.
+  auto count = [&](const uint32_t *k, auto m_tag) {
+    constexpr int M = decltype(m_tag)::value;
+    if constexpr (PACKED) {
+      uint32_t word[M], old[M];
+      uint32_t any = 0;
+#pragma unroll
+      for (int j = 0; j < M; ++j) {
+        // the slice in the top s bits, the local bin below
+        const uint32_t l = SLICED ? __builtin_amdgcn_alignbit(k[j] ^ (k[j] >> s), k[j], s) - slice_top : k[j];
+        word[j] = min(l, l - half);  // l - half wraps for the low bins
+        old[j] = 0;
+        if (l < slice_end) old[j] = atomicAdd(&lds[word[j]], l < half ? 1u : 0x10000u);
+        any |= old[j];
+      }
+      if (any & 0x80008000u) {
+        // A field had reached 0x8000 before the add: whoever clears its top
+        // bit adds 0x8000 to the bin.  The field cannot carry before that: no
+        // work-item adds more than M times without looking.
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+          if (!(old[j] & 0x80008000u)) continue;
+          const uint32_t full = atomicAnd(&lds[word[j]], 0x7fff7fffu);
+          if (full & 0x8000u) add_bin(bin_of(word[j]), 0x8000u);
+          if (full & 0x80000000u) add_bin(bin_of(word[j] + half), 0x8000u);
+        }
       }
     } else {
-      atomicAdd(&lds[(k << copies_log2) + my_copy], 1u);
+#pragma unroll
+      for (int j = 0; j < M; ++j)
+        if (k[j] < p.num_bins) atomicAdd(&lds[(k[j] << p.copies_log2) + my_copy], 1u);
     }
   };
 
+  const uint64_t stride = static_cast<uint64_t>(p.chunks) * blockDim.x;
+  const uint64_t gtid = static_cast<uint64_t>(chunk) * blockDim.x + threadIdx.x;
+  const u32x4 *kv = reinterpret_cast<const u32x4 *>(p.keys + p.gm.head);
+  uint64_t c = gtid;
+  for (; c + (UNROLL - 1) * stride < p.gm.nvec; c += UNROLL * stride) {
+    u32x4 q[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) q[u] = SLICED ? kv[c + u * stride] : __builtin_nontemporal_load(kv + c + u * stride);
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      uint32_t k[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+      count(k, std::integral_constant<int, 4>{});
+    }
+  }
+  for (; c < p.gm.nvec; c += stride) {
+    const u32x4 q = kv[c];
+    uint32_t k[4] = {q.x, q.y, q.z, q.w};
+    count(k, std::integral_constant<int, 4>{});
+  }
+  for (uint64_t i = gtid; i < p.gm.nscalar; i += stride) {
+    const uint32_t k = p.keys[scalar_index(p.gm, i)];
+    count(&k, std::integral_constant<int, 1>{});
+  }
+
+  __syncthreads();
+  // Groups that add to the same bins start at different ones.
+  auto rotated = [&](uint32_t i, uint32_t count) {
+    const uint32_t first = static_cast<uint32_t>(static_cast<uint64_t>(count) * chunk / p.chunks) & ~63u;
+    return i + first < count ? i + first : i + first - count;
+  };
+  if constexpr (PACKED) {
+    uint32_t *mine = p.partials + (static_cast<uint64_t>(slice) * p.chunks + chunk) * half;
+    for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) {
+      if (p.partials) {
+        mine[i] = lds[i];  // both counters of the word
+      } else {
+        const uint32_t w = rotated(i, half);
+        const uint32_t v = lds[w];
+        add_bin(bin_of(w), v & 0xffffu);
+        add_bin(bin_of(w + half), v >> 16);
+      }
+    }
+  } else {
+    uint32_t *mine = p.partials + static_cast<uint64_t>(blockIdx.x) * p.num_bins;
+    for (uint32_t i = threadIdx.x; i < p.num_bins; i += blockDim.x) {
+      const uint32_t b = p.partials ? i : rotated(i, p.num_bins);
+      uint32_t v = 0;
+      for (uint32_t c = 0; c < (1u << p.copies_log2); ++c) v += lds[(b << p.copies_log2) + c];
+      if (p.partials)
+        mine[b] = v;
+      else
+        add_bin(b, v);
+    }
+  }
+}
+
+// One device-scope atomic per key (the reference's pattern).
+template <int UNROLL>
+__global__ __launch_bounds__(1024) void histogram_global_kernel(const uint32_t *__restrict__ keys, geom gm,
+                                                                uint32_t num_bins, uint32_t *bins) {
+  auto count = [&](uint32_t k) {
+    if (k < num_bins) __hip_atomic_fetch_add(&bins[k], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   const uint64_t gtid = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const u32x4 *kv = reinterpret_cast<const u32x4 *>(keys + gm.head);
@@ -134,35 +259,57 @@ __global__ __launch_bounds__(1024) void histogram_kernel(const uint32_t *__restr
     count(q.w);
   }
   for (uint64_t s = gtid; s < gm.nscalar; s += stride) count(keys[scalar_index(gm, s)]);
-
-  if constexpr (!GLOBAL) {
-    __syncthreads();
-    // Partial histogram of this group (coalesced, no atomics).
-    uint32_t *mine = partials + static_cast<uint64_t>(blockIdx.x) * num_bins;
-    for (uint32_t b = threadIdx.x; b < num_bins; b += blockDim.x) {
-      uint32_t v;
-      if constexpr (PACKED) {
-        v = (b >= half) ? (lds[b - half] >> 16) : (lds[b] & 0xffffu);
-      } else {
-        v = 0;
-        for (uint32_t c = 0; c < (1u << copies_log2); ++c) v += lds[(b << copies_log2) + c];
-      }
-      mine[b] = v;
-    }
-  }
 }
 
-// bins[b] += sum over groups of partials[g][b].  blockIdx.y takes every
-// gridDim.y-th group, so the partials are read by many work-groups at once;
-// the per-chunk sums are added with device-scope integer atomics (exact, so
-// the order does not matter).
-__global__ void histogram_combine_kernel(const uint32_t *__restrict__ partials, uint32_t groups,
-                                         uint32_t num_bins, uint32_t *bins) {
-  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= num_bins) return;
-  uint32_t s = 0;
-  for (uint32_t g = blockIdx.y; g < groups; g += gridDim.y) s += partials[static_cast<uint64_t>(g) * num_bins + b];
-  if (s) __hip_atomic_fetch_add(&bins[b], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// bins[b] += sum over groups of the partial counts.  A work-group sums `span`
+// words of every slice over its chunks (blockIdx.y takes every gridDim.y-th
+// chunk, so the partials are read by many work-groups at once) and puts the
+// bins' sums in order in LDS: neighbouring bins come from different slices,
+// and the atomics on the bins are coalesced this way.  Integer atomics: the
+// order does not matter.  PACKED partials are the words of the LDS, 16 bits
+// a counter.
+constexpr uint32_t combine_entries = 4096;  // span << slices_log2 at most
+__host__ __device__ constexpr uint32_t combine_span_log2(uint32_t slices_log2) {
+  return slices_log2 <= 4 ? 8u : 12u - slices_log2;
+}
+template <bool PACKED>
+__global__ __launch_bounds__(256) void histogram_combine_kernel(hist_params p) {
+  __shared__ uint32_t s_low[combine_entries];
+  __shared__ uint32_t s_high[PACKED ? combine_entries : 1];
+  const uint32_t s = p.slices_log2;
+  const uint32_t mask = (1u << s) - 1u;
+  const uint32_t span_log2 = combine_span_log2(s);
+  const uint32_t half = (p.local_bins + 1) / 2;
+  const uint32_t words = PACKED ? half : p.num_bins;
+  const uint32_t w0 = blockIdx.x << span_log2;
+  const uint32_t entries = 1u << (span_log2 + s);
+  for (uint32_t e = threadIdx.x; e < entries; e += blockDim.x) {
+    const uint32_t slice = e >> span_log2;
+    const uint32_t w = w0 + (e & ((1u << span_log2) - 1u));
+    if (w >= words) continue;
+    const uint32_t *src = p.partials + static_cast<uint64_t>(slice) * p.chunks * words + w;
+    uint32_t low = 0, high = 0;
+#pragma unroll 8
+    for (uint32_t ch = blockIdx.y; ch < p.chunks; ch += gridDim.y) {
+      const uint32_t v = src[static_cast<uint64_t>(ch) * words];
+      low += PACKED ? v & 0xffffu : v;
+      high += PACKED ? v >> 16 : 0u;
+    }
+    s_low[((w - w0) << s) | ((w ^ slice) & mask)] = low;
+    if constexpr (PACKED) s_high[((w - w0) << s) | (((w + half) ^ slice) & mask)] = high;
+  }
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < entries; e += blockDim.x) {
+    if (w0 + (e >> s) >= words) continue;
+    const uint32_t b = (w0 << s) + e;
+    if (s_low[e] && b < p.num_bins)
+      __hip_atomic_fetch_add(&p.bins[b], s_low[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (PACKED) {
+      const uint32_t bh = b + (half << s);
+      if (s_high[e] && bh < p.num_bins)
+        __hip_atomic_fetch_add(&p.bins[bh], s_high[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
 }
 
 // --------------------------------------------------------------------------
@@ -341,6 +488,16 @@ uint32_t pick_grid(uint64_t work_items, uint32_t wg, uint64_t max_groups) {
   return static_cast<uint32_t>(g);
 }
 
+// More bins than max_plain_bins are counted in packed 16-bit fields: the
+// partials of 32-bit counters are twice the bytes (2^24 keys into 32768
+// bins: 34.0 -> 27.6 us, into 16384 bins: 25.9 -> 22.3 us).
+constexpr uint32_t max_plain_bins = 8192;
+constexpr uint32_t max_local_bins = 65536;  // packed counters of one LDS
+constexpr uint32_t max_slices_log2 = 6;
+constexpr uint64_t direct_keys = 1ull << 17;
+constexpr uint64_t direct_keys_per_group = 4096;
+constexpr uint64_t direct_atomics = 1ull << 22;
+
 acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32_t *keys,
                       uint64_t n, uint32_t *bins, uint32_t num_bins, int strat,
                       const acpp_launch_config *cfg) {
@@ -355,19 +512,24 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
   int cus = 0;
   acpp_status st = enter_device(g, &cus);
   if (st != ACPP_SUCCESS) return st;
-  const bool fits32 = static_cast<uint64_t>(num_bins) * 4 <= lds_bytes_budget;
   const bool fits16 = static_cast<uint64_t>((num_bins + 1) / 2) * 4 <= lds_bytes_budget;
-  if (strat == strat_auto) strat = fits16 ? strat_privatized : strat_global;
   if (strat == strat_privatized && !fits16)
     return set_error(ACPP_ERROR_UNSUPPORTED,
                      "acpp_histogram_u32: more than 65536 bins do not fit the LDS; use the global strategy");
+  // More bins than one LDS holds are cut into slices.  Every slice visits
+  // every key, so beyond max_slices one atomic per key is the better form.
+  uint32_t slices_log2 = 0;
+  while (!fits16 && slices_log2 < max_slices_log2 && ceil_div(num_bins, 1ull << slices_log2) > max_local_bins) ++slices_log2;
+  const bool sliceable = !fits16 && ceil_div(num_bins, 1ull << slices_log2) <= max_local_bins;
+  const int strat_given = strat;
+  if (strat == strat_auto) strat = (fits16 || sliceable) ? strat_privatized : strat_global;
   const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : 1024;
   if (!valid_work_group_size(wg))
     return set_error(ACPP_ERROR_INVALID_ARGUMENT, "acpp_histogram_u32: bad work_group_size");
   const geom gm = make_geom(keys, n);
 
   if (strat == strat_global) {
-    auto kernel = histogram_kernel<false, true, 4>;
+    auto kernel = histogram_global_kernel<4>;
     int resident = 1;
     st = occupancy(kernel, static_cast<int>(wg), &resident);
     if (st != ACPP_SUCCESS) return st;
@@ -375,45 +537,116 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
     if (cfg && cfg->groups_per_cu)
       groups_cap = std::min<uint64_t>(groups_cap, cfg->groups_per_cu * static_cast<uint64_t>(cus));
     const uint32_t grid = pick_grid(gm.nvec + gm.nscalar, wg * 4, groups_cap);
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), 0, stream, keys, gm, num_bins, nullptr, bins, 0u);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), 0, stream, keys, gm, num_bins, bins);
     st = check_launch(name);
     return st == ACPP_SUCCESS ? clear_error() : st;
   }
 
-  const bool packed = !fits32;
+  // Cost of a form with 2^sl slices, from rates measured on MI355X: the keys'
+  // time falls with the number of groups, the time to write and read the
+  // groups' partials grows with it, and their sum is least at the square
+  // root.  A CU counts a key in 0.15 ns, visits one of a slice in 0.11 ns;
+  // partials move at about 4 TB/s.
+  const uint64_t cu_groups = static_cast<uint64_t>(cus);
+  const bool packed = num_bins > max_plain_bins;
+  struct form {
+    uint32_t slices_log2;
+    uint32_t words;  // 32-bit words of a group's partial
+    double groups;
+    double seconds;
+  };
+  auto cost = [&](uint32_t sl) {
+    form f;
+    f.slices_log2 = sl;
+    f.words = packed ? ((((num_bins - 1) >> sl) + 1) + 1) / 2 : num_bins;
+    const double keys_s = static_cast<double>(n) * (sl ? (1u << sl) * 1.1e-10 : 1.5e-10);
+    const double partial_s = 8.0 * f.words / 4e12;
+    f.groups = std::min(static_cast<double>(cu_groups), std::sqrt(keys_s / partial_s));
+    f.seconds = keys_s / f.groups + partial_s * f.groups;
+    return f;
+  };
+  form best = cost(slices_log2);
+  // Twice the slices halve the partials: better for few keys and many bins
+  // (2^24 keys, 65536 bins: 35.7 -> 29.7 us; 2^23 keys: 30.3 -> 24.2 us).
+  if (packed && slices_log2 < max_slices_log2 && strat_given == strat_auto) {
+    const form twice = cost(slices_log2 + 1);
+    if (twice.seconds < best.seconds) best = twice;
+  }
+  slices_log2 = best.slices_log2;
+  const uint32_t slices = 1u << slices_log2;
+  hist_params p;
+  p.keys = keys;
+  p.gm = gm;
+  p.bins = bins;
+  p.num_bins = num_bins;
+  p.local_bins = ((num_bins - 1) >> slices_log2) + 1;
+  p.slices_log2 = slices_log2;
   // Up to 8 copies of 32-bit counters within the LDS budget.
-  uint32_t copies_log2 = 0;
-  while (!packed && copies_log2 < 3 &&
-         (static_cast<uint64_t>(num_bins) << (copies_log2 + 1)) * 4 <= lds_bytes_budget)
-    ++copies_log2;
-  const size_t lds = packed ? static_cast<size_t>((num_bins + 1) / 2) * 4
-                            : (static_cast<size_t>(num_bins) << copies_log2) * 4;
-  auto kernel = packed ? histogram_kernel<true, false, 4> : histogram_kernel<false, false, 4>;
-  int resident = 1;
-  ACPP_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kernel, static_cast<int>(wg), lds));
-  if (resident < 1) resident = 1;
-  uint64_t groups_cap = static_cast<uint64_t>(resident) * cus;
-  // Each group writes a partial histogram; keep the partials to at most 1/8
-  // of the key bytes (but at least one group per CU).
-  const uint64_t partial_cap = std::max<uint64_t>(static_cast<uint64_t>(cus), (n / 8) / num_bins);
-  groups_cap = std::min(groups_cap, partial_cap);
+  p.copies_log2 = 0;
+  while (!packed && p.copies_log2 < 3 &&
+         (static_cast<uint64_t>(num_bins) << (p.copies_log2 + 1)) * 4 <= lds_bytes_budget)
+    ++p.copies_log2;
+  const uint32_t partial_words = best.words;
+  const size_t lds = (static_cast<size_t>(partial_words) << p.copies_log2) * 4;
+  auto kernel = slices > 1 ? histogram_kernel<true, true, 4>
+                : packed   ? histogram_kernel<true, false, 4>
+                           : histogram_kernel<false, false, 4>;
   // One group per CU by default: the kernel is bound by the CU's LDS atomic
   // rate (about two keys per clock), and a second resident group only adds
   // contention (2^28 Zipf keys, 4096 bins on MI355X: 252 us with one group
   // per CU, 302 us with two).
-  const uint32_t gpc = (cfg && cfg->groups_per_cu) ? cfg->groups_per_cu : 1u;
-  groups_cap = std::min<uint64_t>(groups_cap, gpc * static_cast<uint64_t>(cus));
-  const uint32_t grid = pick_grid(gm.nvec + gm.nscalar, wg * 4, groups_cap);
-  void *partials = nullptr;
-  st = group_obtain(g, static_cast<size_t>(grid) * num_bins * sizeof(uint32_t), &partials);
-  if (st != ACPP_SUCCESS) return st;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), lds, stream, keys, gm, num_bins,
-                     static_cast<uint32_t *>(partials), bins, copies_log2);
+  uint64_t groups = cu_groups;
+  bool direct = false;
+  if (cfg && cfg->groups_per_cu) {
+    int resident = 1;
+    ACPP_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kernel, static_cast<int>(wg), lds));
+    if (resident < 1) resident = 1;
+    groups = std::min<uint64_t>(cfg->groups_per_cu, resident) * cu_groups;
+    // Each group writes a partial histogram; keep the partials to at most 1/8
+    // of the key bytes (but at least one group per CU).
+    groups = std::min(groups, std::max<uint64_t>(cu_groups, (n / 8) / num_bins));
+    groups = pick_grid(gm.nvec + gm.nscalar, wg * 4, groups);
+  } else {
+    // Few keys, or few bins: the counters that are not zero go straight to
+    // the bins, and there is no second launch (calls with the clear of the
+    // bins, up to 2^17 keys: 14.2 -> 10.5 us; 2^24 keys into 4096 bins: 22.4
+    // -> 18.8 us).  Above direct_atomics the partials are faster (65536 bins,
+    // 2^24 keys: 53.6 us direct, 29.7 us with partials; 32768 bins 32.8
+    // against 27.8 us; 16384 bins 22.4 against 26.0 us).
+    const uint64_t part = static_cast<uint64_t>(ceil_div(n, direct_keys_per_group)) << slices_log2;
+    groups = std::min(groups, part);
+    if (n > direct_keys && groups * num_bins > direct_atomics) groups = std::min(groups, static_cast<uint64_t>(best.groups) + 1);
+    else direct = true;
+  }
+  if (slices > 1) {
+    // whole chunks: every slice of a part of the keys, on one XCD if it can be
+    const uint64_t per_xcd = static_cast<uint64_t>(slices) * 8;
+    groups = std::max<uint64_t>(groups / slices, 1) * slices;
+    if (groups > per_xcd) groups = groups / per_xcd * per_xcd;
+  }
+  p.xcd_map = slices > 1 && groups % (static_cast<uint64_t>(slices) * 8) == 0;
+  p.chunks = static_cast<uint32_t>(groups >> slices_log2);
+  const uint32_t grid = static_cast<uint32_t>(groups);
+  // The sliced form serves calls that need no scratch with one atomic per
+  // key: it takes none under stream capture (an allocation there could fail),
+  // nor when there is none to have.
+  p.partials = nullptr;
+  if (!direct && !(slices > 1 && stream_is_capturing(stream))) {
+    void *partials = nullptr;
+    st = group_obtain(g, static_cast<size_t>(grid) * partial_words * sizeof(uint32_t), &partials);
+    if (st != ACPP_SUCCESS && slices == 1) return st;
+    p.partials = st == ACPP_SUCCESS ? static_cast<uint32_t *>(partials) : nullptr;
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), lds, stream, p);
   st = check_launch(name);
   if (st != ACPP_SUCCESS) return st;
-  const uint32_t chunks = std::min<uint32_t>(grid, 32u);
-  hipLaunchKernelGGL(histogram_combine_kernel, dim3(static_cast<uint32_t>(ceil_div(num_bins, 256)), chunks),
-                     dim3(256), 0, stream, static_cast<const uint32_t *>(partials), grid, num_bins, bins);
+  if (!p.partials) return clear_error();
+  const uint32_t x = static_cast<uint32_t>(ceil_div(partial_words, 1ull << combine_span_log2(slices_log2)));
+  const uint32_t y = std::max(1u, std::min(std::min(p.chunks, 32u), 1024u / x));
+  if (packed)
+    hipLaunchKernelGGL(histogram_combine_kernel<true>, dim3(x, y), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL(histogram_combine_kernel<false>, dim3(x, y), dim3(256), 0, stream, p);
   st = check_launch(name);
   return st == ACPP_SUCCESS ? clear_error() : st;
 }

@@ -58,6 +58,62 @@ def test_histogram_misaligned_keys(gpu, q, scratch):
             assert np.array_equal(host(bins), O.histogram(keys[off:], 4096))
 
 
+# Above 65536 bins the bins are cut into 2 .. 64 slices (2^22 bins); one bin
+# more takes one atomic per key.  2^17 keys are the last that need no scratch.
+@pytest.mark.parametrize("num_bins", [65537, 131072, 131073, 200000, 1 << 20, (1 << 20) + 1, 1 << 22, (1 << 22) + 1])
+@pytest.mark.parametrize("n", [1, 4097, 1 << 17, (1 << 17) + 1, (1 << 22) + 3])
+def test_histogram_sliced(gpu, q, scratch, num_bins, n):
+    torch, _ = gpu
+    rng = np.random.default_rng(n)
+    skewed = zipf_keys(n, num_bins + 10, seed=n)  # some keys out of range
+    spread = rng.integers(0, num_bins + 100, n).astype(np.uint32)
+    strided = (np.arange(n, dtype=np.uint64) * 4096 % num_bins).astype(np.uint32)
+    one = np.full(n, num_bins - 1, dtype=np.uint32)  # its 16-bit counter drains
+    for keys in (skewed, spread, strided, one):
+        for off in (0, 1):
+            start = rand(np.uint32, num_bins, seed=1, lo=0, hi=1000)
+            bins = dev(torch, start)
+            acpp.histogram(q, scratch, dev(torch, keys)[off:], bins)
+            q.wait()
+            scratch.release()
+            assert np.array_equal(host(bins), O.histogram(keys[off:], num_bins, start)), off
+
+
+@pytest.mark.parametrize("num_bins", [4096, 65536, 200000])
+def test_histogram_captured(gpu, num_bins):
+    # replays add to the bins like eager calls; the sliced form captures
+    # without scratch
+    torch, _ = gpu
+    n = (1 << 20) + 7
+    keys = zipf_keys(n, num_bins, seed=9)
+    kd = dev(torch, keys)
+    bins = torch.zeros(num_bins, dtype=torch.uint32, device="cuda")
+    cache = acpp.AllocationCache()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        q = acpp.Queue()
+        with acpp.AllocationGroup(cache) as scratch:
+            if num_bins <= 65536:  # leaves the scratch in the cache
+                acpp.histogram(q, scratch, kd, bins)
+                q.wait()
+        scratch = acpp.AllocationGroup(cache)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            acpp.histogram(acpp.Queue(), scratch, kd, bins)
+        calls = 1 if num_bins <= 65536 else 0
+        once = O.histogram(keys, num_bins).astype(np.uint64)
+        for _ in range(3):
+            graph.replay()
+            with acpp.AllocationGroup(cache) as other:
+                acpp.histogram(q, other, kd, bins)
+                q.wait()
+            calls += 2
+            assert np.array_equal(host(bins), (once * calls).astype(np.uint32))
+    del graph
+    scratch.close()
+    cache.close()
+
+
 @pytest.mark.parametrize("dtype", [np.int32, np.uint32, np.int64, np.uint64, np.float32,
                                    np.float64])
 @pytest.mark.parametrize("num_slots", [1, 64, 1000, 1024, 4096, 70000])
