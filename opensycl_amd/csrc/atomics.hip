@@ -21,11 +21,9 @@
 //     atomics) and a second kernel adds their column sums to the bins;
 //   - keys are streamed with 128-bit loads, several per work-item in flight;
 //   - strided fetch_min / fetch_max / fetch_add (slot = i mod num_slots):
-//     the grid is sized so that num_slots divides the grid stride whenever
-//     that fits; then each work-item always meets the same slots, keeps them
-//     in registers, and the group combines them once at the end.  Otherwise
-//     the elements go through LDS atomics, with 16-byte loads and slots
-//     tracked incrementally;
+//     the elements are the rows of a matrix whose columns always meet the
+//     same slots; a work-item keeps a column's slots in registers, and the
+//     group combines its rows once at the end;
 //   - strategy "global": one device-scope atomic per element, the
 //     reference's pattern, kept for comparison.
 #include <algorithm>
@@ -360,116 +358,96 @@ struct rmw_add {
   }
 };
 
-constexpr int scope_wg = __HIP_MEMORY_SCOPE_WORKGROUP;
 constexpr int scope_dev = __HIP_MEMORY_SCOPE_AGENT;
 
-// Register-privatised form: requires num_slots | (VEC * total work-items),
-// which the launcher arranges through the grid size.  Then element
-// head + VEC*c + k of chunk c = gtid + m*stride lands in slot
-// (head + VEC*gtid + k) mod num_slots for every m, so each work-item keeps
-// VEC fixed slots in registers over the whole grid-stride loop.
-template <class T, class R>
-__global__ __launch_bounds__(1024) void strided_register_kernel(const T *__restrict__ v, geom gm,
-                                                                uint32_t num_slots, T *target) {
+// The elements after the scalar head as a matrix of 16-byte vectors whose
+// rows hold a whole multiple of num_slots elements: all of a column's vectors
+// meet the same VEC slots.  A work-group takes a strip of `width` columns (a
+// power of two) and every row_groups-th band of blockDim.x / width rows; each
+// work-item keeps its column's VEC slots in registers over all its rows, the
+// group folds its rows in LDS and adds one value per slot of the strip to the
+// target.
+struct strip_params {
+  geom gm;
+  uint64_t columns;     // vectors in a row
+  uint64_t row_groups;  // work-groups that share a strip
+  uint32_t width_log2;
+  uint64_t num_slots;
+};
+
+// Bound by the loads.  Narrow strips keep the atomics few (a group adds
+// width x VEC values at most), and the rows of a strip read at least 1 KiB in
+// one piece where there are rows enough.  Before, groups kept all slots in
+// LDS: one device atomic per slot and group, with LDS atomics per element
+// unless the slots divided the grid's stride, and device atomics per element
+// for slots that do not fit the LDS: 2^26 fp32 adds into 1024 slots 50 -> 42
+// us, 5000 slots 339 -> 44 us, 100,000 slots 219 -> 43 us; 2^28 into 1024
+// slots 158.6 -> 157.2 us (6.8 TB/s), into 777 slots 1333 -> 160 us; 2^21
+// fp32 max into 1024 slots 103 -> 11 us.
+template <class T, class R, bool NT>
+__global__ __launch_bounds__(1024) void strided_strip_kernel(const T *__restrict__ v, strip_params p, T *target) {
   constexpr int VEC = 16 / sizeof(T);
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  const uint64_t gtid = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const u32x4 *vv = reinterpret_cast<const u32x4 *>(v + gm.head);
+  constexpr int UNROLL = 4;
+  extern __shared__ unsigned char lds_raw[];
+  T *lds = reinterpret_cast<T *>(lds_raw);  // blockDim.x x VEC
+  const uint32_t width = 1u << p.width_log2;
+  const uint32_t rows = blockDim.x >> p.width_log2;
+  const uint64_t strip = blockIdx.x / p.row_groups;
+  const uint64_t row_group = blockIdx.x - strip * p.row_groups;
+  const uint64_t first_column = strip << p.width_log2;
+  const uint64_t column = first_column + (threadIdx.x & (width - 1u));
+  const u32x4 *vv = reinterpret_cast<const u32x4 *>(v + p.gm.head);
   T acc[VEC];
 #pragma unroll
   for (int k = 0; k < VEC; ++k) acc[k] = R::identity();
-  uint64_t c = gtid;
-  for (; c + 3 * stride < gm.nvec; c += 4 * stride) {
-    u32x4 q[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) q[u] = __builtin_nontemporal_load(vv + c + u * stride);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      T e[VEC];
-      __builtin_memcpy(e, &q[u], 16);
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) acc[k] = R::apply(acc[k], e[k]);
-    }
-  }
-  for (; c < gm.nvec; c += stride) {
-    const u32x4 q = vv[c];
+  const uint64_t stride = p.row_groups * rows * p.columns;
+  uint64_t c = (row_group * rows + (threadIdx.x >> p.width_log2)) * p.columns + column;
+  if (column >= p.columns || (threadIdx.x >> p.width_log2) >= rows) c = p.gm.nvec;
+  auto load = [&](uint64_t i) {
+    if constexpr (NT)
+      return __builtin_nontemporal_load(vv + i);
+    else
+      return vv[i];
+  };
+  auto fold = [&](u32x4 q) {
     T e[VEC];
     __builtin_memcpy(e, &q, 16);
 #pragma unroll
     for (int k = 0; k < VEC; ++k) acc[k] = R::apply(acc[k], e[k]);
-  }
-  extern __shared__ unsigned char lds_raw[];
-  T *lds = reinterpret_cast<T *>(lds_raw);
-  for (uint32_t i = threadIdx.x; i < num_slots; i += blockDim.x) lds[i] = R::identity();
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < VEC; ++k)
-    R::template atomic<scope_wg>(&lds[(gm.head + VEC * gtid + k) % num_slots], acc[k]);
-  for (uint64_t s = gtid; s < gm.nscalar; s += stride) {
-    const uint64_t i = scalar_index(gm, s);
-    R::template atomic<scope_wg>(&lds[i % num_slots], v[i]);
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < num_slots; i += blockDim.x)
-    R::template atomic<scope_dev>(&target[i], lds[i]);
-}
-
-// LDS-privatised form for any slot count that fits the LDS budget.  Keys
-// are streamed with 16-byte loads (4 in flight) and the slot of each
-// element is tracked incrementally: chunk c starts at slot
-// (head + VEC c) mod num_slots, and moving c on by the grid stride adds a
-// fixed step.  (One scalar load and one 64-bit modulo per element ran at a
-// sixth of the register form's rate.)
-template <class T, class R>
-__global__ __launch_bounds__(1024) void strided_lds_kernel(const T *__restrict__ v, geom gm,
-                                                           uint32_t num_slots, T *target) {
-  constexpr int VEC = 16 / sizeof(T);
-  constexpr int UNROLL = 4;
-  extern __shared__ unsigned char lds_raw[];
-  T *lds = reinterpret_cast<T *>(lds_raw);
-  for (uint32_t i = threadIdx.x; i < num_slots; i += blockDim.x) lds[i] = R::identity();
-  __syncthreads();
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  const uint64_t gtid = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const u32x4 *vv = reinterpret_cast<const u32x4 *>(v + gm.head);
-  // slot of the first element of chunk c, and its advance per stride
-  const uint32_t step = static_cast<uint32_t>((VEC * stride) % num_slots);
-  uint32_t s0 = static_cast<uint32_t>((gm.head + VEC * gtid) % num_slots);
-  auto advance = [&](uint32_t s, uint32_t by) {
-    s += by;  // s, by < num_slots <= 2^31
-    return s >= num_slots ? s - num_slots : s;
   };
-  auto fold = [&](u32x4 q, uint32_t s) {
-    T e[VEC];
-    __builtin_memcpy(e, &q, 16);
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      R::template atomic<scope_wg>(&lds[s], e[k]);
-      s = advance(s, 1);
-    }
-  };
-  uint64_t c = gtid;
-  for (; c + (UNROLL - 1) * stride < gm.nvec; c += UNROLL * stride) {
+  for (; c + (UNROLL - 1) * stride < p.gm.nvec; c += UNROLL * stride) {
     u32x4 q[UNROLL];
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) q[u] = __builtin_nontemporal_load(vv + c + u * stride);
+    for (int u = 0; u < UNROLL; ++u) q[u] = load(c + u * stride);
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      fold(q[u], s0);
-      s0 = advance(s0, step);
-    }
+    for (int u = 0; u < UNROLL; ++u) fold(q[u]);
   }
-  for (; c < gm.nvec; c += stride) {
-    fold(vv[c], s0);
-    s0 = advance(s0, step);
-  }
-  for (uint64_t s = gtid; s < gm.nscalar; s += stride) {
-    const uint64_t i = scalar_index(gm, s);
-    R::template atomic<scope_wg>(&lds[i % num_slots], v[i]);
+  for (; c < p.gm.nvec; c += stride) fold(load(c));
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) lds[threadIdx.x * VEC + k] = acc[k];
+  __syncthreads();
+  // Values e, e + num_slots, ... of every row of the strip meet one slot.
+  const uint32_t values = width * VEC;
+  const uint64_t in_row = ((p.columns < p.gm.nvec ? p.columns : p.gm.nvec) - first_column) * VEC;
+  const uint32_t used = in_row < values ? static_cast<uint32_t>(in_row) : values;
+  const uint32_t slots = p.num_slots < used ? static_cast<uint32_t>(p.num_slots) : used;
+  for (uint32_t e = threadIdx.x; e < used; e += blockDim.x) {
+    T x = lds[e];
+    for (uint32_t r = 1; r < rows; ++r) x = R::apply(x, lds[r * values + e]);
+    lds[e] = x;  // row 0's value e is read by this work-item only
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < num_slots; i += blockDim.x)
-    R::template atomic<scope_dev>(&target[i], lds[i]);
+  for (uint32_t e = threadIdx.x; e < slots; e += blockDim.x) {
+    T x = lds[e];
+    for (uint32_t j = e + slots; j < used; j += slots) x = R::apply(x, lds[j]);
+    R::template atomic<scope_dev>(&target[(p.gm.head + first_column * VEC + e) % p.num_slots], x);
+  }
+  // The head and the tail (fewer than 2 VEC elements).
+  if (blockIdx.x == 0)
+    for (uint64_t s = threadIdx.x; s < p.gm.nscalar; s += blockDim.x) {
+      const uint64_t i = scalar_index(p.gm, s);
+      R::template atomic<scope_dev>(&target[i % p.num_slots], v[i]);
+    }
 }
 
 // The reference's pattern: one device-scope atomic per element.
@@ -651,6 +629,8 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
   return st == ACPP_SUCCESS ? clear_error() : st;
 }
 
+constexpr uint64_t min_columns = 512;
+
 template <class T, template <class> class RT>
 acpp_status strided(acpp_allocation_group *g, hipStream_t stream, const T *values, uint64_t n,
                     T *target, uint32_t num_slots, int strat, const acpp_launch_config *cfg,
@@ -667,35 +647,54 @@ acpp_status strided(acpp_allocation_group *g, hipStream_t stream, const T *value
   acpp_status st = enter_device(g, &cus);
   if (st != ACPP_SUCCESS) return st;
   constexpr uint32_t VEC = 16 / sizeof(T);
-  const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : 256;
-  if (!valid_work_group_size(wg))
-    return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
-  const bool fits = static_cast<uint64_t>(num_slots) * sizeof(T) <= lds_bytes_budget;
-  if (strat == strat_auto) strat = fits ? strat_privatized : strat_global;
-  if (strat == strat_privatized && !fits)
+  if (strat == strat_privatized && static_cast<uint64_t>(num_slots) * sizeof(T) > lds_bytes_budget)
     return set_error(ACPP_ERROR_UNSUPPORTED, std::string(name) + ": slots do not fit the LDS; use the global strategy");
-  const uint64_t cap_groups =
-      static_cast<uint64_t>(cus) * ((cfg && cfg->groups_per_cu) ? cfg->groups_per_cu : 2);
   if (strat == strat_global) {
+    const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : 256;
+    if (!valid_work_group_size(wg))
+      return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
+    const uint64_t cap_groups =
+        static_cast<uint64_t>(cus) * ((cfg && cfg->groups_per_cu) ? cfg->groups_per_cu : 2);
     const uint32_t grid = pick_grid(n, wg, cap_groups * 8);
     hipLaunchKernelGGL((strided_global_kernel<T, R>), dim3(grid), dim3(wg), 0, stream, values, n, num_slots, target);
   } else {
-    const size_t lds = static_cast<size_t>(num_slots) * sizeof(T);
-    const geom gm = make_geom(values, n);
-    const uint32_t grid = pick_grid(gm.nvec + gm.nscalar, wg * 4, cap_groups);
-    // The register form needs VEC * wg * grid to be a multiple of
-    // num_slots: grid a multiple of `period`.  (1000 slots: period 125 with
-    // 256-wide groups; with per-element LDS atomics instead, fp32 adds ran
-    // at 0.8 TB/s.)
-    const uint64_t period = num_slots / std::gcd<uint64_t>(static_cast<uint64_t>(VEC) * wg, num_slots);
-    if (period <= grid) {
-      const uint32_t grid_reg = static_cast<uint32_t>((grid / period) * period);
-      hipLaunchKernelGGL((strided_register_kernel<T, R>), dim3(grid_reg), dim3(wg), lds, stream, values, gm,
-                         num_slots, target);
-    } else {
-      hipLaunchKernelGGL((strided_lds_kernel<T, R>), dim3(grid), dim3(wg), lds, stream, values, gm,
-                         num_slots, target);
-    }
+    const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : 512;
+    if (!valid_work_group_size(wg))
+      return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
+    strip_params p;
+    p.gm = make_geom(values, n);
+    p.num_slots = num_slots;
+    // The shortest row of whole vectors, repeated to min_columns so that a
+    // last, partly used strip costs little.
+    p.columns = num_slots / std::gcd<uint64_t>(VEC, num_slots);
+    if (p.columns < min_columns) p.columns *= ceil_div(min_columns, p.columns);
+    const uint64_t used_columns = std::max<uint64_t>(1, std::min(p.columns, p.gm.nvec));
+    const uint64_t rows = std::max<uint64_t>(1, ceil_div(p.gm.nvec, p.columns));
+    // Inputs larger than the last-level cache stream past it.
+    const bool large = n * sizeof(T) >= (256ull << 20);
+    // Strips as narrow as a wave (fewest atomics), of 4 KiB a row for large
+    // inputs (2^28 fp32 into 1024 slots: 169 us with 1 KiB, 157 us with 4 KiB;
+    // 2^23: 9.3 and 13.3 us), or wider when there are too few rows for all
+    // work-items.
+    p.width_log2 = large ? 8 : 6;
+    while ((1u << p.width_log2) < wg && (wg >> p.width_log2) > rows) ++p.width_log2;
+    while ((1u << p.width_log2) > wg) --p.width_log2;
+    const uint64_t strips = ceil_div(used_columns, 1ull << p.width_log2);
+    const uint64_t band_rows = wg >> p.width_log2;
+    const uint64_t cap_groups =
+        static_cast<uint64_t>(cus) * ((cfg && cfg->groups_per_cu) ? cfg->groups_per_cu : 1);
+    const uint64_t wanted = std::min(cap_groups, std::max<uint64_t>(1, ceil_div(p.gm.nvec, static_cast<uint64_t>(wg) * 4)));
+    p.row_groups = std::max<uint64_t>(1, std::min(wanted / strips, ceil_div(rows, band_rows)));
+    const uint64_t grid = strips * p.row_groups;
+    if (grid >= (1ull << 31))
+      return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": problem too large");
+    const size_t lds = static_cast<size_t>(wg) * 16;
+    if (large)
+      hipLaunchKernelGGL((strided_strip_kernel<T, R, true>), dim3(static_cast<uint32_t>(grid)), dim3(wg), lds, stream,
+                         values, p, target);
+    else
+      hipLaunchKernelGGL((strided_strip_kernel<T, R, false>), dim3(static_cast<uint32_t>(grid)), dim3(wg), lds, stream,
+                         values, p, target);
   }
   st = check_launch(name);
   return st == ACPP_SUCCESS ? clear_error() : st;

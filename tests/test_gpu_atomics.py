@@ -180,3 +180,45 @@ def test_strided_lds_form_misaligned_view(gpu, q, scratch, dtype):
         exp = start.copy()
         {"max": np.maximum, "min": np.minimum, "add": np.add}[op].at(exp, idx, v[3:])
         assert np.array_equal(host(t), exp), op
+
+
+# Strips of 64 columns of 16 bytes (256 above 256 MiB), rows repeated to at
+# least 512 columns: slot counts around those edges, fewer elements than
+# slots, fewer rows than a group's bands, views, and a group size that is no
+# power of two.
+@pytest.mark.parametrize("dtype", [np.int32, np.float32, np.float64])
+@pytest.mark.parametrize("num_slots", [1, 3, 255, 256, 257, 2047, 2049, 32769, 65537])
+def test_strided_strips(gpu, q, scratch, dtype, num_slots):
+    torch, _ = gpu
+    for n in (1, 5, num_slots - 1, num_slots, num_slots + 1, 3 * num_slots + 2, (1 << 18) + 7):
+        if n < 1:
+            continue
+        # small integers: float sums are exact in any order
+        v = np.round(rand(np.float64, n + 3, seed=num_slots) * 4).astype(dtype)
+        vd = dev(torch, v)
+        for off in (0, 1, 3):
+            x = v[off:off + n]
+            idx = np.arange(n) % num_slots
+            for op, fold in (("add", np.add), ("min", np.minimum), ("max", np.maximum)):
+                for cfg in (None, (192,)):
+                    t = torch.full((num_slots,), 3, dtype=vd.dtype, device="cuda")
+                    acpp.atomic_fetch_strided(q, scratch, op, vd[off:off + n], t, config=cfg)
+                    q.wait()
+                    exp = np.zeros(num_slots, dtype=dtype) + dtype(3)
+                    fold.at(exp, idx, x)
+                    assert np.array_equal(host(t), exp), (n, off, op, cfg)
+
+
+def test_strided_strips_wide(gpu, q, scratch):
+    # above 256 MiB a strip is 256 columns wide and streams past the caches
+    torch, _ = gpu
+    n = (1 << 26) + 1003
+    for num_slots in (1000, 40000):
+        v = (torch.arange(n, device="cuda") % 7 - 3).to(torch.float32)
+        t = torch.zeros(num_slots, dtype=torch.float32, device="cuda")
+        acpp.atomic_fetch_strided(q, scratch, "add", v, t)
+        q.wait()
+        rows = n // num_slots
+        exp = v[:rows * num_slots].view(rows, num_slots).double().sum(0)
+        exp[:n - rows * num_slots] += v[rows * num_slots:]
+        assert torch.equal(t.double(), exp), num_slots
