@@ -233,15 +233,14 @@ struct params {
   const T *in;
   T *out;
   const uint64_t *offsets;  // num_segments + 1 entries
-  const uint32_t *tile_seg;  // first segment of every tile (num_tiles + 1 entries)
-  const uint32_t *heads;     // bit e set: a non-empty segment starts at element e
+  const uint32_t *tile_seg;  // reductions: first segment of every tile (tile_table_kernel), or NULL
+  const uint32_t *heads;     // scans: bit e set: a segment starts at element e; or NULL
   uint64_t head_words_total;  // 32-bit words of the bitmap
   int block_lookback;        // 1: work-group-wide look-back window
   int force_give_up;         // ACPP_VARIANT_FORCE_GIVE_UP (tests of the error path)
   uint64_t num_segments;
   uint64_t total;
   W init;
-  int reduce;  // 0: inclusive scan per segment, 1: reduce per segment
   int vec_io;
   uint32_t num_tiles;
   uint32_t epoch;
@@ -255,43 +254,151 @@ __device__ __forceinline__ uint64_t clamp_off(const uint64_t *offsets, uint64_t 
   return o < total ? o : total;
 }
 
-// Setup: tile_seg[t] = the non-empty segment containing element t*tile_elems
-// (num_segments for t == num_tiles), the head bitmap for the scans (bit b
-// for the first element b of every non-empty segment; the bitmap is cleared
-// beforehand; none for the reductions, heads_out NULL), and init into empty
-// segments' results.
-template <class T>
-__global__ void setup_kernel(params<T> p, uint32_t *tile_seg_out, uint32_t *heads_out, uint64_t tile_elems) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t s = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; s < p.num_segments;
-       s += stride) {
-    const uint64_t b = clamp_off(p.offsets, s, p.total);
-    const uint64_t e = clamp_off(p.offsets, s + 1, p.total);
-    if (e <= b) {
-      if (p.reduce) p.out[s] = static_cast<T>(p.init);
-      continue;
-    }
-    if (heads_out) atomicOr(&heads_out[b >> 5], 1u << (b & 31));
-    // tiles whose first element lies in [b, e)
-    const uint64_t t0 = (b + tile_elems - 1) / tile_elems;
-    const uint64_t t1 = (e + tile_elems - 1) / tile_elems;
-    for (uint64_t t = t0; t < t1; ++t) tile_seg_out[t] = static_cast<uint32_t>(s);
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) tile_seg_out[p.num_tiles] = static_cast<uint32_t>(p.num_segments);
-}
-
-// Largest s in [lo, hi] with offsets[s] <= e (offsets[lo] <= e holds).
-__device__ __forceinline__ uint64_t find_segment(const uint64_t *offsets, uint64_t lo, uint64_t hi,
-                                                 uint64_t e, uint64_t total) {
+// The number of offsets[0 .. n) below key (offsets sorted), found by a whole
+// wave: 64 probes a round shrink the range 65 times, so 65,536 offsets take
+// three dependent loads and 2^26 five.  Unsorted offsets give some value in
+// [0, n].  The result is uniform.
+__device__ __forceinline__ uint64_t wave_lower_bound(const uint64_t *offsets, uint64_t n, uint64_t key) {
+  const uint64_t lane = threadIdx.x & 63;
+  uint64_t lo = 0, hi = n;
   while (lo < hi) {
-    const uint64_t mid = (lo + hi + 1) / 2;
-    if (clamp_off(offsets, mid, total) <= e)
-      lo = mid;
-    else
-      hi = mid - 1;
+    const uint64_t step = (hi - lo + 64) / 65;
+    const uint64_t at = lo + (lane + 1) * step - 1;
+    const bool below = at < hi && offsets[at] < key;
+    const uint64_t c = static_cast<uint64_t>(__builtin_popcountll(wave::ballot(below)));
+    if (c < 64) hi = min(hi, lo + (c + 1) * step - 1);
+    lo += c * step;
   }
   return lo;
 }
+
+// The segments whose start lies in [first, last) (all from the first one on
+// when to_end): found by the work-group's first and last wave, returned to
+// all through s_range.
+__device__ __forceinline__ void find_segments(const uint64_t *offsets, uint64_t num_segments, uint64_t first,
+                                              uint64_t last, bool to_end, uint64_t (&s_range)[2]) {
+  const int w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  if (w == 0) {
+    const uint64_t lo = wave_lower_bound(offsets, num_segments, first);
+    if (lane == 0) s_range[0] = lo;
+  }
+  if (w == static_cast<int>(blockDim.x >> 6) - 1) {
+    const uint64_t hi = to_end ? num_segments : wave_lower_bound(offsets, num_segments, last);
+    if (lane == 0) s_range[1] = hi;
+  }
+}
+
+// tile_seg[t] = the first segment that starts at or after tile t's first
+// element (num_segments for t == num_tiles).  A work-group narrows the
+// offsets to those of its 256 tiles, then every work-item searches its own
+// (in LDS where they fit): no step grows with a segment's length.  (One
+// work-item per segment writing the segment's tiles took 17 us for 48
+// segments of 250 tiles.)
+constexpr uint32_t table_stage = 2048;  // offsets held in LDS
+__global__ __launch_bounds__(256) void tile_table_kernel(const uint64_t *__restrict__ offsets, uint64_t num_segments,
+                                                         uint64_t tile_elems, uint32_t num_tiles, uint32_t *tile_seg) {
+  __shared__ uint64_t s_off[table_stage];
+  __shared__ uint64_t s_range[2];
+  const uint64_t t0 = static_cast<uint64_t>(blockIdx.x) * 256;
+  uint64_t first = 0, count = num_segments;
+  if (num_segments > table_stage) {
+    find_segments(offsets, num_segments, t0 * tile_elems, (t0 + 255) * tile_elems, false, s_range);
+    __syncthreads();
+    first = s_range[0];
+    count = s_range[1] > first ? s_range[1] - first : 0;
+  }
+  const bool staged = count <= table_stage;
+  if (staged) {
+    for (uint32_t i = threadIdx.x; i < count; i += 256) s_off[i] = offsets[first + i];
+    __syncthreads();
+  }
+  const uint64_t t = t0 + threadIdx.x;
+  if (t > num_tiles) return;
+  const uint64_t key = t * tile_elems;
+  uint64_t lo = 0, hi = count;
+  while (lo < hi) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    if ((staged ? s_off[mid] : offsets[first + mid]) < key)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  lo = t == num_tiles ? num_segments : first + lo;
+  tile_seg[t] = static_cast<uint32_t>(lo);
+}
+
+// The same table written by the segments: segment s is the last to start
+// before every tile boundary in (offsets[s], offsets[s + 1]].  One round trip
+// where the search above takes five or more, but it reads all offsets.  A
+// segment of more than serial_tiles tiles is written by the whole work-group.
+__global__ __launch_bounds__(256) void tile_scatter_kernel(const uint64_t *__restrict__ offsets, uint64_t num_segments,
+                                                           uint64_t tile_elems, uint32_t num_tiles,
+                                                           uint32_t *tile_seg) {
+  constexpr uint32_t serial_tiles = 8;
+  __shared__ uint32_t s_count;
+  __shared__ uint32_t s_seg[256];
+  __shared__ uint32_t s_first[256];
+  __shared__ uint32_t s_last[256];
+  if (threadIdx.x == 0) s_count = 0;
+  __syncthreads();
+  const uint64_t s = blockIdx.x * 256ull + threadIdx.x;
+  if (s < num_segments) {
+    const uint64_t b = offsets[s] / tile_elems, e = offsets[s + 1] / tile_elems;
+    const uint32_t first = static_cast<uint32_t>(min(b + 1, static_cast<uint64_t>(num_tiles)));
+    const uint32_t last = static_cast<uint32_t>(min(e + 1, static_cast<uint64_t>(num_tiles)));  // exclusive
+    if (last > first + serial_tiles) {
+      const uint32_t slot = atomicAdd(&s_count, 1u);
+      s_seg[slot] = static_cast<uint32_t>(s) + 1;
+      s_first[slot] = first;
+      s_last[slot] = last;
+    } else {
+      for (uint32_t t = first; t < last; ++t) tile_seg[t] = static_cast<uint32_t>(s) + 1;
+    }
+  }
+  if (s == 0) {
+    tile_seg[0] = 0;
+    tile_seg[num_tiles] = static_cast<uint32_t>(num_segments);
+  }
+  __syncthreads();
+  const uint32_t count = s_count;
+  for (uint32_t i = 0; i < count; ++i)
+    for (uint32_t t = s_first[i] + threadIdx.x; t < s_last[i]; t += 256) tile_seg[t] = s_seg[i];
+}
+
+// The head bitmap of the scans: bit b for every segment start b < total (the
+// start of an empty segment is that of the next one that is not empty).  A
+// work-group marks head_chunk elements in LDS from the offsets inside its
+// range and writes the words once: the bitmap needs no clearing and no global
+// atomics.  (A fill, then one global atomicOr per segment: 2^26 elements in
+// 13.4 million segments took 450 us of 558.)
+constexpr uint32_t head_chunk_words = 1024;
+constexpr uint64_t head_chunk = 32ull * head_chunk_words;
+__global__ __launch_bounds__(256) void head_bitmap_kernel(const uint64_t *__restrict__ offsets, uint64_t num_segments,
+                                                          uint64_t total, uint64_t head_words, uint32_t *heads) {
+  __shared__ uint32_t s_words[head_chunk_words];
+  __shared__ uint64_t s_range[2];
+  const uint64_t base = blockIdx.x * head_chunk;
+  const uint64_t end = min(base + head_chunk, total);
+  find_segments(offsets, num_segments, base, end, false, s_range);
+  for (uint32_t i = threadIdx.x; i < head_chunk_words; i += 256) s_words[i] = 0;
+  __syncthreads();
+  const uint64_t hi = s_range[1];
+#pragma unroll 4
+  for (uint64_t i = s_range[0] + threadIdx.x; i < hi; i += 256) {
+    const uint64_t b = offsets[i];
+    if (b >= base && b < end) atomicOr(&s_words[(b - base) >> 5], 1u << (b & 31));
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < head_chunk_words; i += 256) {
+    const uint64_t w = blockIdx.x * static_cast<uint64_t>(head_chunk_words) + i;
+    if (w < head_words) heads[w] = s_words[i];
+  }
+}
+
+// 32-bit words of a reduction tile's head bits, rounded up so that the values
+// behind them are 16-byte aligned.
+__host__ __device__ constexpr uint32_t reduce_head_words(uint32_t tile_elems) { return ((tile_elems >> 5) + 3u) & ~3u; }
 
 // threadIdx.x through an empty asm statement: a value the compiler cannot
 // move, so what is derived from it inside a loop stays inside the loop.
@@ -348,7 +455,9 @@ __device__ __forceinline__ uint32_t fold_wave_prefixes(uint32_t fm, W (&v)[R][VE
   return xcut;
 }
 
-template <class T, class Op, int R>
+// MARK: the tile marks its segment starts from the offsets itself instead of
+// reading the bitmap (small inputs: one launch instead of two).
+template <class T, class Op, int R, bool MARK>
 __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
   using W = typename elem_traits<T>::work;
   using SIO = seg_status<W>;
@@ -369,6 +478,7 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
   __shared__ int s_q[max_waves];
   __shared__ int s_give_up;
   __shared__ uint64_t s_invalid[max_waves];
+  __shared__ uint64_t s_range[2];  // MARK
   const uint32_t head_words = static_cast<uint32_t>((tile_elems + 1 + 31) / 32);
 
   // A ticket is drawn only when the work-group is ready to work on the
@@ -411,8 +521,10 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
       // load under a branch, or a select the compiler turned back into one,
       // made it wait for every outstanding load, the tile's data included,
       // before the head bits could go to LDS.
-      uint32_t hword0, hword1, hmask0, hmask1;
-      {
+      uint32_t hword0 = 0, hword1 = 0, hmask0 = 0, hmask1 = 0;
+      if constexpr (MARK) {
+        find_segments(p.offsets, p.num_segments, base, base + in_range, false, s_range);
+      } else {
         const uint64_t last = p.head_words_total - 1;
         const uint64_t i0 = (base >> 5) + tid;
         const uint64_t i1 = i0 + B;
@@ -453,6 +565,14 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
       s_heads[tid] = hword0 & hmask0;
       s_heads[tid + B] = hword1 & hmask1;
       __syncthreads();
+      if constexpr (MARK) {
+        const uint64_t hi = s_range[1];
+        for (uint64_t i = s_range[0] + tid; i < hi; i += B) {
+          const uint64_t b = p.offsets[i];
+          if (b >= base && b - base < in_range) atomicOr(&s_heads[(b - base) >> 5], 1u << (b & 31));
+        }
+        __syncthreads();
+      }
 
       auto head_at = [&](uint64_t pos) -> uint32_t {
         return (s_heads[pos >> 5] >> (pos & 31)) & 1u;
@@ -662,23 +782,46 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
 // Segmented reduction without a look-back.
 //
 // A reduction needs only each segment's total, so tiles do not wait for
-// each other.  Every tile (one work-group, launched in any order) runs the
-// same in-tile (head flag, value) scan as the scan kernel and then
-//   - writes op(init, total) for every segment that starts and ends inside
-//     the tile;
-//   - stores head_part[tile]: the fold of the elements before its first
-//     segment start (the whole tile if it has none);
-//   - stores tail_part[tile]: the fold from its last segment start to the
-//     tile's end, when that segment continues into the next tile.
+// each other.  A tile owns the segments that start in it (empty ones too; the
+// last tile also those at the end).  Every tile (one work-group, launched in
+// any order) runs the same in-tile (head flag, value) scan as the scan
+// kernel, keeps the scanned values in LDS, and one work-item per owned
+// segment then
+//   - writes op(init, value at the segment's last element) if the segment
+//     ends inside the tile, init if it is empty;
+// while the tile stores
+//   - head_part[tile]: the fold of the elements before its first segment
+//     start (the whole tile if it has none: such a tile takes a plain fold);
+//   - tail_part[tile], tail_seg[tile]: the fold from its last segment start
+//     to the tile's end and that segment's index, when the segment continues
+//     into the next tile (tail_seg = no_segment otherwise).
 // A fix-up kernel then gives every segment that spans tiles tb < ... <= tl
-// the total tail_part[tb] . head_part[tb+1] . ... . head_part[tl], folded in
-// tile order (deterministic).  The tiles strictly inside such a segment hold
-// no segment start, so their head_part is the whole tile.
+// the total tail_part[tb] . head_part[tb+1] . ... . head_part[tl]
+// (deterministic: the tree depends on the sizes only).
+//
+// Reading the values at the segments' ends from LDS, one work-item per
+// segment, keeps the results coalesced and costs no search: a binary search
+// for the segment of every last element ran in almost every step of the
+// unrolled rows once segments are short (2^26 fp32 in 1.3 million segments: 186
+// -> 67 us).  A tile in which at most three segments start takes plain folds
+// without any scan (2^28 fp32 in 40 segments: 514 -> 180 us with the fix-up
+// below, in 89,479 segments 184 -> 179 us).
 // --------------------------------------------------------------------------
+constexpr uint32_t no_segment = 0xffffffffu;
+
+template <class W>
+struct reduce_parts {
+  W *head;
+  W *tail;
+  uint32_t *tail_seg;
+};
+
+using constant_u32 = const __attribute__((address_space(4))) uint32_t *;
+using constant_u64 = const __attribute__((address_space(4))) uint64_t *;
+
 template <class T, class Op, int R>
 __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
-                                                                typename elem_traits<T>::work *head_part,
-                                                                typename elem_traits<T>::work *tail_part) {
+                                                                reduce_parts<typename elem_traits<T>::work> parts) {
   using W = typename elem_traits<T>::work;
   constexpr int VEC = 16 / sizeof(T);
   const int tid = threadIdx.x;
@@ -686,26 +829,29 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
   const int nw = B >> 6;
   const int w = tid >> 6;
   const int lane = tid & 63;
-  const uint64_t tile_elems = static_cast<uint64_t>(B) * R * VEC;
+  const uint32_t tile_elems = static_cast<uint32_t>(B * R * VEC);
   const W id = Op::identity();
 
-  extern __shared__ uint32_t s_heads[];  // tile_elems + 1 bits
+  extern __shared__ uint32_t s_heads[];     // tile_elems bits, then tile_elems values
+  W *s_val = reinterpret_cast<W *>(s_heads + reduce_head_words(tile_elems));
   __shared__ uint32_t s_tf[R * max_waves];  // per (row, wave): totals, then exclusive prefixes
   __shared__ W s_tv[R * max_waves];
-  // offsets[s_lo .. s_lo + off_cap) of the segments touching the tile: the
-  // binary search that numbers a finished segment then runs in LDS instead
-  // of as a chain of dependent global loads.
+  __shared__ uint64_t s_range[2];
+  // offsets[lo .. lo + off_cap), which are read twice, relative to the tile
+  // (beyond its end: in_range + 1)
   constexpr uint32_t off_cap = 1024;
-  __shared__ uint64_t s_off[off_cap];
-  const uint32_t head_words = static_cast<uint32_t>((tile_elems + 1 + 31) / 32);
+  __shared__ uint32_t s_off[off_cap];
+  constexpr uint32_t max_pieces = 4;
+  __shared__ W s_piece[max_pieces][max_waves];
 
   const uint32_t tile = blockIdx.x;
   if (tile >= p.num_tiles) return;
   const uint64_t base = static_cast<uint64_t>(tile) * tile_elems;
-  uint64_t s_lo = p.tile_seg[tile];
-  uint64_t s_hi = p.tile_seg[tile + 1];
+  const uint32_t in_range = static_cast<uint32_t>(min(p.total - base, static_cast<uint64_t>(tile_elems)));
+  const bool last = tile + 1 == p.num_tiles;
+  if (!p.tile_seg) find_segments(p.offsets, p.num_segments, base, base + in_range, last, s_range);
 
-  const bool full = p.vec_io && (base + tile_elems <= p.total);
+  const bool full = p.vec_io && in_range == tile_elems;
   W v[R][VEC];
   u32x4 q[R];
   if (full) {
@@ -717,32 +863,51 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
     for (int r = 0; r < R; ++r)
 #pragma unroll
       for (int k = 0; k < VEC; ++k) {
-        const uint64_t idx = base + static_cast<uint64_t>(r * B + tid) * VEC + k;
-        v[r][k] = (idx < p.total) ? elem_traits<T>::to_work(p.in[idx]) : id;
+        const uint32_t i = static_cast<uint32_t>(r * B + tid) * VEC + k;
+        v[r][k] = (i < in_range) ? elem_traits<T>::to_work(p.in[base + i]) : id;
       }
   }
-  for (uint32_t i = tid; i < head_words; i += B) s_heads[i] = 0;
-  if (s_lo >= p.num_segments) s_lo = p.num_segments - 1;
-  if (s_hi >= p.num_segments) s_hi = p.num_segments - 1;
-  if (s_hi < s_lo) s_hi = s_lo;
-  // Segments s_lo..s_hi touch the tile; their offsets and the next one's.
-  const uint64_t n_seg = s_hi - s_lo + 1;
-  const bool off_in_lds = n_seg + 1 <= off_cap;
-  if (off_in_lds)
-    for (uint64_t i = tid; i <= n_seg; i += B) s_off[i] = clamp_off(p.offsets, s_lo + i, p.total);
-  __syncthreads();
-  // The tile's head bits (tile elements 0..tile_elems), marked from the
-  // offsets: a reduction needs no global head bitmap, so its plan has no
-  // bitmap to clear and fill.
-  for (uint64_t i = tid; i < n_seg; i += B) {
-    const uint64_t b = off_in_lds ? s_off[i] : clamp_off(p.offsets, s_lo + i, p.total);
-    const uint64_t e = off_in_lds ? s_off[i + 1] : clamp_off(p.offsets, s_lo + i + 1, p.total);
-    if (e > b && b >= base && b - base <= tile_elems) {
-      const uint64_t pos = b - base;
-      atomicOr(&s_heads[pos >> 5], 1u << (pos & 31));
-    }
+  // Scalar loads, which do not wait for the data as vector loads would (those
+  // return in order); nothing writes what they read while the kernel runs.
+  uint32_t lo, hi;
+  if (p.tile_seg) {
+    const constant_u32 table = (constant_u32)p.tile_seg;
+    lo = table[tile];
+    hi = table[tile + 1];
+    // malformed offsets can leave entries of the table unwritten
+    lo = min(lo, static_cast<uint32_t>(p.num_segments));
+    hi = min(hi, static_cast<uint32_t>(p.num_segments));
+  } else {
+    __syncthreads();
+    lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s_range[0]));
+    hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(s_range[1]));
   }
-  __syncthreads();
+  const uint32_t owned = hi > lo ? hi - lo : 0;  // segments lo .. lo + owned - 1
+  // The start of segment lo + i in the tile; in_range + 1 beyond its end.
+  auto in_tile = [&](uint64_t o) -> uint32_t {
+    o = min(o, p.total);
+    return o <= base ? 0u : static_cast<uint32_t>(min(o - base, static_cast<uint64_t>(in_range) + 1));
+  };
+  auto load_off = [&](uint32_t i) { return in_tile(p.offsets[static_cast<uint64_t>(lo) + i]); };
+  const bool off_in_lds = owned + 1 <= off_cap;
+  const bool few = owned < max_pieces;
+  if (!few) {
+    for (uint32_t i = tid; i < (tile_elems >> 5); i += B) s_heads[i] = 0;
+    if (off_in_lds)
+      for (uint32_t i = tid; i <= owned; i += B) s_off[i] = load_off(i);
+  }
+  auto off = [&](uint32_t i) { return off_in_lds ? s_off[i] : load_off(i); };
+  // Few segments start in the tile: up to max_pieces plain folds, of the
+  // elements before the first start, between two starts, and after the last.
+  uint32_t start[max_pieces];
+  if (few) {
+    const constant_u64 offsets = (constant_u64)p.offsets;
+    uint64_t o[max_pieces];
+#pragma unroll
+    for (uint32_t j = 0; j < max_pieces; ++j) o[j] = offsets[min(static_cast<uint64_t>(lo) + j, p.num_segments)];
+#pragma unroll
+    for (uint32_t j = 0; j < max_pieces; ++j) start[j] = j <= owned ? in_tile(o[j]) : in_range + 1;
+  }
   if (full) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -752,23 +917,77 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
       for (int k = 0; k < VEC; ++k) v[r][k] = elem_traits<T>::to_work(tmp[k]);
     }
   }
-
-  auto head_at = [&](uint64_t pos) -> uint32_t {
-    return (s_heads[pos >> 5] >> (pos & 31)) & 1u;
-  };
-  // Largest s in [s_lo, s_hi] with offsets[s] <= e.
-  auto segment_of = [&](uint64_t e) -> uint64_t {
-    if (!off_in_lds) return find_segment(p.offsets, s_lo, s_hi, e, p.total);
-    uint64_t lo = 0, hi = s_hi - s_lo;
-    while (lo < hi) {
-      const uint64_t mid = (lo + hi + 1) / 2;
-      if (s_off[mid] <= e)
-        lo = mid;
-      else
-        hi = mid - 1;
+  if (few) {
+    auto piece_of = [&](uint32_t i) {
+      uint32_t piece = 0;
+#pragma unroll
+      for (uint32_t j = 0; j + 1 < max_pieces; ++j) piece += (j < owned && i >= start[j]) ? 1u : 0u;
+      return piece;
+    };
+    W acc[max_pieces];
+#pragma unroll
+    for (uint32_t j = 0; j < max_pieces; ++j) acc[j] = id;
+    const uint32_t wave_first = __builtin_amdgcn_readfirstlane(w) * 64u * VEC;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      // a wave's 64 vectors of a row lie in one piece unless a segment starts there
+      const uint32_t c = r * B * VEC + wave_first;
+      const uint32_t piece = piece_of(c);
+      if (piece == piece_of(c + 64 * VEC - 1)) {
+        W x = v[r][0];
+#pragma unroll
+        for (int k = 1; k < VEC; ++k) x = Op::apply(x, v[r][k]);
+#pragma unroll
+        for (uint32_t j = 0; j < max_pieces; ++j)
+          if (piece == j) acc[j] = Op::apply(acc[j], x);
+      } else {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+          const uint32_t mine = piece_of(c + lane * VEC + k);
+#pragma unroll
+          for (uint32_t j = 0; j < max_pieces; ++j) acc[j] = Op::apply(acc[j], mine == j ? v[r][k] : id);
+        }
+      }
     }
-    return s_lo + lo;
-  };
+#pragma unroll
+    for (uint32_t j = 0; j < max_pieces; ++j) {
+      if (j <= owned) {
+        const W x = wave::reduce_full<Op>(acc[j]);
+        if (lane == 0) s_piece[j][w] = x;
+      }
+    }
+    __syncthreads();
+    if (w == 0) {
+      uint32_t tail_seg = no_segment;
+#pragma unroll
+      for (uint32_t j = 0; j < max_pieces; ++j) {
+        if (j <= owned) {
+          const W x = wave::reduce_full<Op>(lane < nw ? s_piece[j][lane] : id);
+          if (j == 0) {
+            if (lane == 0) parts.head[tile] = x;
+          } else {
+            const uint64_t s = static_cast<uint64_t>(lo) + j - 1;
+            const uint32_t b = start[j > 0 ? j - 1 : 0], e = start[j];
+            if (e > b && e > in_range) {
+              tail_seg = static_cast<uint32_t>(s);
+              if (lane == 0) parts.tail[tile] = x;
+            } else if (lane == 0) {
+              p.out[s] = static_cast<T>(e > b ? Op::apply(p.init, x) : p.init);
+            }
+          }
+        }
+      }
+      if (lane == 0) parts.tail_seg[tile] = tail_seg;
+    }
+    return;
+  }
+
+  __syncthreads();
+  for (uint32_t i = tid; i < owned; i += B) {
+    const uint32_t b = off(i);
+    if (b < in_range) atomicOr(&s_heads[b >> 5], 1u << (b & 31));
+  }
+  __syncthreads();
 
   const uint32_t fm = row_head_bits<R, VEC>(s_heads, tid, B);
 #pragma unroll
@@ -787,103 +1006,159 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
     (void)av;
   }
   __syncthreads();
-  const uint64_t tile_left = p.total - base;  // > 0: the tile holds elements
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     // The elements hold the fold from their wave's row start (or segment
     // start); Pv is the (row r, wave w) prefix inside the tile, cut off by
-    // a segment start in an earlier lane.
+    // a segment start in an earlier lane or among elements 0..k.
     const uint32_t rowf = (fm >> (r * VEC)) & ((1u << VEC) - 1u);
     const bool wcut = (xcut >> r) & 1u;
-    const uint32_t Pf = s_tf[r * nw + w] | (wcut ? 1u : 0u);
     const W Pv = s_tv[r * nw + w];
-    const uint64_t l0 = static_cast<uint64_t>(r * B + tid) * VEC;  // index inside the tile
-    // Bit k: element k of the vector is the last of its segment in this
-    // tile (a segment start follows, or the data or the tile ends there).
-    uint32_t ends = (rowf >> 1) | (head_at(l0 + VEC) << (VEC - 1));
-    if (l0 + VEC == tile_elems) ends |= 1u << (VEC - 1);
-    if (l0 < tile_left && tile_left <= l0 + VEC) ends |= 1u << (tile_left - 1 - l0);
-    if (tile_left <= l0) ends = 0;
-    else if (tile_left < l0 + VEC) ends &= (1u << (tile_left - l0)) - 1u;
-    if (ends == 0) continue;
+    W o[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
-      if (!((ends >> k) & 1u)) continue;
-      const uint64_t e = base + l0 + k;
-      // a segment start among elements 0..k of the vector cuts the prefix off
       const bool cut = wcut || (rowf & ((2u << k) - 1u)) != 0u;
-      const W val = cut ? v[r][k] : Op::apply(Pv, v[r][k]);
-      const bool next_head = (e + 1 == p.total) || head_at(l0 + k + 1);
-      if (cut || Pf) {  // a segment start lies in [tile start, e]
-        if (next_head) {
-          const uint64_t s = segment_of(e);
-          p.out[s] = static_cast<T>(Op::apply(p.init, val));
-        } else {
-          tail_part[tile] = val;  // the tile's last element; the segment goes on
-        }
-      } else {
-        head_part[tile] = val;
-      }
+      o[k] = cut ? v[r][k] : Op::apply(Pv, v[r][k]);
     }
+    u32x4 qv;
+    __builtin_memcpy(&qv, o, 16);
+    reinterpret_cast<u32x4 *>(s_val)[r * B + tid] = qv;
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < owned; i += B) {
+    const uint32_t b = off(i);
+    const uint32_t e = off(i + 1);
+    const uint64_t s = static_cast<uint64_t>(lo) + i;
+    if (e <= b)
+      p.out[s] = static_cast<T>(p.init);
+    else if (e <= in_range)
+      p.out[s] = static_cast<T>(Op::apply(p.init, s_val[e - 1]));
+  }
+  if (tid == 0) {
+    const uint32_t first = off(0);
+    if (first > 0 && first <= in_range) parts.head[tile] = s_val[first - 1];
+    const bool tail = off(owned) > in_range;
+    if (tail) parts.tail[tile] = s_val[in_range - 1];
+    parts.tail_seg[tile] = tail ? lo + owned - 1 : no_segment;
   }
 }
 
-// op(init, tail_part[tb] . head_part[tb+1] . ... . head_part[tl]) for every
-// segment whose elements span tiles tb < tl.
+// op(init, tail[tb] . head[tb+1] . ... . head[tl]) for every segment that
+// continues from tile tb to tile tl > tb: one work-item per tile tb, a wave
+// for a segment of more than serial_span tiles, the whole group above
+// wave_span.  (One work-item per segment and eight partials in flight: 18 us
+// for 48 segments of 250 tiles, 3.1 ms for one segment of 65,536.)
 template <class T, class Op>
-__global__ void segmented_fixup_kernel(params<T> p, const typename elem_traits<T>::work *head_part,
-                                       const typename elem_traits<T>::work *tail_part, uint64_t tile_elems) {
+__global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
+                                                               reduce_parts<typename elem_traits<T>::work> parts,
+                                                               uint64_t tile_elems) {
   using W = typename elem_traits<T>::work;
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t s = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; s < p.num_segments;
-       s += stride) {
-    const uint64_t b = clamp_off(p.offsets, s, p.total);
-    const uint64_t e = clamp_off(p.offsets, s + 1, p.total);
-    if (e <= b) continue;
-    const uint64_t tb = b / tile_elems;
-    const uint64_t tl = (e - 1) / tile_elems;
-    if (tb == tl || tl >= p.num_tiles) continue;
-    W acc = tail_part[tb];
-    uint64_t t = tb + 1;
-    // Eight partials in flight per step, folded in tile order.
-    for (; t + 8 <= tl + 1; t += 8) {
-      W h[8];
+  constexpr uint32_t serial_span = 16;
+  constexpr uint32_t wave_span = 1024;
+  constexpr uint32_t max_list = 64;  // a group's tiles start at most 61 such segments
+  __shared__ uint32_t s_count;
+  __shared__ uint32_t s_tile[max_list];
+  __shared__ uint32_t s_last[max_list];
+  __shared__ W s_red[max_waves];
+  const W id = Op::identity();
+  const int w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) s_count = 0;
+  __syncthreads();
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t s = t + 1 < p.num_tiles ? parts.tail_seg[t] : no_segment;
+  if (s < p.num_segments) {
+    const uint64_t e = clamp_off(p.offsets, static_cast<uint64_t>(s) + 1, p.total);
+    const uint32_t tl = e ? static_cast<uint32_t>((e - 1) / tile_elems) : 0;
+    uint32_t slot = max_list;
+    if (tl > t + serial_span) slot = atomicAdd(&s_count, 1u);
+    if (slot < max_list) {
+      s_tile[slot] = t;
+      s_last[slot] = tl;
+    } else if (tl > t) {
+      W acc = parts.tail[t];
+      uint32_t u = t + 1;
+      for (; u + 4 <= tl + 1; u += 4) {
+        W h[4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) h[u] = head_part[t + u];
+        for (int j = 0; j < 4; ++j) h[j] = parts.head[u + j];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) acc = Op::apply(acc, h[u]);
+        for (int j = 0; j < 4; ++j) acc = Op::apply(acc, h[j]);
+      }
+      for (; u <= tl; ++u) acc = Op::apply(acc, parts.head[u]);
+      p.out[s] = static_cast<T>(Op::apply(p.init, acc));
     }
-    for (; t <= tl; ++t) acc = Op::apply(acc, head_part[t]);
-    p.out[s] = static_cast<T>(Op::apply(p.init, acc));
+  }
+  __syncthreads();
+  const uint32_t count = min(s_count, max_list);
+  // `lanes` work-items fold head[tb + 1 .. tl], four partials in flight each.
+  auto fold = [&](uint32_t tb, uint32_t tl, uint32_t me, uint32_t lanes) {
+    W acc[4] = {id, id, id, id};
+    uint64_t u = static_cast<uint64_t>(tb) + 1 + me;
+    for (; u + 3ull * lanes <= tl; u += 4ull * lanes) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] = Op::apply(acc[j], parts.head[u + static_cast<uint64_t>(j) * lanes]);
+    }
+    for (; u <= tl; u += lanes) acc[0] = Op::apply(acc[0], parts.head[u]);
+    return wave::reduce_full<Op>(Op::apply(Op::apply(acc[0], acc[1]), Op::apply(acc[2], acc[3])));
+  };
+  auto finish = [&](uint32_t tb, W rest) {
+    p.out[parts.tail_seg[tb]] = static_cast<T>(Op::apply(p.init, Op::apply(parts.tail[tb], rest)));
+  };
+  for (uint32_t i = w; i < count; i += blockDim.x >> 6) {
+    if (s_last[i] - s_tile[i] > wave_span) continue;
+    const W x = fold(s_tile[i], s_last[i], lane, 64);
+    if (lane == 0) finish(s_tile[i], x);
+  }
+  for (uint32_t i = 0; i < count; ++i) {
+    if (s_last[i] - s_tile[i] <= wave_span) continue;
+    W x = fold(s_tile[i], s_last[i], threadIdx.x, blockDim.x);
+    __syncthreads();
+    if (lane == 0) s_red[w] = x;
+    __syncthreads();
+    if (w == 0) {
+      x = wave::reduce_full<Op>(lane < static_cast<int>(blockDim.x >> 6) ? s_red[lane] : id);
+      if (lane == 0) finish(s_tile[i], x);
+    }
   }
 }
 
 // --------------------------------------------------------------------------
 // Host side
 // --------------------------------------------------------------------------
-// Default tile when the caller gives no configuration, by total element
-// count and element size.  Read off the first 400 of 500 segmented shapes
-// up to 2^28 elements timed on MI355X (the tuner's timing database); on the
-// other 100 it has a mean regret of ~4 % against the best of the 15
-// configurations, where any single fixed tile has 15-70 %.
+// Default tile when the caller gives no configuration, by element count,
+// element size and total bytes.  Read off timings on MI355X of every tile
+// from 128 x 2 to 1024 x 8 at 2 x 10^4 .. 3 x 10^7 elements (4 and 8 bytes,
+// segments of 50 and of 3000 elements and 40 segments), and above from the
+// tuner's timing database:
 //   scan:   n < 2^16: 256 x 2;  n < 2^20: 512 x 2 (8-byte: 1024 x 2);
-//           n < 2^26: 512 x 8;  otherwise 1024 x 8
-//   reduce: n < 2^16: 128 x 2;  n < 2^20: 256 x 2;  n < 2^24: 1024 x 2;
-//           otherwise 256 x 4 (8-byte: 512 x 4)
-// Large scans take 8-row tiles (two 512-wide or one 1024-wide group per CU,
-// 123 VGPRs for int64); large reductions take 4-row tiles, which leave room
-// for several groups per CU (the reduction's groups never wait for each
-// other).
-inline uint32_t default_work_group(bool reduce, uint64_t total, int elem_bytes) {
-  if (total < (1ull << 16)) return reduce ? 128 : 256;
-  if (total < (1ull << 20)) return reduce ? 256 : (elem_bytes == 8 ? 1024 : 512);
-  if (reduce) return total < (1ull << 24) ? 1024 : (elem_bytes == 8 ? 512 : 256);
-  return total < (1ull << 26) ? 512 : 1024;
-}
-inline int default_rows(bool reduce, uint64_t total) {
-  if (total < (1ull << 20)) return 2;
-  if (reduce) return total < (1ull << 24) ? 2 : 4;
-  return 8;
+//           < 12 MiB: 1024 x 2;  < 64 MiB: 1024 x 4;  n < 2^26: 512 x 8;
+//           otherwise 1024 x 8
+//   reduce: n < 2^16: 128 x 2;  n < 2^20: 256 x 2;  < 20 MiB: 1024 x 2;
+//           < 48 MiB: 1024 x 4;  otherwise 256 x 4 (8-byte: 512 x 4)
+// 2-row scans of up to max_search_tiles tiles and reductions of as many
+// tiles need one launch less, so the tiles grow with the input as long as
+// they stay below that (2^20 fp32 scan: 8.5 us at 1024 x 2, 11.6 us at 512 x
+// 8; 2^23 fp32 reduction: 11.9 us at 1024 x 4, 14.7 us at 1024 x 2).  Large
+// scans take 8-row tiles (two 512-wide or one 1024-wide group per CU, 123
+// VGPRs for int64); large reductions take 4-row tiles, which leave room for
+// several groups per CU (the reduction's groups never wait for each other).
+inline void default_tile(bool reduce, uint64_t total, int elem_bytes, uint32_t &wg, int &rows) {
+  const bool wide = elem_bytes == 8;
+  const uint64_t mib = total * elem_bytes >> 20;
+  if (total < (1ull << 20)) {
+    rows = 2;
+    if (total < (1ull << 16))
+      wg = reduce ? 128 : 256;
+    else
+      wg = reduce ? 256 : (wide ? 1024 : 512);
+  } else if (reduce) {
+    rows = mib < 20 ? 2 : 4;
+    wg = mib < 48 ? 1024 : (wide ? 512 : 256);
+  } else {
+    rows = mib < 12 ? 2 : mib < 64 ? 4 : 8;
+    wg = (mib < 64 || total >= (1ull << 26)) ? 1024 : 512;
+  }
 }
 
 template <class T, class Op>
@@ -894,7 +1169,6 @@ struct launch_plan {
   uint32_t grid = 1;
   size_t lds = 0;
   uint64_t tile_elems = 0;
-  uint32_t *tile_seg = nullptr;
   uint32_t *heads = nullptr;
   uint64_t head_words = 0;
   void *region = nullptr;
@@ -903,37 +1177,52 @@ struct launch_plan {
   size_t region_cap = 0;
 };
 
-template <class T, class Op, int R>
+// Tiles up to which a work-group finds its segments by itself: the launch of
+// the kernel that does it for all tiles costs more (about 3.5 us) than the
+// searches, which a few hundred resident groups overlap.
+constexpr uint64_t max_search_tiles = 1024;
+// Segments per tile up to which the segments write the tiles' table.
+constexpr uint64_t max_scatter_ratio = 16;
+
+template <class T, class Op, int R, bool MARK>
 acpp_status launch_rows(launch_plan<T, Op> &lp, hipStream_t stream, const char *name) {
-  acpp_status st = fill_zero(lp.heads, lp.head_words * sizeof(uint32_t), stream);
-  if (st != ACPP_SUCCESS) return st;
-  hipLaunchKernelGGL(setup_kernel<T>, dim3(static_cast<uint32_t>(std::min<uint64_t>(ceil_div(lp.p.num_segments + 1, 256), 4096))),
-                     dim3(256), 0, stream, lp.p, lp.tile_seg, lp.heads, lp.tile_elems);
-  st = check_launch(name);
-  if (st != ACPP_SUCCESS) return st;
-  hipLaunchKernelGGL((segmented_kernel<T, Op, R>), dim3(lp.grid), dim3(lp.wg), lp.lds, stream, lp.p);
+  if constexpr (!MARK) {
+    hipLaunchKernelGGL(head_bitmap_kernel, dim3(static_cast<uint32_t>(ceil_div(lp.head_words, head_chunk_words))),
+                       dim3(256), 0, stream, lp.p.offsets, lp.p.num_segments, lp.p.total, lp.head_words, lp.heads);
+    acpp_status st = check_launch(name);
+    if (st != ACPP_SUCCESS) return st;
+  }
+  hipLaunchKernelGGL((segmented_kernel<T, Op, R, MARK>), dim3(lp.grid), dim3(lp.wg), lp.lds, stream, lp.p);
   return check_launch(name);
 }
 
-// Segmented reduction: set up (tile -> first segment, init into empty
-// segments), one work-group per tile (its head bits marked in LDS from the
-// offsets, so no global bitmap is cleared or filled), then the fix-up of
-// segments that span tiles.
+// Segmented reduction: the table of the tiles' first segments (many tiles
+// only), one work-group per tile, then the fix-up of segments that span
+// tiles.
 template <class T, class Op>
 acpp_status enqueue_reduce(acpp_allocation_group *g, launch_plan<T, Op> &lp, hipStream_t stream, const T *in,
                            T *out, const uint64_t *offsets, uint64_t num_segments, uint64_t total,
                            typename elem_traits<T>::work init, uint64_t num_tiles, const char *name) {
   using W = typename elem_traits<T>::work;
-  void *parts = nullptr;
-  acpp_status st = group_obtain(g, 2 * num_tiles * sizeof(W), &parts);
+  void *scratch = nullptr;
+  acpp_status st = group_obtain(g, num_tiles * (2 * sizeof(W) + sizeof(uint32_t)), &scratch);
   if (st != ACPP_SUCCESS) return st;
-  W *head_part = static_cast<W *>(parts);
-  W *tail_part = head_part + num_tiles;
+  reduce_parts<W> parts;
+  parts.head = static_cast<W *>(scratch);
+  parts.tail = parts.head + num_tiles;
+  parts.tail_seg = reinterpret_cast<uint32_t *>(parts.tail + num_tiles);
+  uint32_t *table = nullptr;
+  if (num_tiles > max_search_tiles) {
+    void *ts = nullptr;
+    st = group_obtain(g, (num_tiles + 1) * sizeof(uint32_t), &ts);
+    if (st != ACPP_SUCCESS) return st;
+    table = static_cast<uint32_t *>(ts);
+  }
   params<T> &p = lp.p;
   p.in = in;
   p.out = out;
   p.offsets = offsets;
-  p.tile_seg = lp.tile_seg;
+  p.tile_seg = table;
   p.heads = nullptr;  // the reduce kernel marks its heads from the offsets
   p.head_words_total = 0;
   p.block_lookback = 0;
@@ -941,7 +1230,6 @@ acpp_status enqueue_reduce(acpp_allocation_group *g, launch_plan<T, Op> &lp, hip
   p.num_segments = num_segments;
   p.total = total;
   p.init = init;
-  p.reduce = 1;
   p.vec_io = (reinterpret_cast<uintptr_t>(in) & 3) == 0;
   p.num_tiles = static_cast<uint32_t>(num_tiles);
   p.epoch = 0;
@@ -950,28 +1238,28 @@ acpp_status enqueue_reduce(acpp_allocation_group *g, launch_plan<T, Op> &lp, hip
   p.status = nullptr;
   lp.grid = static_cast<uint32_t>(num_tiles);
 
-  hipLaunchKernelGGL(setup_kernel<T>, dim3(static_cast<uint32_t>(std::min<uint64_t>(ceil_div(num_segments + 1, 256), 4096))),
-                     dim3(256), 0, stream, p, lp.tile_seg, static_cast<uint32_t *>(nullptr), lp.tile_elems);
-  st = check_launch(name);
-  if (st != ACPP_SUCCESS) return st;
-  if (total > 0) {
-    if (lp.rows == 2)
-      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 2>), dim3(lp.grid), dim3(lp.wg), lp.lds, stream, p,
-                         head_part, tail_part);
-    else if (lp.rows == 4)
-      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 4>), dim3(lp.grid), dim3(lp.wg), lp.lds, stream, p,
-                         head_part, tail_part);
+  if (table) {
+    if (num_segments <= max_scatter_ratio * num_tiles && num_tiles <= 8 * num_segments)
+      hipLaunchKernelGGL(tile_scatter_kernel, dim3(static_cast<uint32_t>(ceil_div(num_segments, 256))), dim3(256), 0,
+                         stream, offsets, num_segments, lp.tile_elems, p.num_tiles, table);
     else
-      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 8>), dim3(lp.grid), dim3(lp.wg), lp.lds, stream, p,
-                         head_part, tail_part);
+      hipLaunchKernelGGL(tile_table_kernel, dim3(static_cast<uint32_t>(ceil_div(num_tiles + 1, 256))), dim3(256), 0,
+                         stream, offsets, num_segments, lp.tile_elems, p.num_tiles, table);
     st = check_launch(name);
     if (st != ACPP_SUCCESS) return st;
-    hipLaunchKernelGGL((segmented_fixup_kernel<T, Op>),
-                       dim3(static_cast<uint32_t>(std::min<uint64_t>(ceil_div(num_segments, 256), 4096))), dim3(256), 0,
-                       stream, p, head_part, tail_part, lp.tile_elems);
-    st = check_launch(name);
   }
-  return st;
+  const size_t lds = reduce_head_words(static_cast<uint32_t>(lp.tile_elems)) * 4 + lp.tile_elems * sizeof(W);
+  if (lp.rows == 2)
+    hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 2>), dim3(lp.grid), dim3(lp.wg), lds, stream, p, parts);
+  else if (lp.rows == 4)
+    hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 4>), dim3(lp.grid), dim3(lp.wg), lds, stream, p, parts);
+  else
+    hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 8>), dim3(lp.grid), dim3(lp.wg), lds, stream, p, parts);
+  st = check_launch(name);
+  if (st != ACPP_SUCCESS || num_tiles == 1) return st;
+  hipLaunchKernelGGL((segmented_fixup_kernel<T, Op>), dim3(static_cast<uint32_t>(ceil_div(num_tiles, 1024))),
+                     dim3(1024), 0, stream, p, parts, lp.tile_elems);
+  return check_launch(name);
 }
 
 template <class T, class Op>
@@ -985,10 +1273,11 @@ acpp_status enqueue(acpp_allocation_group *g, hipStream_t stream, const T *in, T
   acpp_status st = enter_device(g, &cus);
   if (st != ACPP_SUCCESS) return st;
   launch_plan<T, Op> lp;
-  lp.wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : default_work_group(reduce, total, static_cast<int>(sizeof(T)));
+  default_tile(reduce, total, static_cast<int>(sizeof(T)), lp.wg, lp.rows);
+  if (cfg && cfg->work_group_size) lp.wg = cfg->work_group_size;
   if (!valid_work_group_size(lp.wg))
     return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
-  lp.rows = (cfg && cfg->items_per_thread) ? static_cast<int>(cfg->items_per_thread) : default_rows(reduce, total);
+  if (cfg && cfg->items_per_thread) lp.rows = static_cast<int>(cfg->items_per_thread);
   if (lp.rows != 2 && lp.rows != 4 && lp.rows != 8)
     return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": items_per_thread must be 2, 4 or 8");
   lp.tile_elems = static_cast<uint64_t>(lp.wg) * lp.rows * VEC;
@@ -999,17 +1288,17 @@ acpp_status enqueue(acpp_allocation_group *g, hipStream_t stream, const T *in, T
   // bits it needs, since rows x 16-byte vector <= 32 elements)
   lp.lds = std::max<size_t>(static_cast<size_t>((lp.tile_elems + 1 + 31) / 32), 2 * static_cast<size_t>(lp.wg)) * 4;
 
-  void *ts = nullptr;
-  st = group_obtain(g, (num_tiles + 1) * sizeof(uint32_t), &ts);
-  if (st != ACPP_SUCCESS) return st;
-  lp.tile_seg = static_cast<uint32_t *>(ts);
   if (reduce) return enqueue_reduce<T, Op>(g, lp, stream, in, out, offsets, num_segments, total, init, num_tiles, name);
-  // Head bitmap over elements [0, total] plus one spare word (scans).
-  lp.head_words = (total + 1 + 31) / 32 + 1;
-  void *hb = nullptr;
-  st = group_obtain(g, lp.head_words * sizeof(uint32_t), &hb);
-  if (st != ACPP_SUCCESS) return st;
-  lp.heads = static_cast<uint32_t *>(hb);
+  // Small inputs (2-row tiles) mark their segment starts in the scan kernel.
+  const bool mark = lp.rows == 2 && num_tiles <= max_search_tiles;
+  if (!mark) {
+    // Head bitmap over elements [0, total] plus one spare word.
+    lp.head_words = (total + 1 + 31) / 32 + 1;
+    void *hb = nullptr;
+    st = group_obtain(g, lp.head_words * sizeof(uint32_t), &hb);
+    if (st != ACPP_SUCCESS) return st;
+    lp.heads = static_cast<uint32_t *>(hb);
+  }
   using SIO = seg_status<typename elem_traits<T>::work>;
   static_assert(SIO::words <= seg_stride_words, "status slot too small");
   lp.region_used = sizeof(sync_header) + num_tiles * seg_stride_words * sizeof(uint64_t);
@@ -1024,7 +1313,7 @@ acpp_status enqueue(acpp_allocation_group *g, hipStream_t stream, const T *in, T
   p.in = in;
   p.out = out;
   p.offsets = offsets;
-  p.tile_seg = lp.tile_seg;
+  p.tile_seg = nullptr;
   p.heads = lp.heads;
   p.head_words_total = lp.head_words;
   p.block_lookback = (cfg && (cfg->flags & ACPP_VARIANT_BLOCK_LOOKBACK)) ? 1 : 0;
@@ -1032,8 +1321,7 @@ acpp_status enqueue(acpp_allocation_group *g, hipStream_t stream, const T *in, T
   p.num_segments = num_segments;
   p.total = total;
   p.init = init;
-  p.reduce = reduce ? 1 : 0;
-  p.vec_io = ((reinterpret_cast<uintptr_t>(in) | (reduce ? 0 : reinterpret_cast<uintptr_t>(out))) & 3) == 0;
+  p.vec_io = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3) == 0;
   p.num_tiles = static_cast<uint32_t>(num_tiles);
   p.epoch = rl.epoch;
   p.ticket_base = rl.ticket_base;
@@ -1060,17 +1348,22 @@ acpp_status enqueue(acpp_allocation_group *g, hipStream_t stream, const T *in, T
     lp.grid = static_cast<uint32_t>(std::min<uint64_t>(cap, num_tiles));
     return ACPP_SUCCESS;
   };
+  auto run = [&](auto rows_tag, auto mark_tag) -> acpp_status {
+    constexpr int R = decltype(rows_tag)::value;
+    constexpr bool MARK = decltype(mark_tag)::value;
+    acpp_status e = pick(segmented_kernel<T, Op, R, MARK>);
+    return e == ACPP_SUCCESS ? launch_rows<T, Op, R, MARK>(lp, stream, name) : e;
+  };
+  using std::integral_constant;
   acpp_status s;
-  if (lp.rows == 2) {
-    if ((s = pick(segmented_kernel<T, Op, 2>)) != ACPP_SUCCESS) return s;
-    s = launch_rows<T, Op, 2>(lp, stream, name);
-  } else if (lp.rows == 4) {
-    if ((s = pick(segmented_kernel<T, Op, 4>)) != ACPP_SUCCESS) return s;
-    s = launch_rows<T, Op, 4>(lp, stream, name);
-  } else {
-    if ((s = pick(segmented_kernel<T, Op, 8>)) != ACPP_SUCCESS) return s;
-    s = launch_rows<T, Op, 8>(lp, stream, name);
-  }
+  if (mark)
+    s = run(integral_constant<int, 2>{}, std::true_type{});
+  else if (lp.rows == 2)
+    s = run(integral_constant<int, 2>{}, std::false_type{});
+  else if (lp.rows == 4)
+    s = run(integral_constant<int, 4>{}, std::false_type{});
+  else
+    s = run(integral_constant<int, 8>{}, std::false_type{});
   // every work-group draws one ticket past the last tile before it exits
   end_region_launch(lp.rs, rl, static_cast<uint32_t>(num_tiles) + lp.grid, s);
   return s;

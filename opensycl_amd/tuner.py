@@ -52,15 +52,19 @@ DEFAULT_CONFIG = (512, 4)
 
 def default_config(kind: str, n: int, dtype: str = "i32") -> tuple:
     """The library's own choice when no configuration is given: the size
-    and element-size rule of segmented.hip (default_work_group /
-    default_rows)."""
-    wide = DTYPES.get(dtype, 4) == 8
+    and element-size rule of segmented.hip (default_tile)."""
+    width = DTYPES.get(dtype, 4)
+    mib = n * width >> 20
     if n < (1 << 16):
         return (128, 2) if kind == "reduce" else (256, 2)
     if n < (1 << 20):
-        return (256, 2) if kind == "reduce" else ((1024, 2) if wide else (512, 2))
+        return (256, 2) if kind == "reduce" else ((1024, 2) if width == 8 else (512, 2))
     if kind == "reduce":
-        return (1024, 2) if n < (1 << 24) else ((512, 4) if wide else (256, 4))
+        if mib < 48:
+            return (1024, 2) if mib < 20 else (1024, 4)
+        return (512, 4) if width == 8 else (256, 4)
+    if mib < 64:
+        return (1024, 2) if mib < 12 else (1024, 4)
     return (512, 8) if n < (1 << 26) else (1024, 8)
 
 

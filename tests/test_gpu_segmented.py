@@ -254,3 +254,50 @@ def test_plan_keeps_its_group_and_buffers_alive(gpu, q):
     assert np.array_equal(host(yd), O.segmented_inclusive_scan(x, off))
     assert int(host(junk[2])[-1]) == 7 * n * (n + 1) // 2  # n < 2^23: no wrap
     plan.close()
+
+
+def _edge_layouts():
+    rng = np.random.default_rng(11)
+
+    def of(lens):
+        return np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+
+    yield "no_elements", of([0] * 300)
+    yield "one_element", of([0, 1, 0])
+    # starts on, before and after multiples of every tile size (512 .. 32768)
+    yield "tile_edges", of([511, 1, 0, 0, 512, 1023, 1, 2049, 0, 4095, 4096, 0, 8191, 1, 0, 32768, 32767, 0])
+    yield "three_and_four_starts", of([600, 700, 800] * 30 + [500, 500, 500, 500] * 30)
+    # more than 1024 starts in a tile, with empty segments
+    yield "ones_and_empty", of(rng.integers(0, 2, 60000))
+    # more than 4096 segments, fewer and more than 16 a tile, over 1024 tiles
+    # of the (64, 2) configuration below
+    yield "many_long", of(rng.integers(0, 400, 9000))
+    yield "many_short", of(rng.integers(0, 9, 400000))
+    # one segment over more than 1024 tiles, some over 17 .. 1024 tiles
+    yield "spans", of([3, 1 << 20, 0, 20000, 9000, 5, 500000, 77])
+
+
+# (64, 2): 512 (4-byte) or 256 (8-byte) elements a tile, so the table of the
+# tiles' segments and every span of the fix-up; default: the library's tiles
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.float64])
+@pytest.mark.parametrize("cfg", [(64, 2), (1024, 8), None])
+def test_segmented_edges(gpu, q, scratch, dtype, cfg):
+    torch, _ = gpu
+    for name, off in _edge_layouts():
+        n = int(off[-1])
+        # small integers: sums are exact in any order
+        x = _values(np.int32, n, seed=n + 2) % 1000 if n else np.zeros(0, np.int32)
+        x = x.astype(dtype)
+        xd, od = dev(torch, x), dev(torch, off)
+        xi = x.astype(np.int64)
+        for op, init in ((acpp.PLUS, 7), (acpp.MAX, -2000)):
+            out = torch.full((len(off) - 1,), -99, dtype=xd.dtype, device="cuda")
+            acpp.segmented_reduce(q, scratch, xd, od, out, init, op, config=cfg)
+            yd = torch.full_like(xd, -99)
+            acpp.segmented_inclusive_scan(q, scratch, xd, yd, od, op, config=cfg)
+            q.wait()
+            scratch.release()
+            exp = O.segmented_reduce(xi, off, np.int64(init), op)
+            assert np.array_equal(host(out).astype(np.int64), exp), (name, op)
+            if n:
+                assert np.array_equal(host(yd).astype(np.int64), O.segmented_inclusive_scan(xi, off, op)), (name, op)
