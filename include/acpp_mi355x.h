@@ -477,10 +477,11 @@ acpp_status acpp_segmented_reduce_i64(acpp_allocation_group *scratch, acpp_strea
 acpp_status acpp_segmented_reduce_f32(acpp_allocation_group *scratch, acpp_stream_t stream, const float *first, uint64_t n, const uint64_t *offsets, uint64_t num_segments, float *out, float init, acpp_algorithm_op op, const acpp_launch_config *config);
 acpp_status acpp_segmented_reduce_f64(acpp_allocation_group *scratch, acpp_stream_t stream, const double *first, uint64_t n, const uint64_t *offsets, uint64_t num_segments, double *out, double init, acpp_algorithm_op op, const acpp_launch_config *config);
 
-/* hipGraph plans: the same work captured once (setup kernel + persistent
-   kernel, scratch from `scratch`) and replayed with one graph launch.  The
-   plan references `scratch`, the input, output and offsets buffers: keep
-   them alive (and the group unreleased) while the plan is used. */
+/* Plans: the same work with its scratch (from `scratch`) and parameters kept,
+   enqueued by every launch.  The plan references `scratch`, the input, output
+   and offsets buffers: keep them alive (and the group unreleased) while the
+   plan is used; launches that may overlap need plans of their own.  A launch
+   may be captured into a graph. */
 typedef struct acpp_segmented_plan acpp_segmented_plan;
 acpp_status acpp_segmented_plan_inclusive_scan_i32(acpp_allocation_group *scratch, const int32_t *first, uint64_t n, int32_t *d_first, const uint64_t *offsets, uint64_t num_segments, acpp_algorithm_op op, const acpp_launch_config *config, acpp_segmented_plan **plan);
 acpp_status acpp_segmented_plan_inclusive_scan_i64(acpp_allocation_group *scratch, const int64_t *first, uint64_t n, int64_t *d_first, const uint64_t *offsets, uint64_t num_segments, acpp_algorithm_op op, const acpp_launch_config *config, acpp_segmented_plan **plan);

@@ -171,7 +171,7 @@ class AllocationGroup:
         check(lib.acpp_allocation_group_create(cache.handle, device, ctypes.byref(h)))
         self._h = h
         self._cache = cache
-        self._plans = 0             # live SegmentedPlans captured from this group
+        self._plans = 0             # live SegmentedPlans made from this group
         self._close_pending = False
 
     @property
@@ -186,7 +186,7 @@ class AllocationGroup:
 
     def release(self) -> None:
         """Return the group's regions to the cache now.  Refused while a
-        SegmentedPlan captured from this group is alive: its graph still
+        SegmentedPlan made from this group is alive: it still
         uses them, and replays would corrupt whichever call got them next."""
         if self._plans > 0:
             raise RuntimeError("AllocationGroup.release: a SegmentedPlan captured from this group is alive; "
@@ -203,7 +203,7 @@ class AllocationGroup:
 
     def close(self) -> None:
         """Return the group's regions to the cache.  While a SegmentedPlan
-        captured from this group is alive, its graph still uses them: the
+        made from this group is alive, it still uses them: the
         release then waits until the last such plan is closed."""
         if self._plans > 0:
             self._close_pending = True
@@ -577,10 +577,10 @@ def segmented_reduce(q: Queue, scratch: AllocationGroup, x, offsets, out, init=0
 
 
 class SegmentedPlan:
-    """A segmented scan or reduction captured into a hipGraph once and
-    replayed with ``launch``.
+    """A segmented scan or reduction whose scratch and parameters are kept
+    for every ``launch``.
 
-    The captured graph holds raw pointers to the input, output and offsets
+    The plan holds raw pointers to the input, output and offsets
     tensors and to scratch regions of the allocation group, so the plan
     keeps references to all of them (and to the group's cache) for as long
     as it lives: a replay never touches freed or reissued memory."""

@@ -211,6 +211,10 @@ uint32_t *host_trip_flag_if_allocated(int device);
 acpp_status group_obtain_sync(acpp_allocation_group *g, size_t bytes,
                               hipStream_t stream, void **out,
                               size_t *capacity_bytes, region_state **state = nullptr);
+// The same before any stream is known: a fresh region is cleared by its first
+// launch.
+acpp_status group_obtain_sync_uncleared(acpp_allocation_group *g, size_t bytes, void **out, size_t *capacity_bytes,
+                                        region_state **state);
 
 // Zero `bytes` of device memory with a kernel (also inside stream capture,
 // where memset nodes are avoided).

@@ -231,9 +231,10 @@ acpp_status group_obtain(acpp_allocation_group *g, size_t bytes, void **out) {
   return ACPP_SUCCESS;
 }
 
-acpp_status group_obtain_sync(acpp_allocation_group *g, size_t bytes,
-                              hipStream_t stream, void **out,
-                              size_t *capacity_bytes, region_state **state) {
+namespace {
+// `stream`: where a fresh region is cleared; NULL: by its first launch.
+acpp_status obtain_sync(acpp_allocation_group *g, size_t bytes, const hipStream_t *stream, void **out,
+                        size_t *capacity_bytes, region_state **state) {
   if (g->parent->type != ACPP_ALLOCATION_DEVICE && g->parent->type != ACPP_ALLOCATION_SHARED)
     return set_error(ACPP_ERROR_INVALID_ARGUMENT,
                      "kernels need device-accessible scratch; use an "
@@ -252,13 +253,13 @@ acpp_status group_obtain_sync(acpp_allocation_group *g, size_t bytes,
     if (s != ACPP_SUCCESS) return s;
     a.sync = true;
     a.state = std::make_shared<region_state>();
-    if (stream_is_capturing(stream)) {
+    if (!stream || stream_is_capturing(*stream)) {
       // The captured launch clears the part it uses (begin_region_launch
       // under capture), and the first eager launch clears all of it: a
       // clear here would be a second one in every replay of the graph.
       a.state->mode = region_state::graph;
     } else {
-      s = reset_sync_region(a.ptr, a.size, g->dev, stream);
+      s = reset_sync_region(a.ptr, a.size, g->dev, *stream);
       if (s != ACPP_SUCCESS) {
         g->parent->deallocate(a);
         return s;
@@ -270,6 +271,18 @@ acpp_status group_obtain_sync(acpp_allocation_group *g, size_t bytes,
   *capacity_bytes = a.size;
   if (state) *state = a.state.get();
   return ACPP_SUCCESS;
+}
+}  // namespace
+
+acpp_status group_obtain_sync(acpp_allocation_group *g, size_t bytes,
+                              hipStream_t stream, void **out,
+                              size_t *capacity_bytes, region_state **state) {
+  return obtain_sync(g, bytes, &stream, out, capacity_bytes, state);
+}
+
+acpp_status group_obtain_sync_uncleared(acpp_allocation_group *g, size_t bytes, void **out, size_t *capacity_bytes,
+                                        region_state **state) {
+  return obtain_sync(g, bytes, nullptr, out, capacity_bytes, state);
 }
 
 acpp_status begin_region_launch(acpp_allocation_group *g, void *region, size_t used, size_t capacity,

@@ -27,9 +27,10 @@
 //     writes the totals of the segments it holds whole and two partial
 //     folds, and a fix-up kernel joins the partials of segments that span
 //     tiles (segmented_reduce_kernel below);
-//   - the setup and main kernels can be captured into a hipGraph once and
-//     replayed (acpp_segmented_plan_*).
+//   - a plan keeps a call's scratch and parameters (acpp_segmented_plan_*).
 #include <memory>
+#include <mutex>
+#include <new>
 
 #include "launch_util.hpp"
 
@@ -368,20 +369,19 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(const uint64_t *__res
 
 // The head bitmap of the scans: bit b for every segment start b < total (the
 // start of an empty segment is that of the next one that is not empty).  A
-// work-group marks head_chunk elements in LDS from the offsets inside its
+// work-group marks 32 x WORDS elements in LDS from the offsets inside its
 // range and writes the words once: the bitmap needs no clearing and no global
 // atomics.  (A fill, then one global atomicOr per segment: 2^26 elements in
 // 13.4 million segments took 450 us of 558.)
-constexpr uint32_t head_chunk_words = 1024;
-constexpr uint64_t head_chunk = 32ull * head_chunk_words;
+template <uint32_t WORDS>
 __global__ __launch_bounds__(256) void head_bitmap_kernel(const uint64_t *__restrict__ offsets, uint64_t num_segments,
                                                           uint64_t total, uint64_t head_words, uint32_t *heads) {
-  __shared__ uint32_t s_words[head_chunk_words];
+  __shared__ uint32_t s_words[WORDS];
   __shared__ uint64_t s_range[2];
-  const uint64_t base = blockIdx.x * head_chunk;
-  const uint64_t end = min(base + head_chunk, total);
+  const uint64_t base = blockIdx.x * 32ull * WORDS;
+  const uint64_t end = min(base + 32ull * WORDS, total);
   find_segments(offsets, num_segments, base, end, false, s_range);
-  for (uint32_t i = threadIdx.x; i < head_chunk_words; i += 256) s_words[i] = 0;
+  for (uint32_t i = threadIdx.x; i < WORDS; i += 256) s_words[i] = 0;
   __syncthreads();
   const uint64_t hi = s_range[1];
 #pragma unroll 4
@@ -390,8 +390,8 @@ __global__ __launch_bounds__(256) void head_bitmap_kernel(const uint64_t *__rest
     if (b >= base && b < end) atomicOr(&s_words[(b - base) >> 5], 1u << (b & 31));
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < head_chunk_words; i += 256) {
-    const uint64_t w = blockIdx.x * static_cast<uint64_t>(head_chunk_words) + i;
+  for (uint32_t i = threadIdx.x; i < WORDS; i += 256) {
+    const uint64_t w = blockIdx.x * static_cast<uint64_t>(WORDS) + i;
     if (w < head_words) heads[w] = s_words[i];
   }
 }
@@ -1161,218 +1161,236 @@ inline void default_tile(bool reduce, uint64_t total, int elem_bytes, uint32_t &
   }
 }
 
+// Tiles up to which a work-group finds its segments by itself: the launch of
+// the kernel that does it for all tiles costs more (about 3.5 us) than the
+// searches, which a few hundred resident groups overlap.
+constexpr uint64_t max_search_tiles = 1024;
+// Segments per tile up to which the segments write the tiles' table, and
+// tiles per segment: 2^23 fp32 in 2797 segments 16.7 us written, 19.3 us
+// searched; in 40 segments 20.6 and 17.5 us.
+constexpr uint64_t max_scatter_segments = 16;
+constexpr uint64_t max_scatter_tiles = 8;
+
+// A segmented call with its scratch, ready to be enqueued any number of
+// times (once by the calls, on every launch by a plan).
+struct prepared {
+  virtual ~prepared() = default;
+  virtual acpp_status enqueue(hipStream_t stream) = 0;
+  int device = 0;
+};
+
 template <class T, class Op>
-struct launch_plan {
+struct call : prepared {
+  using W = typename elem_traits<T>::work;
+  static constexpr int VEC = 16 / sizeof(T);
+  const char *name = "";
   params<T> p;
+  bool reduce = false;
+  bool mark = false;  // scans: segment starts are marked in the scan kernel
   uint32_t wg = 256;
   int rows = 8;
   uint32_t grid = 1;
   size_t lds = 0;
   uint64_t tile_elems = 0;
-  uint32_t *heads = nullptr;
+  uint32_t *table = nullptr;  // reductions
+  reduce_parts<W> parts = {};
+  uint32_t *heads = nullptr;  // scans
   uint64_t head_words = 0;
   void *region = nullptr;
   region_state *rs = nullptr;
   size_t region_used = 0;
   size_t region_cap = 0;
+  uint32_t *trip_flag = nullptr;
+
+  // Checks the configuration and obtains the scratch.  `stream`: where a new
+  // sync region is cleared; NULL defers that to the first enqueue.
+  acpp_status prepare(acpp_allocation_group *g, const hipStream_t *stream, const T *in, T *out,
+                      const uint64_t *offsets, uint64_t num_segments, uint64_t total, W init, bool is_reduce,
+                      const acpp_launch_config *cfg) {
+    static_assert(sizeof(T) >= 4, "16-byte vector accesses at 4-byte alignment (u32x4_a4)");
+    int cus = 0;
+    acpp_status st = enter_device(g, &cus);
+    if (st != ACPP_SUCCESS) return st;
+    device = group_device(g);
+    reduce = is_reduce;
+    default_tile(reduce, total, static_cast<int>(sizeof(T)), wg, rows);
+    if (cfg && cfg->work_group_size) wg = cfg->work_group_size;
+    if (!valid_work_group_size(wg))
+      return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
+    if (cfg && cfg->items_per_thread) rows = static_cast<int>(cfg->items_per_thread);
+    if (rows != 2 && rows != 4 && rows != 8)
+      return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": items_per_thread must be 2, 4 or 8");
+    tile_elems = static_cast<uint64_t>(wg) * rows * VEC;
+    const uint64_t num_tiles = std::max<uint64_t>(1, ceil_div(total, tile_elems));
+    if (num_tiles >= (1ull << 31) || num_segments >= (1ull << 32))
+      return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": problem too large");
+    p.in = in;
+    p.out = out;
+    p.offsets = offsets;
+    p.tile_seg = nullptr;
+    p.heads = nullptr;
+    p.head_words_total = 0;
+    p.block_lookback = 0;
+    p.force_give_up = 0;
+    p.num_segments = num_segments;
+    p.total = total;
+    p.init = init;
+    p.num_tiles = static_cast<uint32_t>(num_tiles);
+    p.epoch = 0;
+    p.ticket_base = 0;
+    p.sync = nullptr;
+    p.status = nullptr;
+    return reduce ? prepare_reduce(g) : prepare_scan(g, stream, cus, cfg);
+  }
+
+  acpp_status prepare_reduce(acpp_allocation_group *g) {
+    const uint64_t num_tiles = p.num_tiles;
+    void *scratch = nullptr;
+    acpp_status st = group_obtain(g, num_tiles * (2 * sizeof(W) + sizeof(uint32_t)), &scratch);
+    if (st != ACPP_SUCCESS) return st;
+    parts.head = static_cast<W *>(scratch);
+    parts.tail = parts.head + num_tiles;
+    parts.tail_seg = reinterpret_cast<uint32_t *>(parts.tail + num_tiles);
+    if (num_tiles > max_search_tiles) {
+      void *ts = nullptr;
+      st = group_obtain(g, (num_tiles + 1) * sizeof(uint32_t), &ts);
+      if (st != ACPP_SUCCESS) return st;
+      table = static_cast<uint32_t *>(ts);
+    }
+    p.tile_seg = table;
+    p.vec_io = (reinterpret_cast<uintptr_t>(p.in) & 3) == 0;
+    grid = p.num_tiles;
+    lds = reduce_head_words(static_cast<uint32_t>(tile_elems)) * 4 + tile_elems * sizeof(W);
+    return ACPP_SUCCESS;
+  }
+
+  acpp_status prepare_scan(acpp_allocation_group *g, const hipStream_t *stream, int cus,
+                           const acpp_launch_config *cfg) {
+    const uint64_t num_tiles = p.num_tiles;
+    acpp_status st;
+    // the scan kernel stores 2 x wg words of head bits (>= the tile_elems + 1
+    // bits it needs, since rows x 16-byte vector <= 32 elements)
+    lds = std::max<size_t>(static_cast<size_t>((tile_elems + 1 + 31) / 32), 2 * static_cast<size_t>(wg)) * 4;
+    // Small inputs (2-row tiles) mark their segment starts in the scan kernel.
+    mark = rows == 2 && num_tiles <= max_search_tiles;
+    if (!mark) {
+      // Head bitmap over elements [0, total] plus one spare word.
+      head_words = (p.total + 1 + 31) / 32 + 1;
+      void *hb = nullptr;
+      st = group_obtain(g, head_words * sizeof(uint32_t), &hb);
+      if (st != ACPP_SUCCESS) return st;
+      heads = static_cast<uint32_t *>(hb);
+    }
+    p.heads = heads;
+    p.head_words_total = head_words;
+    using SIO = seg_status<W>;
+    static_assert(SIO::words <= seg_stride_words, "status slot too small");
+    region_used = sizeof(sync_header) + num_tiles * seg_stride_words * sizeof(uint64_t);
+    st = stream ? group_obtain_sync(g, region_used, *stream, &region, &region_cap, &rs)
+                : group_obtain_sync_uncleared(g, region_used, &region, &region_cap, &rs);
+    if (st != ACPP_SUCCESS) return st;
+    trip_flag = host_trip_flag(device);
+    p.block_lookback = (cfg && (cfg->flags & ACPP_VARIANT_BLOCK_LOOKBACK)) ? 1 : 0;
+    p.force_give_up = (cfg && (cfg->flags & ACPP_VARIANT_FORCE_GIVE_UP)) ? 1 : 0;
+    p.vec_io = ((reinterpret_cast<uintptr_t>(p.in) | reinterpret_cast<uintptr_t>(p.out)) & 3) == 0;
+    p.sync = static_cast<sync_header *>(region);
+    p.status = reinterpret_cast<uint64_t *>(static_cast<char *>(region) + sizeof(sync_header));
+
+    // Persistent grid: one wave of resident work-groups, each drawing tiles
+    // from the queue until it is empty.  With ACPP_VARIANT_TILE_PER_GROUP the
+    // grid has one work-group per tile (the hardware dispatcher then keeps
+    // the CUs full while groups wait in their look-back), still fed by the
+    // same queue.  Every work-group draws one ticket past the last tile
+    // before it exits; the ticket base counts those too.
+    grid = static_cast<uint32_t>(num_tiles);
+    if (cfg && (cfg->flags & ACPP_VARIANT_TILE_PER_GROUP)) return ACPP_SUCCESS;
+    const uint32_t per_cu = cfg ? cfg->groups_per_cu : 0;
+    return with_scan_kernel([&](auto kernel) -> acpp_status {
+      int resident = 1;
+      ACPP_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kernel, static_cast<int>(wg), lds));
+      if (resident < 1) resident = 1;
+      uint64_t cap = static_cast<uint64_t>(resident) * cus;
+      if (per_cu) cap = std::min<uint64_t>(cap, static_cast<uint64_t>(per_cu) * cus);
+      grid = static_cast<uint32_t>(std::min<uint64_t>(cap, num_tiles));
+      return ACPP_SUCCESS;
+    });
+  }
+
+  template <class F>
+  acpp_status with_scan_kernel(F &&f) {
+    if (mark) return f(segmented_kernel<T, Op, 2, true>);
+    if (rows == 2) return f(segmented_kernel<T, Op, 2, false>);
+    if (rows == 4) return f(segmented_kernel<T, Op, 4, false>);
+    return f(segmented_kernel<T, Op, 8, false>);
+  }
+
+  acpp_status enqueue(hipStream_t stream) override { return reduce ? enqueue_reduce(stream) : enqueue_scan(stream); }
+
+  // The table of the tiles' first segments (many tiles only), one work-group
+  // per tile, then the fix-up of segments that span tiles.
+  acpp_status enqueue_reduce(hipStream_t stream) {
+    acpp_status st;
+    const uint64_t num_tiles = p.num_tiles, num_segments = p.num_segments;
+    if (table) {
+      if (num_segments <= max_scatter_segments * num_tiles && num_tiles <= max_scatter_tiles * num_segments)
+        hipLaunchKernelGGL(tile_scatter_kernel, dim3(static_cast<uint32_t>(ceil_div(num_segments, 256))), dim3(256), 0,
+                           stream, p.offsets, num_segments, tile_elems, p.num_tiles, table);
+      else
+        hipLaunchKernelGGL(tile_table_kernel, dim3(static_cast<uint32_t>(ceil_div(num_tiles + 1, 256))), dim3(256), 0,
+                           stream, p.offsets, num_segments, tile_elems, p.num_tiles, table);
+      st = check_launch(name);
+      if (st != ACPP_SUCCESS) return st;
+    }
+    if (rows == 2)
+      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 2>), dim3(grid), dim3(wg), lds, stream, p, parts);
+    else if (rows == 4)
+      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 4>), dim3(grid), dim3(wg), lds, stream, p, parts);
+    else
+      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 8>), dim3(grid), dim3(wg), lds, stream, p, parts);
+    st = check_launch(name);
+    if (st != ACPP_SUCCESS || num_tiles == 1) return st;
+    hipLaunchKernelGGL((segmented_fixup_kernel<T, Op>), dim3(static_cast<uint32_t>(ceil_div(num_tiles, 1024))),
+                       dim3(1024), 0, stream, p, parts, tile_elems);
+    return check_launch(name);
+  }
+
+  template <uint32_t WORDS>
+  acpp_status mark_heads(hipStream_t stream) {
+    hipLaunchKernelGGL(head_bitmap_kernel<WORDS>, dim3(static_cast<uint32_t>(ceil_div(head_words, WORDS))), dim3(256),
+                       0, stream, p.offsets, p.num_segments, p.total, head_words, heads);
+    return check_launch(name);
+  }
+
+  acpp_status enqueue_scan(hipStream_t stream) {
+    region_launch rl;
+    acpp_status st = begin_region_launch_flag(trip_flag, region, region_used, region_cap, rs, stream, &rl);
+    if (st != ACPP_SUCCESS) return st;
+    p.epoch = rl.epoch;
+    p.ticket_base = rl.ticket_base;
+    // Chunks small enough to occupy the chip, large enough that the searches
+    // do not count (2^28 fp32 in 89,479 segments: 411 us with 1024 words, 404
+    // us with 4096; 2^23 in 1.7 million: 31 and 56 us).
+    if (!mark)
+      st = p.total >= (1ull << 27) ? mark_heads<4096>(stream)
+           : p.total >= (1ull << 23) ? mark_heads<1024>(stream)
+                                     : mark_heads<256>(stream);
+    if (st == ACPP_SUCCESS)
+      st = with_scan_kernel([&](auto kernel) -> acpp_status {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), lds, stream, p);
+        return check_launch(name);
+      });
+    // every work-group draws one ticket past the last tile before it exits
+    end_region_launch(rs, rl, p.num_tiles + grid, st);
+    return st;
+  }
 };
 
-// Tiles up to which a work-group finds its segments by itself: the launch of
-// the kernel that does it for all tiles costs more (about 3.5 us) than the
-// searches, which a few hundred resident groups overlap.
-constexpr uint64_t max_search_tiles = 1024;
-// Segments per tile up to which the segments write the tiles' table.
-constexpr uint64_t max_scatter_ratio = 16;
-
-template <class T, class Op, int R, bool MARK>
-acpp_status launch_rows(launch_plan<T, Op> &lp, hipStream_t stream, const char *name) {
-  if constexpr (!MARK) {
-    hipLaunchKernelGGL(head_bitmap_kernel, dim3(static_cast<uint32_t>(ceil_div(lp.head_words, head_chunk_words))),
-                       dim3(256), 0, stream, lp.p.offsets, lp.p.num_segments, lp.p.total, lp.head_words, lp.heads);
-    acpp_status st = check_launch(name);
-    if (st != ACPP_SUCCESS) return st;
-  }
-  hipLaunchKernelGGL((segmented_kernel<T, Op, R, MARK>), dim3(lp.grid), dim3(lp.wg), lp.lds, stream, lp.p);
-  return check_launch(name);
-}
-
-// Segmented reduction: the table of the tiles' first segments (many tiles
-// only), one work-group per tile, then the fix-up of segments that span
-// tiles.
-template <class T, class Op>
-acpp_status enqueue_reduce(acpp_allocation_group *g, launch_plan<T, Op> &lp, hipStream_t stream, const T *in,
-                           T *out, const uint64_t *offsets, uint64_t num_segments, uint64_t total,
-                           typename elem_traits<T>::work init, uint64_t num_tiles, const char *name) {
-  using W = typename elem_traits<T>::work;
-  void *scratch = nullptr;
-  acpp_status st = group_obtain(g, num_tiles * (2 * sizeof(W) + sizeof(uint32_t)), &scratch);
-  if (st != ACPP_SUCCESS) return st;
-  reduce_parts<W> parts;
-  parts.head = static_cast<W *>(scratch);
-  parts.tail = parts.head + num_tiles;
-  parts.tail_seg = reinterpret_cast<uint32_t *>(parts.tail + num_tiles);
-  uint32_t *table = nullptr;
-  if (num_tiles > max_search_tiles) {
-    void *ts = nullptr;
-    st = group_obtain(g, (num_tiles + 1) * sizeof(uint32_t), &ts);
-    if (st != ACPP_SUCCESS) return st;
-    table = static_cast<uint32_t *>(ts);
-  }
-  params<T> &p = lp.p;
-  p.in = in;
-  p.out = out;
-  p.offsets = offsets;
-  p.tile_seg = table;
-  p.heads = nullptr;  // the reduce kernel marks its heads from the offsets
-  p.head_words_total = 0;
-  p.block_lookback = 0;
-  p.force_give_up = 0;
-  p.num_segments = num_segments;
-  p.total = total;
-  p.init = init;
-  p.vec_io = (reinterpret_cast<uintptr_t>(in) & 3) == 0;
-  p.num_tiles = static_cast<uint32_t>(num_tiles);
-  p.epoch = 0;
-  p.ticket_base = 0;
-  p.sync = nullptr;
-  p.status = nullptr;
-  lp.grid = static_cast<uint32_t>(num_tiles);
-
-  if (table) {
-    if (num_segments <= max_scatter_ratio * num_tiles && num_tiles <= 8 * num_segments)
-      hipLaunchKernelGGL(tile_scatter_kernel, dim3(static_cast<uint32_t>(ceil_div(num_segments, 256))), dim3(256), 0,
-                         stream, offsets, num_segments, lp.tile_elems, p.num_tiles, table);
-    else
-      hipLaunchKernelGGL(tile_table_kernel, dim3(static_cast<uint32_t>(ceil_div(num_tiles + 1, 256))), dim3(256), 0,
-                         stream, offsets, num_segments, lp.tile_elems, p.num_tiles, table);
-    st = check_launch(name);
-    if (st != ACPP_SUCCESS) return st;
-  }
-  const size_t lds = reduce_head_words(static_cast<uint32_t>(lp.tile_elems)) * 4 + lp.tile_elems * sizeof(W);
-  if (lp.rows == 2)
-    hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 2>), dim3(lp.grid), dim3(lp.wg), lds, stream, p, parts);
-  else if (lp.rows == 4)
-    hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 4>), dim3(lp.grid), dim3(lp.wg), lds, stream, p, parts);
-  else
-    hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 8>), dim3(lp.grid), dim3(lp.wg), lds, stream, p, parts);
-  st = check_launch(name);
-  if (st != ACPP_SUCCESS || num_tiles == 1) return st;
-  hipLaunchKernelGGL((segmented_fixup_kernel<T, Op>), dim3(static_cast<uint32_t>(ceil_div(num_tiles, 1024))),
-                     dim3(1024), 0, stream, p, parts, lp.tile_elems);
-  return check_launch(name);
-}
-
-template <class T, class Op>
-acpp_status enqueue(acpp_allocation_group *g, hipStream_t stream, const T *in, T *out,
-                    const uint64_t *offsets, uint64_t num_segments, uint64_t total,
-                    typename elem_traits<T>::work init, bool reduce,
-                    const acpp_launch_config *cfg, const char *name) {
-  static_assert(sizeof(T) >= 4, "16-byte vector accesses at 4-byte alignment (u32x4_a4)");
-  constexpr int VEC = 16 / sizeof(T);
-  int cus = 0;
-  acpp_status st = enter_device(g, &cus);
-  if (st != ACPP_SUCCESS) return st;
-  launch_plan<T, Op> lp;
-  default_tile(reduce, total, static_cast<int>(sizeof(T)), lp.wg, lp.rows);
-  if (cfg && cfg->work_group_size) lp.wg = cfg->work_group_size;
-  if (!valid_work_group_size(lp.wg))
-    return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
-  if (cfg && cfg->items_per_thread) lp.rows = static_cast<int>(cfg->items_per_thread);
-  if (lp.rows != 2 && lp.rows != 4 && lp.rows != 8)
-    return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": items_per_thread must be 2, 4 or 8");
-  lp.tile_elems = static_cast<uint64_t>(lp.wg) * lp.rows * VEC;
-  const uint64_t num_tiles = std::max<uint64_t>(1, ceil_div(total, lp.tile_elems));
-  if (num_tiles >= (1ull << 31) || num_segments >= (1ull << 32))
-    return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": problem too large");
-  // the scan kernel stores 2 x wg words of head bits (>= the tile_elems + 1
-  // bits it needs, since rows x 16-byte vector <= 32 elements)
-  lp.lds = std::max<size_t>(static_cast<size_t>((lp.tile_elems + 1 + 31) / 32), 2 * static_cast<size_t>(lp.wg)) * 4;
-
-  if (reduce) return enqueue_reduce<T, Op>(g, lp, stream, in, out, offsets, num_segments, total, init, num_tiles, name);
-  // Small inputs (2-row tiles) mark their segment starts in the scan kernel.
-  const bool mark = lp.rows == 2 && num_tiles <= max_search_tiles;
-  if (!mark) {
-    // Head bitmap over elements [0, total] plus one spare word.
-    lp.head_words = (total + 1 + 31) / 32 + 1;
-    void *hb = nullptr;
-    st = group_obtain(g, lp.head_words * sizeof(uint32_t), &hb);
-    if (st != ACPP_SUCCESS) return st;
-    lp.heads = static_cast<uint32_t *>(hb);
-  }
-  using SIO = seg_status<typename elem_traits<T>::work>;
-  static_assert(SIO::words <= seg_stride_words, "status slot too small");
-  lp.region_used = sizeof(sync_header) + num_tiles * seg_stride_words * sizeof(uint64_t);
-  st = group_obtain_sync(g, lp.region_used, stream, &lp.region, &lp.region_cap, &lp.rs);
-  if (st != ACPP_SUCCESS) return st;
-
-  region_launch rl;
-  st = begin_region_launch(g, lp.region, lp.region_used, lp.region_cap, lp.rs, stream, &rl);
-  if (st != ACPP_SUCCESS) return st;
-
-  params<T> &p = lp.p;
-  p.in = in;
-  p.out = out;
-  p.offsets = offsets;
-  p.tile_seg = nullptr;
-  p.heads = lp.heads;
-  p.head_words_total = lp.head_words;
-  p.block_lookback = (cfg && (cfg->flags & ACPP_VARIANT_BLOCK_LOOKBACK)) ? 1 : 0;
-  p.force_give_up = (cfg && (cfg->flags & ACPP_VARIANT_FORCE_GIVE_UP)) ? 1 : 0;
-  p.num_segments = num_segments;
-  p.total = total;
-  p.init = init;
-  p.vec_io = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 3) == 0;
-  p.num_tiles = static_cast<uint32_t>(num_tiles);
-  p.epoch = rl.epoch;
-  p.ticket_base = rl.ticket_base;
-  p.sync = static_cast<sync_header *>(lp.region);
-  p.status = reinterpret_cast<uint64_t *>(static_cast<char *>(lp.region) + sizeof(sync_header));
-
-  // Persistent grid: one wave of resident work-groups, each drawing tiles
-  // from the queue until it is empty.  With ACPP_VARIANT_TILE_PER_GROUP the
-  // grid has one work-group per tile (the hardware dispatcher then keeps
-  // the CUs full while groups wait in their look-back), still fed by the
-  // same queue.  Every work-group draws one ticket past the last tile
-  // before it exits; the ticket base counts those too.
-  const bool per_tile = cfg && (cfg->flags & ACPP_VARIANT_TILE_PER_GROUP);
-  auto pick = [&](auto kernel) -> acpp_status {
-    if (per_tile) {
-      lp.grid = static_cast<uint32_t>(num_tiles);
-      return ACPP_SUCCESS;
-    }
-    int resident = 1;
-    ACPP_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kernel, static_cast<int>(lp.wg), lp.lds));
-    if (resident < 1) resident = 1;
-    uint64_t cap = static_cast<uint64_t>(resident) * cus;
-    if (cfg && cfg->groups_per_cu) cap = std::min<uint64_t>(cap, static_cast<uint64_t>(cfg->groups_per_cu) * cus);
-    lp.grid = static_cast<uint32_t>(std::min<uint64_t>(cap, num_tiles));
-    return ACPP_SUCCESS;
-  };
-  auto run = [&](auto rows_tag, auto mark_tag) -> acpp_status {
-    constexpr int R = decltype(rows_tag)::value;
-    constexpr bool MARK = decltype(mark_tag)::value;
-    acpp_status e = pick(segmented_kernel<T, Op, R, MARK>);
-    return e == ACPP_SUCCESS ? launch_rows<T, Op, R, MARK>(lp, stream, name) : e;
-  };
-  using std::integral_constant;
-  acpp_status s;
-  if (mark)
-    s = run(integral_constant<int, 2>{}, std::true_type{});
-  else if (lp.rows == 2)
-    s = run(integral_constant<int, 2>{}, std::false_type{});
-  else if (lp.rows == 4)
-    s = run(integral_constant<int, 4>{}, std::false_type{});
-  else
-    s = run(integral_constant<int, 8>{}, std::false_type{});
-  // every work-group draws one ticket past the last tile before it exits
-  end_region_launch(lp.rs, rl, static_cast<uint32_t>(num_tiles) + lp.grid, s);
-  return s;
-}
-
-template <class T>
-acpp_status entry(acpp_allocation_group *g, hipStream_t stream, const T *in, T *out,
-                  const uint64_t *offsets, uint64_t num_segments, uint64_t total, T init, int op,
-                  bool reduce, const acpp_launch_config *cfg, const char *name) {
+// Validates a call and hands the prepared one to `run` (NULL when there is
+// nothing to do).  `stream`: see call::prepare.
+template <class T, class F>
+acpp_status with_prepared(acpp_allocation_group *g, const hipStream_t *stream, const T *in, T *out,
+                          const uint64_t *offsets, uint64_t num_segments, uint64_t total, T init, int op, bool reduce,
+                          const acpp_launch_config *cfg, const char *name, F &&run) {
   using W = typename elem_traits<T>::work;
   if (!g) return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": scratch group is NULL");
   if (num_segments > 0 && !offsets)
@@ -1381,17 +1399,31 @@ acpp_status entry(acpp_allocation_group *g, hipStream_t stream, const T *in, T *
     return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": in or out is NULL");
   if (op < ops::op_plus || op > ops::op_max)
     return set_error(ACPP_ERROR_UNSUPPORTED, std::string(name) + ": segmented forms support plus, multiply, min and max");
-  if (num_segments == 0) return clear_error();
+  if (num_segments == 0) {
+    acpp_status s = run(static_cast<call<T, ops::plus<W, T>> *>(nullptr));
+    return s == ACPP_SUCCESS ? clear_error() : s;
+  }
   return with_op<W, T>(op, [&](auto opv) -> acpp_status {
     using Op = decltype(opv);
     if constexpr (Op::id > ops::op_max) {
       return set_error(ACPP_ERROR_UNSUPPORTED, "unsupported operator");
     } else {
-      acpp_status s = enqueue<T, Op>(g, stream, in, out, offsets, num_segments, total,
-                                     elem_traits<T>::to_work(init), reduce, cfg, name);
+      call<T, Op> c;
+      c.name = name;
+      acpp_status s = c.prepare(g, stream, in, out, offsets, num_segments, total, elem_traits<T>::to_work(init),
+                                reduce, cfg);
+      if (s == ACPP_SUCCESS) s = run(&c);
       return s == ACPP_SUCCESS ? clear_error() : s;
     }
   });
+}
+
+template <class T>
+acpp_status entry(acpp_allocation_group *g, hipStream_t stream, const T *in, T *out, const uint64_t *offsets,
+                  uint64_t num_segments, uint64_t total, T init, int op, bool reduce, const acpp_launch_config *cfg,
+                  const char *name) {
+  return with_prepared<T>(g, &stream, in, out, offsets, num_segments, total, init, op, reduce, cfg, name,
+                          [&](auto *c) { return c ? c->enqueue(stream) : ACPP_SUCCESS; });
 }
 
 }  // namespace seg_detail
@@ -1401,50 +1433,40 @@ using namespace acpp_impl;
 using namespace acpp_impl::seg_detail;
 
 // --------------------------------------------------------------------------
-// Graph plans
+// Plans: a call whose scratch is kept.  Every launch enqueues its kernels
+// directly: replaying them as a graph of as many nodes took 6 to 9 us longer
+// on MI355X (2^19 fp32 scan 16.0 us as a graph, 6.8 us direct), and
+// a graph has to clear the scan's sync region in every replay.
 // --------------------------------------------------------------------------
 struct acpp_segmented_plan {
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  std::unique_ptr<prepared> call;  // empty: nothing to do
+  std::mutex mutex;                // the epochs of the sync region, in launch order
   int device = 0;
 };
 
 namespace {
-template <class F>
-acpp_status capture_plan(acpp_allocation_group *g, F &&enqueue_fn, acpp_segmented_plan **out) {
-  if (!out) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "plan output pointer is NULL");
+template <class T>
+acpp_status make_plan(acpp_allocation_group *g, const T *in, T *out, const uint64_t *offsets, uint64_t num_segments,
+                      uint64_t total, T init, int op, bool reduce, const acpp_launch_config *cfg, const char *name,
+                      acpp_segmented_plan **plan) {
+  if (!g) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "scratch group is NULL");
+  if (!plan) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "plan output pointer is NULL");
   int cus = 0;
   acpp_status st = enter_device(g, &cus);
   if (st != ACPP_SUCCESS) return st;
-  hipStream_t cs = nullptr;
-  ACPP_CHECK_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
-  std::unique_ptr<acpp_segmented_plan> plan(new acpp_segmented_plan);
-  plan->device = group_device(g);
-  // Relaxed mode: the first capture of a plan may have to allocate its
-  // scratch (hipMalloc through the allocation cache); the allocation is made
-  // at once and is not part of the graph.
-  hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeRelaxed);
-  if (e != hipSuccess) {
-    (void)hipStreamDestroy(cs);
-    return hip_error(e, "hipStreamBeginCapture");
-  }
-  acpp_status s = enqueue_fn(cs);
-  hipGraph_t graph = nullptr;
-  e = hipStreamEndCapture(cs, &graph);
-  (void)hipStreamDestroy(cs);
-  if (s != ACPP_SUCCESS) {
-    if (graph) (void)hipGraphDestroy(graph);
-    return s;
-  }
-  if (e != hipSuccess) return hip_error(e, "hipStreamEndCapture");
-  plan->graph = graph;
-  e = hipGraphInstantiate(&plan->exec, graph, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    (void)hipGraphDestroy(graph);
-    return hip_error(e, "hipGraphInstantiate");
-  }
-  *out = plan.release();
-  return clear_error();
+  std::unique_ptr<acpp_segmented_plan> made(new (std::nothrow) acpp_segmented_plan);
+  if (!made) return set_error(ACPP_ERROR_OUT_OF_MEMORY, "host allocation failed");
+  made->device = group_device(g);
+  st = with_prepared<T>(g, nullptr, in, out, offsets, num_segments, total, init, op, reduce, cfg, name,
+                        [&](auto *c) -> acpp_status {
+                          if (!c) return ACPP_SUCCESS;
+                          using C = std::remove_pointer_t<decltype(c)>;
+                          made->call.reset(new (std::nothrow) C(*c));
+                          if (!made->call) return set_error(ACPP_ERROR_OUT_OF_MEMORY, "host allocation failed");
+                          return ACPP_SUCCESS;
+                        });
+  if (st == ACPP_SUCCESS) *plan = made.release();
+  return st;
 }
 }  // namespace
 
@@ -1470,27 +1492,15 @@ extern "C" {
       acpp_allocation_group *scratch, const T *first, uint64_t n, T *d_first,                         \
       const uint64_t *offsets, uint64_t num_segments, acpp_algorithm_op op,                           \
       const acpp_launch_config *config, acpp_segmented_plan **plan) {                                 \
-    if (!scratch) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "scratch group is NULL");             \
-    return capture_plan(                                                                              \
-        scratch,                                                                                      \
-        [&](hipStream_t cs) {                                                                         \
-          return entry<T>(scratch, cs, first, d_first, offsets, num_segments, n, T{}, op, false,      \
-                          config, "acpp_segmented_plan_inclusive_scan_" #tag);                       \
-        },                                                                                            \
-        plan);                                                                                        \
+    return make_plan<T>(scratch, first, d_first, offsets, num_segments, n, T{}, op, false, config,    \
+                        "acpp_segmented_plan_inclusive_scan_" #tag, plan);                            \
   }                                                                                                   \
   acpp_status acpp_segmented_plan_reduce_##tag(                                                        \
       acpp_allocation_group *scratch, const T *first, uint64_t n, const uint64_t *offsets,            \
       uint64_t num_segments, T *out, T init, acpp_algorithm_op op, const acpp_launch_config *config, \
       acpp_segmented_plan **plan) {                                                                   \
-    if (!scratch) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "scratch group is NULL");             \
-    return capture_plan(                                                                              \
-        scratch,                                                                                      \
-        [&](hipStream_t cs) {                                                                         \
-          return entry<T>(scratch, cs, first, out, offsets, num_segments, n, init, op, true, config,   \
-                          "acpp_segmented_plan_reduce_" #tag);                                        \
-        },                                                                                            \
-        plan);                                                                                        \
+    return make_plan<T>(scratch, first, out, offsets, num_segments, n, init, op, true, config,        \
+                        "acpp_segmented_plan_reduce_" #tag, plan);                                    \
   }
 
 ACPP_DEFINE_SEGMENTED(i32, int32_t)
@@ -1499,18 +1509,18 @@ ACPP_DEFINE_SEGMENTED(f32, float)
 ACPP_DEFINE_SEGMENTED(f64, double)
 
 acpp_status acpp_segmented_plan_launch(acpp_segmented_plan *plan, acpp_stream_t stream) {
-  if (!plan || !plan->exec) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "plan is NULL");
+  if (!plan) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "plan is NULL");
   int cur = 0;
   ACPP_CHECK_HIP(hipGetDevice(&cur));
   if (cur != plan->device) ACPP_CHECK_HIP(hipSetDevice(plan->device));
-  ACPP_CHECK_HIP(hipGraphLaunch(plan->exec, static_cast<hipStream_t>(stream)));
-  return clear_error();
+  if (!plan->call) return clear_error();
+  std::lock_guard<std::mutex> lock{plan->mutex};
+  acpp_status s = plan->call->enqueue(static_cast<hipStream_t>(stream));
+  return s == ACPP_SUCCESS ? clear_error() : s;
 }
 
 acpp_status acpp_segmented_plan_destroy(acpp_segmented_plan *plan) {
   if (!plan) return set_error(ACPP_ERROR_INVALID_ARGUMENT, "plan is NULL");
-  if (plan->exec) (void)hipGraphExecDestroy(plan->exec);
-  if (plan->graph) (void)hipGraphDestroy(plan->graph);
   delete plan;
   return clear_error();
 }

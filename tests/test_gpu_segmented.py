@@ -301,3 +301,51 @@ def test_segmented_edges(gpu, q, scratch, dtype, cfg):
             assert np.array_equal(host(out).astype(np.int64), exp), (name, op)
             if n:
                 assert np.array_equal(host(yd).astype(np.int64), O.segmented_inclusive_scan(xi, off, op)), (name, op)
+
+
+@pytest.mark.parametrize("n", [5000, 1 << 21, (1 << 23) + 5])
+def test_plan_launched_eagerly_and_in_a_graph(gpu, n):
+    # a plan's launches continue its region's epochs, also on another stream
+    # and after replays of a graph that holds one
+    torch, _ = gpu
+    off = np.concatenate([[0], np.sort(np.random.default_rng(n).integers(0, n, 300)), [n]]).astype(np.uint64)
+    x = exact_ints(torch, n, 3)
+    od = dev(torch, off)
+    cache = acpp.AllocationCache()
+    scratch = acpp.AllocationGroup(cache)
+    yd = torch.zeros_like(x)
+    out = torch.zeros(len(off) - 1, dtype=x.dtype, device="cuda")
+    scan = acpp.SegmentedPlan.inclusive_scan(scratch, x, yd, od)
+    red = acpp.SegmentedPlan.reduce(scratch, x, od, out)
+
+    def check(what):
+        torch.cuda.synchronize()
+        xh = host(x)
+        assert np.array_equal(host(yd), O.segmented_inclusive_scan(xh, off)), what
+        assert np.array_equal(host(out), O.segmented_reduce(xh, off, np.int32(0))), what
+        yd.zero_()
+        out.zero_()
+        x.add_(1)
+
+    side = torch.cuda.Stream()
+    for what in ("first", "second"):
+        scan.launch(acpp.Queue())
+        red.launch(acpp.Queue())
+        check(what)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        scan.launch(acpp.Queue())
+        red.launch(acpp.Queue())
+    for what in range(3):
+        graph.replay()
+        check(("replay", what))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            scan.launch(acpp.Queue())
+            red.launch(acpp.Queue())
+        check(("eager after replay", what))
+    del graph
+    scan.close()
+    red.close()
+    scratch.close()
+    cache.close()
