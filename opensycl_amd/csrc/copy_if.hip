@@ -42,8 +42,6 @@ struct params {
   uint64_t n;
   T operand;
   T mask;
-  int vec_io;
-  int stencil_vec;  // stencil aligned to VEC bytes: one load per 16-byte data vector
   uint32_t num_tiles;
   uint32_t epoch;
   uint32_t ticket_base;
@@ -53,7 +51,7 @@ struct params {
 };
 
 template <int PRED, class T>
-__device__ __forceinline__ bool eval(const params<T> &p, T x, uint64_t idx) {
+__device__ __forceinline__ bool eval(const params<T> &p, T x) {
   if constexpr (PRED == ACPP_PRED_NONZERO) return x != T(0);
   else if constexpr (PRED == ACPP_PRED_EQ) return x == p.operand;
   else if constexpr (PRED == ACPP_PRED_NE) return x != p.operand;
@@ -61,44 +59,70 @@ __device__ __forceinline__ bool eval(const params<T> &p, T x, uint64_t idx) {
   else if constexpr (PRED == ACPP_PRED_LE) return x <= p.operand;
   else if constexpr (PRED == ACPP_PRED_GT) return x > p.operand;
   else if constexpr (PRED == ACPP_PRED_GE) return x >= p.operand;
-  else if constexpr (PRED == ACPP_PRED_MASK_EQ) {
+  else {
+    static_assert(PRED == ACPP_PRED_MASK_EQ, "predicate on the element");
     if constexpr (std::is_integral_v<T>) return (x & p.mask) == p.operand;
     else return false;
-  } else {
-    return p.stencil[idx] != 0;  // ACPP_PRED_STENCIL
   }
 }
 
-// Selection bits of the tile: bit k of fm[r] = element k of row r is copied.
-template <int PRED, class T, int R, int VEC>
-__device__ __forceinline__ void select_bits(const params<T> &p, const T (&v)[R][VEC], uint64_t base, bool full,
-                                            uint32_t (&fm)[R]) {
+// The VEC stencil bytes of a data vector, loaded as one word at any address.
+template <int VEC>
+struct stencil_word;
+template <>
+struct stencil_word<2> {
+  typedef uint16_t type;
+};
+template <>
+struct stencil_word<4> {
+  typedef uint32_t type;
+};
+template <>
+struct stencil_word<8> {
+  typedef uint64_t type;
+};
+template <>
+struct stencil_word<16> {
+  typedef u32x4 type;
+};
+
+// Selection bits of the tile's vectors from the stencil: bit k of fm[r] =
+// element k of row r is copied (elements past the end of a partial tile read
+// as 0).
+template <bool FULL, int R, int VEC>
+__device__ __forceinline__ void stencil_bits(const uint8_t *tile, const scan_detail::partial_tile &part,
+                                             uint32_t (&fm)[R]) {
+  using SW = typename stencil_word<VEC>::type;
+  typedef SW SW1 __attribute__((aligned(1)));
   const int B = blockDim.x;
-  if constexpr (PRED == ACPP_PRED_STENCIL && (VEC == 2 || VEC == 4)) {
-    if (full && p.stencil_vec) {
-      // The VEC stencil bytes of a data vector in one load.
-      using SW = std::conditional_t<VEC == 4, uint32_t, uint16_t>;
-      const SW *sw = reinterpret_cast<const SW *>(p.stencil + base);
-      SW bytes[R];
+  const int tid = threadIdx.x;
+  const SW1 *sw = reinterpret_cast<const SW1 *>(tile);
+  uint32_t cut_bits = 0;
+  if constexpr (!FULL) {
+    if (part.count != 0 && static_cast<uint32_t>(tid) == part.tid) {
+      const uint8_t *src = tile + static_cast<uint64_t>(part.row * B + part.tid) * VEC;
 #pragma unroll
-      for (int r = 0; r < R; ++r) bytes[r] = sw[r * B + threadIdx.x];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        fm[r] = 0;
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) fm[r] |= (((bytes[r] >> (8 * k)) & 0xffu) != 0u ? 1u : 0u) << k;
-      }
-      return;
+      for (int k = 0; k < VEC; ++k)
+        if (static_cast<uint32_t>(k) < part.count && src[k] != 0) cut_bits |= 1u << k;
     }
+  }
+  SW bytes[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    bytes[r] = SW{};
+    if (FULL || static_cast<uint32_t>(r * B + tid + 1) * VEC <= part.in_range) bytes[r] = sw[r * B + tid];
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
+    uint32_t words[4] = {};
+    __builtin_memcpy(words, &bytes[r], sizeof(SW));
+    // the words, not the bytes extracted from them, are kept until here
+#pragma unroll
+    for (int i = 0; i < (VEC + 3) / 4; ++i) asm volatile("" : "+v"(words[i]));
     fm[r] = 0;
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      const uint64_t idx = base + static_cast<uint64_t>(r * B + threadIdx.x) * VEC + k;
-      if ((full || idx < p.n) && eval<PRED>(p, v[r][k], idx)) fm[r] |= 1u << k;
-    }
+    for (int k = 0; k < VEC; ++k) fm[r] |= (((words[k >> 2] >> (8 * (k & 3))) & 0xffu) != 0u ? 1u : 0u) << k;
+    if (!FULL && part.cut(r, tid)) fm[r] = cut_bits;
   }
 }
 
@@ -110,39 +134,27 @@ __device__ __forceinline__ T elem(const u32x4 &q, int k) {
   return tmp[k];
 }
 
-// select_bits for 1- and 2-byte elements kept packed in their vectors (q);
-// in_range: the tile's elements before the end of the input.
-template <int PRED, class T, int R>
-__device__ __forceinline__ void select_bits_packed(const params<T> &p, const u32x4 (&q)[R], uint64_t base,
-                                                   uint32_t in_range, bool full, uint32_t (&fm)[R]) {
+// Selection bits of a vector from the predicate.
+template <int PRED, class T>
+__device__ __forceinline__ uint32_t select_bits(const params<T> &p, const u32x4 &q) {
   constexpr int VEC = 16 / sizeof(T);
-  const int B = blockDim.x;
-  if constexpr (PRED == ACPP_PRED_STENCIL) {
-    if (full && p.stencil_vec) {
-      // The VEC stencil bytes of a data vector in one load.
-      using SW = std::conditional_t<VEC == 16, u32x4, uint64_t>;
-      const SW *sw = reinterpret_cast<const SW *>(p.stencil + base);
-      SW bytes[R];
+  uint32_t fm = 0;
 #pragma unroll
-      for (int r = 0; r < R; ++r) bytes[r] = sw[r * B + threadIdx.x];
+  for (int k = 0; k < VEC; ++k)
+    if (eval<PRED>(p, elem<T>(q, k))) fm |= 1u << k;
+  return fm;
+}
+
+// Vectors of 1- and 2-byte elements through an empty asm statement: elements
+// extracted before it are not kept for uses after it.
+template <class T, int R>
+__device__ __forceinline__ void repack(u32x4 (&q)[R]) {
+  if constexpr (sizeof(T) < 4) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        uint32_t words[4] = {};
-        __builtin_memcpy(words, &bytes[r], sizeof(SW));
-        fm[r] = 0;
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) fm[r] |= (((words[k >> 2] >> (8 * (k & 3))) & 0xffu) != 0u ? 1u : 0u) << k;
-      }
-      return;
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    fm[r] = 0;
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      const uint32_t i = static_cast<uint32_t>(r * B + threadIdx.x) * VEC + k;
-      if ((full || i < in_range) && eval<PRED>(p, elem<T>(q[r], k), base + i)) fm[r] |= 1u << k;
+    for (int r = 0; r < R; ++r) {
+      uint32_t a = q[r].x, b = q[r].y, c = q[r].z, d = q[r].w;
+      asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+      q[r] = u32x4{a, b, c, d};
     }
   }
 }
@@ -174,68 +186,45 @@ __device__ __forceinline__ void copy_if_tile(const params<T> &p, uint32_t tile, 
   const uint64_t tile_elems = static_cast<uint64_t>(B) * R * VEC;
   const uint64_t base = static_cast<uint64_t>(tile) * tile_elems;
 
-  // 1- and 2-byte elements stay packed in their 16-byte vectors (four
-  // registers a row) and are extracted where they are used: 8 rows of 8 or
-  // 16 unpacked elements spill.
-  constexpr bool NARROW = sizeof(T) < 4;
+  const uint32_t in_range =
+      FULL ? static_cast<uint32_t>(tile_elems) : static_cast<uint32_t>(p.n > base ? min(p.n - base, tile_elems) : 0);
+  const scan_detail::partial_tile part = scan_detail::partial_tile::of<T>(in_range, B);
+
+  // The elements stay packed in their 16-byte vectors (four registers a row)
+  // and are extracted where they are used: 8 rows of 8 or 16 unpacked
+  // elements spill.
   u32x4 q[R];
-  T v[NARROW ? 1 : R][VEC];
+  const scan_detail::u32x4_a1 *src = reinterpret_cast<const scan_detail::u32x4_a1 *>(p.in + base);
   if constexpr (FULL) {
-    const scan_detail::u32x4_a4 *src = reinterpret_cast<const scan_detail::u32x4_a4 *>(p.in + base);
 #pragma unroll
     for (int r = 0; r < R; ++r) q[r] = src[r * B + tid];
-    if constexpr (!NARROW) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) __builtin_memcpy(v[r], &q[r], 16);
-    }
-  } else if constexpr (NARROW) {
-    const uint32_t in_range = static_cast<uint32_t>(p.n > base ? min(p.n - base, tile_elems) : 0);
-    const T *in_tile = p.in + base;
-    using U = std::make_unsigned_t<T>;
+  } else {
+    const u32x4 cut = part.load_cut<T>(p.in + base, tid, B);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const uint32_t first = static_cast<uint32_t>(r * B + tid) * VEC;
-      if (p.vec_io && first + VEC <= in_range) {
-        // a whole vector inside the input: one load
-        q[r] = *reinterpret_cast<const scan_detail::u32x4_a4 *>(in_tile + first);
-      } else {
-        // the vector across the end (or an input not 4-byte aligned):
-        // element by element, each ORed into its word
-        uint32_t d[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-          constexpr int sz = static_cast<int>(sizeof(T));
-          if (first + k < in_range)
-            d[(k * sz) >> 2] |= static_cast<uint32_t>(static_cast<U>(in_tile[first + k])) << (8 * ((k * sz) & 3));
-        }
-        q[r] = u32x4{d[0], d[1], d[2], d[3]};
-      }
+      q[r] = part.cut(r, tid) ? cut : u32x4{0, 0, 0, 0};
+      if (static_cast<uint32_t>(r * B + tid + 1) * VEC <= in_range) q[r] = src[r * B + tid];
     }
-  } else {
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        const uint64_t idx = base + static_cast<uint64_t>(r * B + tid) * VEC + k;
-        v[r][k] = (idx < p.n) ? p.in[idx] : T(0);
-      }
+    repack<T>(q);
   }
   uint32_t fm[R];
-  if constexpr (NARROW) {
-    const uint32_t in_range = FULL ? static_cast<uint32_t>(tile_elems)
-                                   : static_cast<uint32_t>(p.n > base ? min(p.n - base, tile_elems) : 0);
-    select_bits_packed<PRED>(p, q, base, in_range, FULL, fm);
-    // The compaction below extracts the elements again from the packed
-    // vectors instead of keeping the predicate's extracted copies alive.
+  if constexpr (PRED == ACPP_PRED_STENCIL) {
+    stencil_bits<FULL, R, VEC>(p.stencil + base, part, fm);
+  } else {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      uint32_t a = q[r].x, b = q[r].y, c = q[r].z, d = q[r].w;
-      asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-      q[r] = u32x4{a, b, c, d};
+      fm[r] = select_bits<PRED>(p, q[r]);
+      if constexpr (!FULL) {
+        // only the elements in range
+        const uint32_t first = static_cast<uint32_t>(r * B + tid) * VEC;
+        const uint32_t cnt = in_range > first ? in_range - first : 0u;
+        if (cnt < VEC) fm[r] &= (1u << cnt) - 1u;
+      }
     }
-  } else {
-    select_bits<PRED>(p, v, base, FULL, fm);
   }
+  // The compaction below extracts the elements again from the packed vectors
+  // instead of keeping the predicate's extracted copies alive.
+  repack<T>(q);
   // Ranks inside each wave row; the (row, wave) counts go to LDS.
   uint32_t wexcl[R];
 #pragma unroll
@@ -272,10 +261,7 @@ __device__ __forceinline__ void copy_if_tile(const params<T> &p, uint32_t tile, 
     const uint32_t bits = fm[r];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
-      if (bits & (1u << k)) {
-        if constexpr (NARROW) s_stage[pos++] = elem<T>(q[r], k);
-        else s_stage[pos++] = v[r][k];
-      }
+      if (bits & (1u << k)) s_stage[pos++] = elem<T>(q[r], k);
     }
   }
   // Wave 0 looks back for the tile's output offset.
@@ -353,7 +339,7 @@ __global__ __launch_bounds__(1024) void copy_if_kernel(params<T> p) {
   if (tile >= p.num_tiles) return;
   const uint64_t tile_elems = static_cast<uint64_t>(blockDim.x) * R * VEC;
   const uint64_t base = static_cast<uint64_t>(tile) * tile_elems;
-  if (p.vec_io && base + tile_elems <= p.n)
+  if (base + tile_elems <= p.n)
     copy_if_tile<PRED, true>(p, tile, sh, s_stage);
   else
     copy_if_tile<PRED, false>(p, tile, sh, s_stage);
@@ -391,7 +377,15 @@ acpp_status entry(acpp_allocation_group *g, hipStream_t stream, const T *in, uin
     }
     return clear_error();
   }
-  const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : 1024;
+  // 1024-wide tiles, narrower for short inputs of 1- and 2-byte elements:
+  // their tiles hold four or two times the elements, and a CU works through a
+  // tile alone (whole calls with 256 / 512 / 1024 work-items, half kept: int8
+  // 2^20 10.8 / 11.5 / 14.5 us, 2^24 20.6 / 17.7 / 18.2 us, 2^26 51.3 / 42.0 /
+  // 42.2 us; int16 2^19 8.4 / 8.8 / 10.2 us, 2^22 12.7 / 11.6 / 11.9 us; int32
+  // 2^21 10.4 / 9.0 / 8.8 us).
+  constexpr uint64_t mid_n = sizeof(T) == 1 ? 3ull << 19 : sizeof(T) == 2 ? 3ull << 18 : 0;
+  constexpr uint64_t wide_n = sizeof(T) == 1 ? 1ull << 26 : sizeof(T) == 2 ? 3ull << 21 : 0;
+  const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : n >= wide_n ? 1024 : n >= mid_n ? 512 : 256;
   if (!valid_work_group_size(wg))
     return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");
   if (cfg && cfg->items_per_thread && static_cast<int>(cfg->items_per_thread) != rows<T>())
@@ -415,12 +409,8 @@ acpp_status entry(acpp_allocation_group *g, hipStream_t stream, const T *in, uin
   p.out = out;
   p.num_copied = num_copied;
   p.n = n;
-  p.stencil_vec = stencil && (reinterpret_cast<uintptr_t>(stencil) % VEC) == 0;
   p.operand = operand;
   p.mask = mask;
-  // 16-byte input loads need only element alignment for 4- and 8-byte
-  // elements (see scan_detail::u32x4_a4).
-  p.vec_io = (reinterpret_cast<uintptr_t>(in) & 3) == 0;
   p.num_tiles = static_cast<uint32_t>(num_tiles);
   p.epoch = rl.epoch;
   p.ticket_base = rl.ticket_base;

@@ -57,11 +57,12 @@ constexpr int max_waves = 16;
 constexpr int lookback_slots = 1;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-// The same 16-byte vector with only 4-byte alignment: global_load_dwordx4 /
-// global_store_dwordx4 need dword alignment only, so tiles of 4- and
-// 8-byte elements take the vector path at any element-aligned address
-// (a view such as x[1:]); the element-wise path took 1.75x as long.
-typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+// The same 16-byte vector at any address: the global loads and stores of
+// gfx950 need no alignment (unaligned access is on for HSA code objects), so
+// tiles of every element type take the vector path, also in a view such as
+// x[1:] (2 x 10^7 int16 elements in such a view: 65 us element by element,
+// SCAN_A1 us; 2^28 int8: 580 us, SCAN_A8 us).
+typedef unsigned int u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
 
 enum : uint32_t { st_invalid = 0, st_aggregate = 1, st_prefix = 2 };
 
@@ -314,7 +315,6 @@ struct params {
   W init;
   int has_init;
   int exclusive;
-  int vec_io;  // 16-byte vector loads and stores (see u32x4_a4)
   int block_lookback;
   int force_give_up;     // ACPP_VARIANT_FORCE_GIVE_UP (tests of the error path)
   int unary;             // element transform (unary.hpp) of the transform scans
@@ -323,6 +323,51 @@ struct params {
   uint32_t ticket_base;  // tile ticket counter value when this launch starts
   sync_header *sync;
   uint64_t *status;
+};
+
+// The vectors of a partial tile: those wholly in range take one load or
+// store each; at most one, of work-item `tid` and row `row`, is cut by the end
+// of the range after its first `count` elements and goes element by element.
+// (Element by element throughout, the last tile was the slowest: 1000 int8
+// elements 11.6 us, PART_I8 us.)
+struct partial_tile {
+  uint32_t in_range;  // elements of the tile in range
+  uint32_t row;
+  uint32_t tid;
+  uint32_t count;  // 0: no vector is cut
+  template <class T>
+  __device__ __forceinline__ static partial_tile of(uint32_t in_range, uint32_t B) {
+    constexpr uint32_t VEC = 16 / sizeof(T);
+    const uint32_t vec = in_range / VEC;
+    return {in_range, vec / B, vec % B, in_range % VEC};
+  }
+  __device__ __forceinline__ bool cut(uint32_t r, uint32_t t) const { return count != 0 && r == row && t == tid; }
+  // The cut vector, zero after its last element; valid in work-item `tid`.
+  template <class T>
+  __device__ __forceinline__ u32x4 load_cut(const T *tile, uint32_t t, uint32_t B) const {
+    constexpr int VEC = 16 / sizeof(T);
+    T e[VEC] = {};
+    if (count != 0 && t == tid) {
+      const T *src = tile + static_cast<uint64_t>(row * B + tid) * VEC;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+        if (static_cast<uint32_t>(k) < count) e[k] = src[k];
+    }
+    u32x4 q;
+    __builtin_memcpy(&q, e, 16);
+    return q;
+  }
+  template <class T>
+  __device__ __forceinline__ void store_cut(T *tile, u32x4 q, uint32_t t, uint32_t B) const {
+    constexpr int VEC = 16 / sizeof(T);
+    if (count == 0 || t != tid) return;
+    T e[VEC];
+    __builtin_memcpy(e, &q, 16);
+    T *dst = tile + static_cast<uint64_t>(row * B + tid) * VEC;
+#pragma unroll
+    for (int k = 0; k < VEC; ++k)
+      if (static_cast<uint32_t>(k) < count) dst[k] = e[k];
+  }
 };
 
 // Shared words of a scan work-group.
@@ -336,7 +381,7 @@ struct scan_shared {
   W red[max_waves];
 };
 
-// One tile.  FULL tiles (all R x B vectors in range, 16-byte I/O allowed)
+// One tile.  FULL tiles (all R x B vectors in range)
 // and the partial last tile are separate compile-time paths: with no join
 // after the loads, the compiler waits for each row's load only when that
 // row is processed (vmcnt(7), (6), ...), so the local and wave scans of
@@ -365,10 +410,12 @@ __device__ __forceinline__ void scan_tile(const params<T> &p, uint32_t tile,
   const uint32_t in_range = FULL ? static_cast<uint32_t>(tile_elems)
                                  : static_cast<uint32_t>(p.n > base ? min(p.n - base, tile_elems) : 0);
 
+  const partial_tile part = partial_tile::of<T>(in_range, B);
+
   // The R loads are issued back to back, then converted to the work type.
   u32x4 q[R];
+  const u32x4_a1 *src = reinterpret_cast<const u32x4_a1 *>(p.in + base);
   if constexpr (FULL) {
-    const u32x4_a4 *src = reinterpret_cast<const u32x4_a4 *>(p.in + base);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if constexpr (NT)
@@ -380,15 +427,11 @@ __device__ __forceinline__ void scan_tile(const params<T> &p, uint32_t tile,
       if constexpr (XF) __builtin_amdgcn_sched_barrier(0);
     }
   } else {
+    const u32x4 cut = part.load_cut<T>(p.in + base, tid, B);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      T tmp[VEC];
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        const uint32_t i = static_cast<uint32_t>(r * B + tid) * VEC + k;
-        tmp[k] = (i < in_range) ? p.in[base + i] : T{};
-      }
-      __builtin_memcpy(&q[r], tmp, 16);
+      q[r] = part.cut(r, tid) ? cut : u32x4{0, 0, 0, 0};
+      if (static_cast<uint32_t>(r * B + tid + 1) * VEC <= in_range) q[r] = src[r * B + tid];
     }
   }
   W v[R][VEC];
@@ -466,6 +509,8 @@ __device__ __forceinline__ void scan_tile(const params<T> &p, uint32_t tile,
     tile_prefix = sh.excl;
   }
 
+  u32x4_a1 *dst = reinterpret_cast<u32x4_a1 *>(p.out + base);
+  u32x4 cut_out = {0, 0, 0, 0};
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const W P = Op::apply(tile_prefix, Op::apply(before[r], wexcl[r]));
@@ -485,24 +530,22 @@ __device__ __forceinline__ void scan_tile(const params<T> &p, uint32_t tile,
       // every operator except the logical ones, which turn x into 0/1.
       if (r == 0 && tile == 0 && tid == 0 && !p.has_init) o[0] = static_cast<T>(v[0][0]);
     }
+    u32x4 qo;
+    __builtin_memcpy(&qo, o, 16);
     if constexpr (FULL) {
-      u32x4 qo;
-      __builtin_memcpy(&qo, o, 16);
       // Ordinary stores by default: non-temporal output stores alone
       // measured no faster (380 us against 377 us at 2^28 int32).  The NT
       // variant streams both directions, as the fastest tile copy does.
       if constexpr (NT)
-        __builtin_nontemporal_store(qo, reinterpret_cast<u32x4_a4 *>(p.out + base) + r * B + tid);
+        __builtin_nontemporal_store(qo, dst + r * B + tid);
       else
-        reinterpret_cast<u32x4_a4 *>(p.out + base)[r * B + tid] = qo;
+        dst[r * B + tid] = qo;
     } else {
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        const uint32_t i = static_cast<uint32_t>(r * B + tid) * VEC + k;
-        if (i < in_range) p.out[base + i] = o[k];
-      }
+      if (static_cast<uint32_t>(r * B + tid + 1) * VEC <= in_range) dst[r * B + tid] = qo;
+      if (part.cut(r, tid)) cut_out = qo;
     }
   }
+  if constexpr (!FULL) part.store_cut<T>(p.out + base, cut_out, tid, B);
 }
 
 template <class T, class Op, int R, bool XF = false, bool NT = false>
@@ -524,7 +567,7 @@ __global__ __launch_bounds__(1024) void scan_kernel(params<T> p) {
   if (tile >= p.num_tiles) return;
   const uint64_t tile_elems = static_cast<uint64_t>(blockDim.x) * R * VEC;
   const uint64_t base = static_cast<uint64_t>(tile) * tile_elems;
-  if (p.vec_io && base + tile_elems <= p.n)
+  if (base + tile_elems <= p.n)
     scan_tile<true, T, Op, R, XF, NT>(p, tile, sh);
   else
     scan_tile<false, T, Op, R, XF, NT>(p, tile, sh);
@@ -620,9 +663,10 @@ __device__ __forceinline__ void scan8_tile(const params<T> &p, uint32_t tile, ui
   const uint8_t *in8 = reinterpret_cast<const uint8_t *>(p.in) + base;
   uint8_t *out8 = reinterpret_cast<uint8_t *>(p.out) + base;
 
+  const partial_tile part = partial_tile::of<uint8_t>(in_range, B);
   u32x4 q[R];
+  const u32x4_a1 *src = reinterpret_cast<const u32x4_a1 *>(in8);
   if constexpr (FULL) {
-    const u32x4 *src = reinterpret_cast<const u32x4 *>(in8);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       q[r] = src[r * B + tid];
@@ -631,36 +675,11 @@ __device__ __forceinline__ void scan8_tile(const params<T> &p, uint32_t tile, ui
       if constexpr (XF) __builtin_amdgcn_sched_barrier(0);
     }
   } else {
+    const u32x4 cut = part.load_cut<uint8_t>(in8, tid, B);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      constexpr uint32_t fill4 = 0x01010101u * fill;
-      if constexpr (XF) {
-        // transform the loaded bytes, then fill the bytes past the end
-        uint32_t d[4] = {0u, 0u, 0u, 0u};
-        const uint32_t first = static_cast<uint32_t>(r * B + tid) * 16;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          if (first + k < in_range) d[k >> 2] |= static_cast<uint32_t>(in8[first + k]) << (8 * (k & 3));
-        }
-        unary_detail::apply_bytes<T>(p.unary, d);
-        const uint32_t cnt = in_range > first ? min(in_range - first, 16u) : 0u;
-#pragma unroll
-        for (int k4 = 0; k4 < 4; ++k4) {
-          const uint32_t vb = cnt > 4u * k4 ? min(cnt - 4u * k4, 4u) : 0u;  // loaded bytes in word k4
-          const uint32_t m = vb >= 4u ? ~0u : ((1u << (8u * vb)) - 1u);
-          d[k4] = (d[k4] & m) | (fill4 & ~m);
-        }
-        q[r] = u32x4{d[0], d[1], d[2], d[3]};
-      } else {
-        uint32_t d[4] = {fill4, fill4, fill4, fill4};
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const uint32_t i = static_cast<uint32_t>(r * B + tid) * 16 + k;
-          if (i < in_range)
-            d[k >> 2] = (d[k >> 2] & ~(0xffu << (8 * (k & 3)))) | (static_cast<uint32_t>(in8[i]) << (8 * (k & 3)));
-        }
-        q[r] = u32x4{d[0], d[1], d[2], d[3]};
-      }
+      q[r] = part.cut(r, tid) ? cut : u32x4{0, 0, 0, 0};
+      if (static_cast<uint32_t>(r * B + tid + 1) * 16 <= in_range) q[r] = src[r * B + tid];
     }
   }
   u16x2 P[R][8];
@@ -669,7 +688,19 @@ __device__ __forceinline__ void scan8_tile(const params<T> &p, uint32_t tile, ui
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     uint32_t d[4] = {q[r].x, q[r].y, q[r].z, q[r].w};
-    if constexpr (XF && FULL) unary_detail::apply_bytes<T>(p.unary, d);
+    if constexpr (XF) unary_detail::apply_bytes<T>(p.unary, d);
+    if constexpr (!FULL) {
+      // bytes past the end (transformed zeros by now) become the identity
+      constexpr uint32_t fill4 = 0x01010101u * fill;
+      const uint32_t first = static_cast<uint32_t>(r * B + tid) * 16;
+      const uint32_t cnt = in_range > first ? min(in_range - first, 16u) : 0u;
+#pragma unroll
+      for (int k4 = 0; k4 < 4; ++k4) {
+        const uint32_t vb = cnt > 4u * k4 ? min(cnt - 4u * k4, 4u) : 0u;  // bytes of word k4 in range
+        const uint32_t m = vb >= 4u ? ~0u : ((1u << (8u * vb)) - 1u);
+        d[k4] = (d[k4] & m) | (fill4 & ~m);
+      }
+    }
 #pragma unroll
     for (int k = 0; k < 4; ++k) d[k] ^= flip_mask;
     // pair j = (byte j, byte j + 8), zero-extended to 16 bits each
@@ -711,6 +742,8 @@ __device__ __forceinline__ void scan8_tile(const params<T> &p, uint32_t tile, ui
   }
   __syncthreads();
   const uint32_t tile_prefix = s_excl;
+  u32x4_a1 *dst = reinterpret_cast<u32x4_a1 *>(out8);
+  u32x4 cut_out = {0, 0, 0, 0};
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const uint32_t P32 = Op32::apply(tile_prefix, Op32::apply(s_wave[r * nw + w], wexcl[r]));
@@ -738,16 +771,15 @@ __device__ __forceinline__ void scan8_tile(const params<T> &p, uint32_t tile, ui
                            __builtin_amdgcn_perm(a3, a2, 0x05040100u) ^ flip_mask,
                            __builtin_amdgcn_perm(a1, a0, 0x07060302u) ^ flip_mask,
                            __builtin_amdgcn_perm(a3, a2, 0x07060302u) ^ flip_mask};
+    const u32x4 qo = {o[0], o[1], o[2], o[3]};
     if constexpr (FULL) {
-      reinterpret_cast<u32x4 *>(out8)[r * B + tid] = u32x4{o[0], o[1], o[2], o[3]};
+      dst[r * B + tid] = qo;
     } else {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const uint32_t i = static_cast<uint32_t>(r * B + tid) * 16 + k;
-        if (i < in_range) out8[i] = static_cast<uint8_t>(o[k >> 2] >> (8 * (k & 3)));
-      }
+      if (static_cast<uint32_t>(r * B + tid + 1) * 16 <= in_range) dst[r * B + tid] = qo;
+      if (part.cut(r, tid)) cut_out = qo;
     }
   }
+  if constexpr (!FULL) part.store_cut<uint8_t>(out8, cut_out, tid, B);
 }
 
 template <class T, class Op, bool XF>
@@ -764,7 +796,7 @@ __global__ __launch_bounds__(1024) void scan8_kernel(params<T> p) {
   if (tile >= p.num_tiles) return;
   const uint64_t tile_elems = static_cast<uint64_t>(blockDim.x) * R * 16;
   const uint64_t base = static_cast<uint64_t>(tile) * tile_elems;
-  if (p.vec_io && base + tile_elems <= p.n)
+  if (base + tile_elems <= p.n)
     scan8_tile<true, T, Op, R, XF>(p, tile, s_wave, s_excl);
   else
     scan8_tile<false, T, Op, R, XF>(p, tile, s_wave, s_excl);

@@ -31,11 +31,9 @@ acpp_status launch(acpp_allocation_group *g, hipStream_t stream, const T *in, ui
                    const fixed_region *fixed = nullptr) {
   using W = typename elem_traits<T>::work;
   constexpr int VEC = 16 / sizeof(T);
-  int cus = 0;
   acpp_status st = ACPP_SUCCESS;
-  if (fixed) {
-    cus = fixed->compute_units;
-  } else {
+  if (!fixed) {
+    int cus = 0;
     st = enter_device(g, &cus);
     if (st != ACPP_SUCCESS) return st;
   }
@@ -47,16 +45,17 @@ acpp_status launch(acpp_allocation_group *g, hipStream_t stream, const T *in, ui
   const bool block_lb = cfg && (cfg->flags & variant_block_lookback);
   const int dflt_rows = (packed8 && !block_lb) ? packed8_rows : default_rows<T>();
 
-  // Default work-group size: 1024-wide tiles (fewest tiles, so the fewest
-  // look-back links) when the input still gives every CU a few tiles,
-  // otherwise 256-wide tiles for parallelism on small inputs.
-  uint32_t wg = 256;
-  if (cfg && cfg->work_group_size) {
-    wg = cfg->work_group_size;
-  } else {
-    const int rows0 = (cfg && cfg->items_per_thread) ? static_cast<int>(cfg->items_per_thread) : dflt_rows;
-    if (ceil_div(n, static_cast<uint64_t>(1024) * rows0 * VEC) >= 4ull * static_cast<uint64_t>(cus)) wg = 1024;
-  }
+  // Default work-group size by bytes.  The look-back chain grows with the
+  // number of tiles, so wide tiles win as soon as there is one for about
+  // every third CU; below that narrower ones finish sooner.  1- and 2-byte
+  // elements hold a wide tile's CU longer and change over later.  Whole calls
+  // on MI355X with 256 / 512 / 1024 work-items (8 rows): int32 2^20 kernel
+  // 6.4 / 5.9 / 6.7 us, 2^23 25.7 / 18.6 / 16.3 us, 2^24 43.2 / 33.1 / 28.0
+  // us; int16 2^22 9.3 / 7.9 / 8.7 us, 2^24 26.7 / 19.9 / 16.7 us; int8 2^24
+  // 15.3 / 11.8 / 12.4 us, 2^25 27.1 / 20.8 / 19.2 us.
+  constexpr uint64_t wide_mib = sizeof(T) == 1 ? 18 : sizeof(T) == 2 ? 14 : 9;
+  const uint64_t mib = n * sizeof(T) >> 20;
+  const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : mib >= wide_mib ? 1024 : mib >= 3 ? 512 : 256;
   if (!valid_work_group_size(wg))
     return set_error(ACPP_ERROR_INVALID_ARGUMENT,
                      std::string(name) + ": work_group_size must be a multiple of 64 in [64, 1024]");
@@ -114,10 +113,6 @@ acpp_status launch(acpp_allocation_group *g, hipStream_t stream, const T *in, ui
   p.init = init;
   p.has_init = has_init ? 1 : 0;
   p.exclusive = exclusive ? 1 : 0;
-  // 16-byte vectors need 16-byte alignment for 1- and 2-byte elements, only
-  // element (4-byte) alignment for 4- and 8-byte elements.
-  p.vec_io = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) &
-              (sizeof(T) >= 4 ? 3u : 15u)) == 0;
   p.block_lookback = (cfg && (cfg->flags & variant_block_lookback)) ? 1 : 0;
   p.force_give_up = (cfg && (cfg->flags & ACPP_VARIANT_FORCE_GIVE_UP)) ? 1 : 0;
   p.unary = unary;
