@@ -224,16 +224,17 @@ __device__ __forceinline__ u32x4 load16(const T *base, uint64_t chunk) {
     return reinterpret_cast<const u32x4 *>(base)[chunk];
 }
 
-// The same load at 4-byte alignment (global_load_dwordx4 needs dword
-// alignment only): the second operand of a dot product of 4- or 8-byte
-// elements, whose misalignment may differ from the first operand's.
-typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+// The same load at any address (gfx950's global loads need no alignment): the
+// second operand of a dot product, whose misalignment may differ from the
+// first operand's (2 x 2^28 bf16 misaligned differently: 538 us element by
+// element, 187 us this way).
+typedef unsigned int u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
 template <bool NT, class T>
-__device__ __forceinline__ u32x4 load16_a4(const T *base, uint64_t chunk) {
+__device__ __forceinline__ u32x4 load16_a1(const T *base, uint64_t chunk) {
   if constexpr (NT)
-    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a4 *>(base) + chunk);
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_a1 *>(base) + chunk);
   else
-    return reinterpret_cast<const u32x4_a4 *>(base)[chunk];
+    return reinterpret_cast<const u32x4_a1 *>(base)[chunk];
 }
 
 template <class T, class W, int VEC>
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(1024) void reduce_kernel(params<T, M, OutT> p) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       qa[u] = load16<NT>(va, c + u * stride);
-      if constexpr (DOT) qb[u] = load16_a4<NT>(vb, c + u * stride);
+      if constexpr (DOT) qb[u] = load16_a1<NT>(vb, c + u * stride);
       // keeps the loads in order ahead of the transform's branch
       if constexpr (BYTE_SUM && XF) __builtin_amdgcn_sched_barrier(0);
     }
@@ -348,13 +349,13 @@ __global__ __launch_bounds__(1024) void reduce_kernel(params<T, M, OutT> p) {
     if constexpr (XF) unary_detail::apply_row<T>(p.unary, xa);
     if constexpr (DOT && BX) {
       W xb[VEC], t[VEC];
-      unpack<T, W, VEC>(load16_a4<NT>(vb, c), xb);
+      unpack<T, W, VEC>(load16_a1<NT>(vb, c), xb);
       binary_detail::apply_row<T, W, VEC>(p.binary, xa, xb, t);
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[0] = M::insert(acc[0], t[k]);
     } else if constexpr (DOT) {
       W xb[VEC];
-      unpack<T, W, VEC>(load16_a4<NT>(vb, c), xb);
+      unpack<T, W, VEC>(load16_a1<NT>(vb, c), xb);
 #pragma unroll
       for (int k = 0; k < VEC; ++k) acc[0] = M::insert2(acc[0], xa[k], xb[k]);
     } else {

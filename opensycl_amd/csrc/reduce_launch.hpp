@@ -70,14 +70,8 @@ acpp_status launch(acpp_allocation_group *g, hipStream_t stream, const T *a,
   const uintptr_t abytes = reinterpret_cast<uintptr_t>(a);
   uint64_t head = ((16 - (abytes & 15)) & 15) / sizeof(typename elem_traits<T>::storage);
   bool vec_ok = (abytes % sizeof(typename elem_traits<T>::storage)) == 0;
-  // The head aligns a; b is read with dword-aligned 16-byte loads, so for
-  // 4- and 8-byte elements it only has to be element-aligned (2-byte
-  // elements need b misaligned exactly like a).
-  if (DOT) {
-    constexpr size_t es = sizeof(typename elem_traits<T>::storage);
-    const uintptr_t bbytes = reinterpret_cast<uintptr_t>(b);
-    vec_ok = vec_ok && (es >= 4 ? (bbytes % es) == 0 : (bbytes & 15) == (abytes & 15));
-  }
+  // The head aligns a; b is read with 16-byte loads at any address.
+  if (DOT) vec_ok = vec_ok && (reinterpret_cast<uintptr_t>(b) % sizeof(typename elem_traits<T>::storage)) == 0;
   if (!vec_ok || head > n) head = n;
   const uint64_t nvec = (n - head) / VEC;
   const uint64_t tail_start = head + nvec * VEC;

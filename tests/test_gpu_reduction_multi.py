@@ -12,7 +12,7 @@ import pytest
 
 import opensycl_amd as acpp
 import oracle as O
-from gpu_util import dev, host, fold_bound, reduce_depth
+from gpu_util import dev, host, fold_bound, rand, reduce_depth
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +113,27 @@ def test_rejects_bad_arguments(gpu, q, scratch):
         acpp.reduction_multi(q, scratch, [x], [o], [acpp.BIT_AND])
     with pytest.raises(ValueError):
         acpp.reduction_multi(q, scratch, [x] * 5, [o] * 5, [acpp.PLUS] * 5)
+
+
+# One array in two, three or four of the reductions, beside others or alone,
+# at sizes around the vectors, the batches of loads and the grid.
+@pytest.mark.parametrize("dtype", [np.int8, np.int16, np.int32, np.int64, np.float32, np.float64])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_shared_arrays(gpu, q, scratch, dtype, offset):
+    torch, _ = gpu
+    ops = (acpp.PLUS, acpp.MIN, acpp.MAX, acpp.PLUS)
+    for n in (1, 15, 17, 512 * 4 * 16 - 1, 512 * 4 * 16 * 3 + 5, (1 << 21) + 3):
+        # integer-valued: float sums are exact
+        a = rand(np.int32, n + offset, seed=n, lo=-50, hi=50).astype(dtype)
+        b = rand(np.int32, n + offset, seed=n + 1, lo=-50, hi=50).astype(dtype)
+        ad, bd = dev(torch, a)[offset:], dev(torch, b)[offset:]
+        for pick in ((0, 0), (0, 0, 0), (0, 1, 0), (1, 1, 0, 0), (0, 0, 0, 0), (0, 1, 1, 1)):
+            ins = [(ad, bd)[i] for i in pick]
+            outs = [torch.zeros(1, dtype=ad.dtype, device="cuda") for _ in pick]
+            acpp.reduction_multi(q, scratch, ins, outs, ops[:len(pick)], True)
+            q.wait()
+            scratch.release()
+            for i, op, out in zip(pick, ops, outs):
+                x = (a, b)[i][offset:].astype(np.int64)
+                exp = {acpp.PLUS: x.sum(), acpp.MIN: x.min(), acpp.MAX: x.max()}[op]
+                assert host(out)[0] == np.array(exp).astype(dtype), (n, pick, op)
