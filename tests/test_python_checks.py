@@ -96,3 +96,28 @@ def test_release_refused_while_a_plan_is_alive():
         g.release()
     g.close()  # deferred while the plan lives
     assert g._close_pending
+
+
+@pytest.mark.parametrize("groups", [1, 16, 20])
+def test_closed_groups_are_kept_for_new_ones(groups):
+    """A cache keeps the handles of at most 16 closed groups per device, hands
+    each to one new group only, and gives them back with a purge or its end."""
+    cache = acpp.AllocationCache()
+    for _ in range(2):
+        opened = [acpp.AllocationGroup(cache) for _ in range(groups)]
+        assert len({g.handle.value for g in opened}) == groups
+        assert not cache._groups[0]
+        for g in opened:
+            g.close()
+            g.close()  # a second close does nothing
+            assert g.handle is None
+        assert len({h.value for h in cache._groups[0]}) == len(cache._groups[0]) == min(groups, 16)
+    cache.purge()
+    assert not cache._groups[0]
+    late = acpp.AllocationGroup(cache)
+    cache_handles = cache._groups[0]
+    acpp.AllocationGroup(cache).close()
+    assert len(cache_handles) == 1
+    late.close()
+    cache.close()
+    assert not cache_handles
