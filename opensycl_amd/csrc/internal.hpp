@@ -46,6 +46,9 @@ acpp_status check_launch(const char *kernel_name);
 // This removes the reference's separate status-initialisation kernel
 // (decoupled_lookback_scan.hpp:584-589) and any memset from the hot path.
 // ---------------------------------------------------------------------------
+constexpr uint32_t ticket_lines = 16;       // see draw_last_ticket (reduce_common.hpp)
+constexpr uint32_t ticket_line_words = 32;  // one 128-byte line each
+
 struct sync_header {
   uint32_t epoch;           // unused by eager launches (epochs are kernel arguments)
   uint32_t tile_counter;    // dynamic tile ticket, monotonic across launches
@@ -55,10 +58,12 @@ struct sync_header {
   // the host without a device read (host_trip_flag in runtime.cpp); written
   // into every region whenever the region is cleared (reset_sync_region).
   uint32_t *host_trip_flag;
-  uint32_t pad[58];         // header occupies 256 bytes
+  uint32_t pad[58];
+  uint32_t line_counters[ticket_lines * ticket_line_words];  // first-level group tickets
 };
 
-static_assert(sizeof(sync_header) == 256, "sync header is 256 bytes");
+static_assert(sizeof(sync_header) == 256 + 4 * ticket_lines * ticket_line_words,
+              "the counters above fill 256 bytes, the ticket lines follow");
 static_assert(offsetof(sync_header, host_trip_flag) == 16, "trip flag pointer is the second 16-byte chunk");
 
 // A wait inside a kernel gave up: count it in the region and raise the

@@ -16,8 +16,9 @@
 //     misaligned head/tail elements go through a scalar grid-stride loop;
 //   - the work-group reduces with DPP inside each wave and one LDS exchange
 //     across waves;
-//   - every group stores its partial, then takes a ticket; the group that
-//     draws the last ticket folds all partials in a fixed order, writes
+//   - every group stores its partial, then takes a ticket (in two levels
+//     above 96 groups, draw_last_ticket); the group that draws the last
+//     ticket folds all partials in a fixed order, writes
 //     *out and resets the ticket to zero for the next launch;
 //   - the partials are self-validating: each is stored with the launch's
 //     epoch tag (the scan's status-word layout), and the last group waits
@@ -216,6 +217,33 @@ __device__ V wait_partial(uint64_t *slots, uint64_t idx, uint32_t epoch, sync_he
   }
 }
 
+// One draw per work-group; true for the group that draws last in the launch.
+//
+// Device-scope atomics on one 128-byte line are served one after the other,
+// 11.6 ns each: 256 groups that draw from one counter spend 3 us on it, most
+// of a short reduction.  So above 96 groups the groups draw from ticket_lines
+// counters in lines of their own, and the last one of each line draws from
+// the launch's counter (a kernel that only draws: 4.2 us with one counter
+// and 2.5 us with two levels for 256 groups, 2.8 and 2.4 us for 128, 2.2 and
+// 2.4 us for 64, where the second draw's latency costs more than it saves;
+// the sum of 3 000 001 fp32 in 256 groups: 6.4 -> 4.7 us of kernel time).
+// A line's counter is zero again once its last group has drawn; the caller
+// resets done_counter.
+constexpr uint32_t one_level_groups = 96;
+__device__ __forceinline__ bool draw_last_ticket(sync_header *sync) {
+  auto draw = [](uint32_t *counter) {
+    return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const uint32_t groups = gridDim.x;
+  if (groups <= one_level_groups) return draw(&sync->done_counter) == groups - 1;
+  const uint32_t line = blockIdx.x % ticket_lines;
+  const uint32_t members = (groups - line + ticket_lines - 1) / ticket_lines;
+  uint32_t *counter = sync->line_counters + line * ticket_line_words;
+  if (draw(counter) != members - 1) return false;
+  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return draw(&sync->done_counter) == ticket_lines - 1;
+}
+
 template <bool NT, class T>
 __device__ __forceinline__ u32x4 load16(const T *base, uint64_t chunk) {
   if constexpr (NT)
@@ -343,24 +371,39 @@ __global__ __launch_bounds__(1024) void reduce_kernel(params<T, M, OutT> p) {
       }
     }
   }
-  for (; c < p.nvec; c += stride) {
-    W xa[VEC];
-    unpack<T, W, VEC>(load16<NT>(va, c), xa);
-    if constexpr (XF) unary_detail::apply_row<T>(p.unary, xa);
-    if constexpr (DOT && BX) {
-      W xb[VEC], t[VEC];
-      unpack<T, W, VEC>(load16_a1<NT>(vb, c), xb);
-      binary_detail::apply_row<T, W, VEC>(p.binary, xa, xb, t);
+  // The last, partial batch: its loads go out together too.
+  if (c < p.nvec) {
+    u32x4 qa[UNROLL - 1];
+    u32x4 qb[UNROLL - 1];
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) acc[0] = M::insert(acc[0], t[k]);
-    } else if constexpr (DOT) {
-      W xb[VEC];
-      unpack<T, W, VEC>(load16_a1<NT>(vb, c), xb);
+    for (int u = 0; u < UNROLL - 1; ++u) {
+      if (c + u * stride < p.nvec) {
+        qa[u] = load16<NT>(va, c + u * stride);
+        if constexpr (DOT) qb[u] = load16_a1<NT>(vb, c + u * stride);
+      }
+    }
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) acc[0] = M::insert2(acc[0], xa[k], xb[k]);
-    } else {
+    for (int u = 0; u < UNROLL - 1; ++u) {
+      if (c + u * stride < p.nvec) {
+        W xa[VEC];
+        unpack<T, W, VEC>(qa[u], xa);
+        if constexpr (XF) unary_detail::apply_row<T>(p.unary, xa);
+        if constexpr (DOT && BX) {
+          W xb[VEC], t[VEC];
+          unpack<T, W, VEC>(qb[u], xb);
+          binary_detail::apply_row<T, W, VEC>(p.binary, xa, xb, t);
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) acc[0] = M::insert(acc[0], xa[k]);
+          for (int k = 0; k < VEC; ++k) acc[u] = M::insert(acc[u], t[k]);
+        } else if constexpr (DOT) {
+          W xb[VEC];
+          unpack<T, W, VEC>(qb[u], xb);
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[u] = M::insert2(acc[u], xa[k], xb[k]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) acc[u] = M::insert(acc[u], xa[k]);
+        }
+      }
     }
   }
   // Scalar elements: the misaligned head and the tail.
@@ -380,26 +423,46 @@ __global__ __launch_bounds__(1024) void reduce_kernel(params<T, M, OutT> p) {
 #pragma unroll
   for (int u = 1; u < UNROLL; ++u) v = M::apply(v, acc[u]);
 
+  // Writes the result; `r` folds the whole range.
+  auto finish = [&](auto r) {
+    if constexpr (M::compensated) {
+      if (p.mode == final_with_init) r = static_cast<double>(p.init) + r;
+      else if (p.mode == final_accumulate) r = static_cast<double>(*p.out) + r;
+    } else {
+      if (p.mode == final_with_init || p.mode == final_given_identity) r = Op::apply(p.init, r);
+      else if (p.mode == final_accumulate) r = Op::apply(static_cast<W>(*p.out), r);
+    }
+    *p.out = static_cast<OutT>(r);
+  };
+
   __shared__ V s_waves[max_waves];
   __shared__ int s_last;
   V bv = block_reduce<M>(v, s_waves);
+  const bool force = p.force_give_up != 0;
+  // A single group has nothing to exchange (1000 fp32: 2.9 us with a partial
+  // and a ticket, 1.5 us without).
+  if (gridDim.x == 1 && !force) {
+    if (threadIdx.x == 0) {
+      if constexpr (M::compensated) finish(static_cast<double>(bv.s) + static_cast<double>(bv.c));
+      else finish(bv);
+    }
+    return;
+  }
   if (threadIdx.x == 0) {
-    // Tagged partial, then the ticket.  The last group waits for each
-    // partial's tag, so the order in which the two become visible does not
-    // matter; waiting for the store first (vmcnt) only makes such a wait
-    // rare.
+    // Tagged partial, then the ticket, the one right behind the other: the
+    // last group waits for each partial's tag, so the order in which the two
+    // become visible does not matter, and a store that is behind the ticket
+    // arrives within the last group's first polls.  (Waiting for the store
+    // before the ticket put its latency into every launch: 2^22 fp32 6.6 us,
+    // without it and with a batched remainder 6.3 us.)
     publish_partial(p.partials, blockIdx.x, p.epoch, bv);
-    wait_own_stores();
-    uint32_t prev = __hip_atomic_fetch_add(&p.sync->done_counter, 1u, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (prev == gridDim.x - 1);
+    s_last = draw_last_ticket(p.sync);
   }
   __syncthreads();
   if (!s_last) return;
 
   // Last work-group: fold the partials in a fixed order.
   const int nparts = gridDim.x;
-  const bool force = p.force_give_up != 0;
   if constexpr (M::compensated) {
     // Cross-group combine of (sum, error) pairs in FP64.
     __shared__ double s_dwaves[max_waves];
@@ -409,29 +472,17 @@ __global__ __launch_bounds__(1024) void reduce_kernel(params<T, M, OutT> p) {
       d += static_cast<double>(q.s) + static_cast<double>(q.c);
     }
     d = block_reduce<double_plus<double>>(d, s_dwaves);
-    if (threadIdx.x == 0) {
-      double r = d;
-      if (p.mode == final_with_init) r = static_cast<double>(p.init) + d;
-      else if (p.mode == final_accumulate) r = static_cast<double>(*p.out) + d;
-      *p.out = static_cast<OutT>(r);
-      __hip_atomic_store(&p.sync->done_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0) finish(d);
   } else {
     V r = M::identity();
     for (int i = threadIdx.x; i < nparts; i += blockDim.x)
       r = M::apply(r, wait_partial<V>(p.partials, i, p.epoch, p.sync, force, M::identity()));
     __syncthreads();  // s_waves is reused
     r = block_reduce<M>(r, s_waves);
-    if (threadIdx.x == 0) {
-      if (p.mode == final_with_init || p.mode == final_given_identity) {
-        r = Op::apply(p.init, r);
-      } else if (p.mode == final_accumulate) {
-        r = Op::apply(static_cast<W>(*p.out), r);
-      }
-      *p.out = static_cast<OutT>(r);
-      __hip_atomic_store(&p.sync->done_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0) finish(r);
   }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&p.sync->done_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace reduce_detail

@@ -252,15 +252,11 @@ __global__ __launch_bounds__(1024) void multi_kernel(params<T> p) {
   }
   group_reduce(blockDim.x >> 6, p, v, s_waves, [&](int m, W x) {
     publish_partial(p.partials, static_cast<uint64_t>(m) * gridDim.x + blockIdx.x, p.epoch, x);
-    wait_own_stores();
   });
   __syncthreads();
   if (threadIdx.x == 0) {
-    // The last group waits for each partial's tag; the stores were waited for
-    // only to make such a wait rare.
-    const uint32_t prev =
-        __hip_atomic_fetch_add(&p.sync->done_counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = (prev == gridDim.x - 1);
+    // (the last group waits for each partial's tag)
+    s_last = reduce_detail::draw_last_ticket(p.sync);
   }
   __syncthreads();
   if (!s_last) return;

@@ -326,3 +326,33 @@ def test_reduce_large_int32_exact(gpu, q, scratch):
     acpp.reduce(q, scratch, xd, out, np.int32(0))
     q.wait()
     assert host(out)[0] == O.reduce(host(xd), np.int32(0))
+
+
+# Group counts around the one group that writes its result directly, the last
+# count with one ticket counter (96) and the 16 counters above it; each with
+# whole and partial last batches of loads.  Every launch is repeated on the
+# same scratch: the counters must be back at zero.
+@pytest.mark.parametrize("groups", [1, 2, 95, 96, 97, 111, 112, 113, 256])
+@pytest.mark.parametrize("dtype", [np.int16, np.int32, np.float64])
+def test_reduce_group_counts(gpu, q, scratch, groups, dtype):
+    torch, _ = gpu
+    per_group = 64 * 4 * (16 // np.dtype(dtype).itemsize)
+    cfg = (64, 4, 1)
+    for n in (groups * per_group, groups * per_group - 64 * 16 // np.dtype(dtype).itemsize - 1,
+              (256 * 2 + groups) * per_group + 3):
+        # integer-valued: float sums and products of two are exact
+        x = rand(np.int32, n, seed=n, lo=-50, hi=50).astype(dtype)
+        y = rand(np.int32, n, seed=n + 1, lo=-50, hi=50).astype(dtype)
+        xd, yd = dev(torch, x), dev(torch, y)
+        wide = x.astype(np.int64)
+        for _ in range(2):
+            out = [torch.full((1,), 7, dtype=xd.dtype, device="cuda") for _ in range(4)]
+            acpp.reduce(q, scratch, xd, out[0], 3, acpp.PLUS, config=cfg)
+            acpp.reduction(q, scratch, xd, out[1], acpp.MAX, False, config=cfg)
+            if dtype != np.int16:
+                acpp.transform_reduce(q, scratch, xd, yd, out[2], 0, config=cfg)
+            acpp.reduction_multi(q, scratch, [xd], [out[3]], [acpp.PLUS], True, config=cfg)
+            q.wait()
+            scratch.release()
+            exp = [wide.sum() + 3, max(wide.max(), 7), (wide * y).sum() if dtype != np.int16 else 7, wide.sum()]
+            assert [host(o)[0] for o in out] == [np.array(e).astype(dtype) for e in exp], n
