@@ -195,18 +195,24 @@ __global__ __launch_bounds__(1024) void histogram_kernel(hist_params p) {
   }
 
   __syncthreads();
-  // Groups that add to the same bins start at different ones.
+  // Groups that add to the same bins start at different ones, a wave's 64
+  // always in whole lines: `count` is rounded up to 64, and callers skip what
+  // lies past the end (10.4M keys into 500 bins: 15.5 us with a wave's bins
+  // across lines, 13.7 us so; through partials 14.0 us).
+  auto whole_waves = [](uint32_t count) { return (count + 63u) & ~63u; };
   auto rotated = [&](uint32_t i, uint32_t count) {
-    const uint32_t first = static_cast<uint32_t>(static_cast<uint64_t>(count) * chunk / p.chunks) & ~63u;
-    return i + first < count ? i + first : i + first - count;
+    const uint32_t n = whole_waves(count);
+    const uint32_t first = static_cast<uint32_t>(static_cast<uint64_t>(n) * chunk / p.chunks) & ~63u;
+    return i + first < n ? i + first : i + first - n;
   };
   if constexpr (PACKED) {
     uint32_t *mine = p.partials + (static_cast<uint64_t>(slice) * p.chunks + chunk) * half;
-    for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < whole_waves(half); i += blockDim.x) {
       if (p.partials) {
-        mine[i] = lds[i];  // both counters of the word
+        if (i < half) mine[i] = lds[i];  // both counters of the word
       } else {
         const uint32_t w = rotated(i, half);
+        if (w >= half) continue;
         const uint32_t v = lds[w];
         add_bin(bin_of(w), v & 0xffffu);
         add_bin(bin_of(w + half), v >> 16);
@@ -214,8 +220,9 @@ __global__ __launch_bounds__(1024) void histogram_kernel(hist_params p) {
     }
   } else {
     uint32_t *mine = p.partials + static_cast<uint64_t>(blockIdx.x) * p.num_bins;
-    for (uint32_t i = threadIdx.x; i < p.num_bins; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < whole_waves(p.num_bins); i += blockDim.x) {
       const uint32_t b = p.partials ? i : rotated(i, p.num_bins);
+      if (b >= p.num_bins) continue;
       uint32_t v = 0;
       for (uint32_t c = 0; c < (1u << p.copies_log2); ++c) v += lds[(b << p.copies_log2) + c];
       if (p.partials)
@@ -437,11 +444,22 @@ __global__ __launch_bounds__(1024) void strided_strip_kernel(const T *__restrict
     lds[e] = x;  // row 0's value e is read by this work-item only
   }
   __syncthreads();
-  for (uint32_t e = threadIdx.x; e < slots; e += blockDim.x) {
-    T x = lds[e];
-    for (uint32_t j = e + slots; j < used; j += slots) x = R::apply(x, lds[j]);
-    R::template atomic<scope_dev>(&target[(p.gm.head + first_column * VEC + e) % p.num_slots], x);
+  // Four to one per step: with 18 slots a chain of 57 LDS reads took 2.5 us
+  // at the end of every launch.
+  for (uint32_t left = used; left > slots;) {
+    const uint32_t next = (left + 4 * slots - 1) / (4 * slots) * slots;  // whole periods
+    for (uint32_t e = threadIdx.x; e < next; e += blockDim.x) {
+      T x = lds[e];
+#pragma unroll
+      for (uint32_t j = 1; j < 4; ++j)
+        if (e + j * next < left) x = R::apply(x, lds[e + j * next]);
+      lds[e] = x;
+    }
+    __syncthreads();
+    left = next;
   }
+  for (uint32_t e = threadIdx.x; e < slots; e += blockDim.x)
+    R::template atomic<scope_dev>(&target[(p.gm.head + first_column * VEC + e) % p.num_slots], lds[e]);
   // The head and the tail (fewer than 2 VEC elements).
   if (blockIdx.x == 0)
     for (uint64_t s = threadIdx.x; s < p.gm.nscalar; s += blockDim.x) {
@@ -630,6 +648,7 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
 }
 
 constexpr uint64_t min_columns = 512;
+constexpr uint64_t max_columns = 8192;
 
 template <class T, template <class> class RT>
 acpp_status strided(acpp_allocation_group *g, hipStream_t stream, const T *values, uint64_t n,
@@ -664,19 +683,40 @@ acpp_status strided(acpp_allocation_group *g, hipStream_t stream, const T *value
     strip_params p;
     p.gm = make_geom(values, n);
     p.num_slots = num_slots;
-    // The shortest row of whole vectors, repeated to min_columns so that a
-    // last, partly used strip costs little.
+    // The shortest row of whole vectors, repeated to min_columns at least.
     p.columns = num_slots / std::gcd<uint64_t>(VEC, num_slots);
-    if (p.columns < min_columns) p.columns *= ceil_div(min_columns, p.columns);
+    // Inputs that the last-level cache does not hold beside others stream past
+    // it, in strips of 4 KiB a row (1 KiB cached and 4 KiB streaming: 2^28
+    // fp32 into 1024 slots 169 and 157 us, 240 MB 44.6 and 39.2 us, 180 MB
+    // 33.2 and 31.6 us, 130 MB 21.9 and 25.7 us).
+    const bool large = n * sizeof(T) >= (160ull << 20);
+    const uint32_t narrow = large ? 8 : 6;
+    // Where the last strip of that row would leave more than a quarter of the
+    // groups idle, the row up to max_columns with the least of it, in whole
+    // cache lines (2^27 fp32 max into 18 slots: 513 columns in 3 strips 92
+    // us, 1512 in 6 strips 81 us).  Less idle costs nothing, the loads are
+    // bound by the memory (2^26 fp32 into 777 slots: 777 columns in 4 strips
+    // 44.7 us, 6216 in 25 strips 46.8 us).
+    auto idle = [&](uint64_t columns) {
+      const uint64_t whole = ceil_div(columns, 1ull << narrow) << narrow;
+      return static_cast<double>(whole - columns) / static_cast<double>(whole);
+    };
+    const uint64_t line_row = std::lcm<uint64_t>(p.columns, 8);
+    const uint64_t tallest = std::min(max_columns, p.gm.nvec / (4 * ceil_div(wg, 1ull << narrow)));
+    p.columns *= ceil_div(min_columns, p.columns);
+    double least = idle(p.columns);
+    if (least > 0.26)
+      for (uint64_t c = ceil_div(min_columns, line_row) * line_row; c <= tallest && least > 1.0 / 64; c += line_row)
+        if (idle(c) < least) {
+          p.columns = c;
+          least = idle(c);
+        }
     const uint64_t used_columns = std::max<uint64_t>(1, std::min(p.columns, p.gm.nvec));
     const uint64_t rows = std::max<uint64_t>(1, ceil_div(p.gm.nvec, p.columns));
-    // Inputs larger than the last-level cache stream past it.
-    const bool large = n * sizeof(T) >= (256ull << 20);
-    // Strips as narrow as a wave (fewest atomics), of 4 KiB a row for large
-    // inputs (2^28 fp32 into 1024 slots: 169 us with 1 KiB, 157 us with 4 KiB;
-    // 2^23: 9.3 and 13.3 us), or wider when there are too few rows for all
+    // Strips as narrow as a wave (fewest atomics; 2^23 fp32 into 1024 slots:
+    // 9.3 us, 13.3 us with 4 KiB a row), or wider when there are too few rows for all
     // work-items.
-    p.width_log2 = large ? 8 : 6;
+    p.width_log2 = narrow;
     while ((1u << p.width_log2) < wg && (wg >> p.width_log2) > rows) ++p.width_log2;
     while ((1u << p.width_log2) > wg) --p.width_log2;
     const uint64_t strips = ceil_div(used_columns, 1ull << p.width_log2);

@@ -182,7 +182,7 @@ def test_strided_lds_form_misaligned_view(gpu, q, scratch, dtype):
         assert np.array_equal(host(t), exp), op
 
 
-# Strips of 64 columns of 16 bytes (256 above 256 MiB), rows repeated to at
+# Strips of 64 columns of 16 bytes (256 above 160 MiB), rows repeated to at
 # least 512 columns: slot counts around those edges, fewer elements than
 # slots, fewer rows than a group's bands, views, and a group size that is no
 # power of two.
@@ -210,7 +210,7 @@ def test_strided_strips(gpu, q, scratch, dtype, num_slots):
 
 
 def test_strided_strips_wide(gpu, q, scratch):
-    # above 256 MiB a strip is 256 columns wide and streams past the caches
+    # above 160 MiB a strip is 256 columns wide and streams past the caches
     torch, _ = gpu
     n = (1 << 26) + 1003
     for num_slots in (1000, 40000):
@@ -222,3 +222,38 @@ def test_strided_strips_wide(gpu, q, scratch):
         exp = v[:rows * num_slots].view(rows, num_slots).double().sum(0)
         exp[:n - rows * num_slots] += v[rows * num_slots:]
         assert torch.equal(t.double(), exp), num_slots
+
+
+# Rows of a little more than two strips are replaced by longer ones (18, 33, 50
+# and 130 slots of fp32) where the values are enough for four bands of them;
+# few slots are folded in steps of four.
+@pytest.mark.parametrize("num_slots", [1, 3, 17, 18, 33, 50, 130, 513])
+@pytest.mark.parametrize("n", [1 << 15, (1 << 21) + 5, 160 * (1 << 18) - 1, 160 * (1 << 18) + 3])
+def test_strided_long_rows(gpu, q, scratch, num_slots, n):
+    torch, _ = gpu
+    rows = n // num_slots
+    v = (torch.arange(n, device="cuda") % 7 - 3).to(torch.float32)  # sums are exact in any order
+    for op in ("add", "max"):
+        t = torch.full((num_slots,), -5.0, dtype=torch.float32, device="cuda")
+        acpp.atomic_fetch_strided(q, scratch, op, v, t)
+        q.wait()
+        whole, rest = v[:rows * num_slots].view(rows, num_slots), v[rows * num_slots:]
+        if op == "add":
+            exp = whole.double().sum(0) - 5
+            exp[:rest.numel()] += rest
+        else:
+            exp = whole.max(0).values.double()
+            exp[:rest.numel()] = torch.maximum(exp[:rest.numel()], rest.double())
+        assert torch.equal(t.double(), exp), op
+
+
+@pytest.mark.parametrize("num_bins", [1, 63, 64, 65, 127, 500, 1747, 8192, 8193, 16001])
+def test_histogram_direct_flush_whole_waves(gpu, q, scratch, num_bins):
+    torch, _ = gpu
+    for n in (1, 4097, 1 << 17, 1 << 20):
+        keys = (torch.arange(n, device="cuda") * 7919 % (num_bins + 2)).to(torch.int32)  # two out of range
+        bins = torch.full((num_bins,), 9, dtype=torch.int32, device="cuda")
+        acpp.histogram(q, scratch, keys.view(torch.uint32), bins.view(torch.uint32))
+        q.wait()
+        exp = torch.bincount(keys.long(), minlength=num_bins)[:num_bins] + 9
+        assert torch.equal(bins.long(), exp), n
