@@ -105,8 +105,8 @@ __device__ __forceinline__ uint32_t slice_bin(uint32_t local, uint32_t slice, ui
 // XCD and meet in its L2.  Bound by the instructions per visited key (four
 // keys per clock and CU).  One device atomic per key, the form before,
 // serialises on hot bins and reaches 26 G keys/s on uniform ones: 2^25
-// Zipf(1.1) keys into 200,000 bins 48.7 ms -> 76 us, 2^24 uniform keys
-// 640 -> 48 us, 2^25 Zipf keys into 1,000,000 bins 46 ms -> 249 us.  (32-bit
+// Zipf(1.1) keys into 200,000 bins 48.7 ms -> 74 us, 2^24 uniform keys
+// 640 -> 46 us, 2^25 Zipf keys into 1,000,000 bins 46 ms -> 230 us.  (32-bit
 // counters without a returned value, in twice the slices: 120 and 399 us.)
 template <bool PACKED, bool SLICED, int UNROLL>
 __global__ __launch_bounds__(1024) void histogram_kernel(hist_params p) {
@@ -273,9 +273,13 @@ __global__ __launch_bounds__(1024) void histogram_global_kernel(const uint32_t *
 // and the atomics on the bins are coalesced this way.  Integer atomics: the
 // order does not matter.  PACKED partials are the words of the LDS, 16 bits
 // a counter.
-constexpr uint32_t combine_entries = 4096;  // span << slices_log2 at most
+// Bound by the lines that the atomics touch (11 G lines/s), which is the
+// bins' bytes times gridDim.y: so the spans are short, and the grid has its
+// blocks in x (428,362 keys into 905,561 bins: 40.3 us with spans of 4096
+// entries, 28.0 us so; 2^24 keys: 142 and 121 us).
+constexpr uint32_t combine_entries = 1024;  // span << slices_log2 at most
 __host__ __device__ constexpr uint32_t combine_span_log2(uint32_t slices_log2) {
-  return slices_log2 <= 4 ? 8u : 12u - slices_log2;
+  return slices_log2 <= 1 ? 8u : slices_log2 <= 5 ? 9u - slices_log2 : 4u;
 }
 template <bool PACKED>
 __global__ __launch_bounds__(256) void histogram_combine_kernel(hist_params p) {
