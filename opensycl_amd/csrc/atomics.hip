@@ -488,15 +488,30 @@ uint32_t pick_grid(uint64_t work_items, uint32_t wg, uint64_t max_groups) {
   return static_cast<uint32_t>(g);
 }
 
-// More bins than max_plain_bins are counted in packed 16-bit fields: the
-// partials of 32-bit counters are twice the bytes (2^24 keys into 32768
-// bins: 34.0 -> 27.6 us, into 16384 bins: 25.9 -> 22.3 us).
+// More bins than max_plain_bins are counted in packed 16-bit fields, unless
+// there are few keys: the partials of 32-bit counters are twice the bytes
+// (2^24 keys into 32768 bins: 34.0 -> 27.6 us, into 16384 bins: 25.9 -> 22.3
+// us).
 constexpr uint32_t max_plain_bins = 8192;
 constexpr uint32_t max_local_bins = 65536;  // packed counters of one LDS
 constexpr uint32_t max_slices_log2 = 6;
-constexpr uint64_t direct_keys = 1ull << 17;
 constexpr uint64_t direct_keys_per_group = 4096;
-constexpr uint64_t direct_atomics = 1ull << 22;
+
+// True where the groups add their counters that are not zero straight to the
+// bins: few keys, or few bins.  No second launch and no partials, but atomics
+// on every line of the bins by every group.  Calls with the clear of the bins,
+// through partials and so: up to 2^17 keys 14.2 and 10.5 us; 2^24 keys into
+// 4096 bins 22.4 and 18.8 us, 3M into 8192 14.8 and 10.4 us; 600,000 keys
+// (147 groups) into 9548 bins 14.5 and 10.3 us, into 20000 bins 14.4 and
+// 12.5 us, into 25000 bins 14.5 and 15.5 us; 1.5M keys (256 groups) into 9548
+// bins 11.5 and 14.1 us.  In these calls the counters are plain where they fit
+// the LDS: flushing packed ones takes two atomics a word (600,000 keys into
+// 9548 bins: 14.4 us packed).
+bool direct_flush(uint64_t n, uint32_t num_bins) {
+  if (n <= (1ull << 17) || num_bins <= max_plain_bins) return true;
+  return n <= 5ull << 17 && static_cast<uint64_t>(num_bins) * 4 <= lds_bytes_budget &&
+         ceil_div(n, direct_keys_per_group) * num_bins <= 3ull << 20;
+}
 
 acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32_t *keys,
                       uint64_t n, uint32_t *bins, uint32_t num_bins, int strat,
@@ -548,7 +563,9 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
   // root.  A CU counts a key in 0.15 ns, visits one of a slice in 0.11 ns;
   // partials move at about 4 TB/s.
   const uint64_t cu_groups = static_cast<uint64_t>(cus);
-  const bool packed = num_bins > max_plain_bins;
+  const bool groups_given = cfg && cfg->groups_per_cu;
+  const bool direct = !groups_given && direct_flush(n, num_bins);
+  const bool packed = num_bins > max_plain_bins && !(direct && static_cast<uint64_t>(num_bins) * 4 <= lds_bytes_budget);
   struct form {
     uint32_t slices_log2;
     uint32_t words;  // 32-bit words of a group's partial
@@ -596,8 +613,7 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
   // contention (2^28 Zipf keys, 4096 bins on MI355X: 252 us with one group
   // per CU, 302 us with two).
   uint64_t groups = cu_groups;
-  bool direct = false;
-  if (cfg && cfg->groups_per_cu) {
+  if (groups_given) {
     int resident = 1;
     ACPP_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kernel, static_cast<int>(wg), lds));
     if (resident < 1) resident = 1;
@@ -607,16 +623,9 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
     groups = std::min(groups, std::max<uint64_t>(cu_groups, (n / 8) / num_bins));
     groups = pick_grid(gm.nvec + gm.nscalar, wg * 4, groups);
   } else {
-    // Few keys, or few bins: the counters that are not zero go straight to
-    // the bins, and there is no second launch (calls with the clear of the
-    // bins, up to 2^17 keys: 14.2 -> 10.5 us; 2^24 keys into 4096 bins: 22.4
-    // -> 18.8 us).  Above direct_atomics the partials are faster (65536 bins,
-    // 2^24 keys: 53.6 us direct, 29.7 us with partials; 32768 bins 32.8
-    // against 27.8 us; 16384 bins 22.4 against 26.0 us).
     const uint64_t part = static_cast<uint64_t>(ceil_div(n, direct_keys_per_group)) << slices_log2;
     groups = std::min(groups, part);
-    if (n > direct_keys && groups * num_bins > direct_atomics) groups = std::min(groups, static_cast<uint64_t>(best.groups) + 1);
-    else direct = true;
+    if (!direct) groups = std::min(groups, static_cast<uint64_t>(best.groups) + 1);
   }
   if (slices > 1) {
     // whole chunks: every slice of a part of the keys, on one XCD if it can be

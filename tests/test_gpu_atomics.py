@@ -247,10 +247,13 @@ def test_strided_long_rows(gpu, q, scratch, num_slots, n):
         assert torch.equal(t.double(), exp), op
 
 
-@pytest.mark.parametrize("num_bins", [1, 63, 64, 65, 127, 500, 1747, 8192, 8193, 16001])
+# Plain counters added straight to the bins (up to 8192 bins; up to 32768 for
+# at most 5 x 2^17 keys and 3 x 2^20 counters in all groups), and the packed
+# ones with partials beyond.
+@pytest.mark.parametrize("num_bins", [1, 63, 64, 65, 127, 500, 1747, 8192, 8193, 16001, 19660, 19661, 32768, 32769])
 def test_histogram_direct_flush_whole_waves(gpu, q, scratch, num_bins):
     torch, _ = gpu
-    for n in (1, 4097, 1 << 17, 1 << 20):
+    for n in (1, 4097, 1 << 17, (1 << 17) + 1, 5 << 17, (5 << 17) + 1, 1 << 20):
         keys = (torch.arange(n, device="cuda") * 7919 % (num_bins + 2)).to(torch.int32)  # two out of range
         bins = torch.full((num_bins,), 9, dtype=torch.int32, device="cuda")
         acpp.histogram(q, scratch, keys.view(torch.uint32), bins.view(torch.uint32))
