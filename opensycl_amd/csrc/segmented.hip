@@ -332,16 +332,20 @@ __global__ __launch_bounds__(256) void tile_table_kernel(const uint64_t *__restr
 // The same table written by the segments: segment s is the last to start
 // before every tile boundary in (offsets[s], offsets[s + 1]].  One round trip
 // where the search above takes five or more, but it reads all offsets.  A
-// segment of more than serial_tiles tiles is written by the whole work-group.
+// segment of more than serial_tiles tiles is written by 16 lanes, one of more
+// than shared_tiles by the whole work-group (by the whole group from 9 tiles
+// on, 120M int32 in 3977 segments took 93 us, 87 us so;
+// 30M int64 in 1000 55 and 49 us).
 __global__ __launch_bounds__(256) void tile_scatter_kernel(const uint64_t *__restrict__ offsets, uint64_t num_segments,
                                                            uint64_t tile_elems, uint32_t num_tiles,
                                                            uint32_t *tile_seg) {
-  constexpr uint32_t serial_tiles = 8;
-  __shared__ uint32_t s_count;
+  constexpr uint32_t serial_tiles = 4;
+  constexpr uint32_t shared_tiles = 512;
+  __shared__ uint32_t s_count[2];  // segments for 16 lanes, from slot 0 up; for the group, from 255 down
   __shared__ uint32_t s_seg[256];
   __shared__ uint32_t s_first[256];
   __shared__ uint32_t s_last[256];
-  if (threadIdx.x == 0) s_count = 0;
+  if (threadIdx.x < 2) s_count[threadIdx.x] = 0;
   __syncthreads();
   const uint64_t s = blockIdx.x * 256ull + threadIdx.x;
   if (s < num_segments) {
@@ -349,7 +353,9 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(const uint64_t *__res
     const uint32_t first = static_cast<uint32_t>(min(b + 1, static_cast<uint64_t>(num_tiles)));
     const uint32_t last = static_cast<uint32_t>(min(e + 1, static_cast<uint64_t>(num_tiles)));  // exclusive
     if (last > first + serial_tiles) {
-      const uint32_t slot = atomicAdd(&s_count, 1u);
+      const bool whole = last - first > shared_tiles;
+      const uint32_t place = atomicAdd(&s_count[whole ? 1 : 0], 1u);
+      const uint32_t slot = whole ? 255u - place : place;
       s_seg[slot] = static_cast<uint32_t>(s) + 1;
       s_first[slot] = first;
       s_last[slot] = last;
@@ -362,8 +368,9 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(const uint64_t *__res
     tile_seg[num_tiles] = static_cast<uint32_t>(num_segments);
   }
   __syncthreads();
-  const uint32_t count = s_count;
-  for (uint32_t i = 0; i < count; ++i)
+  for (uint32_t i = threadIdx.x >> 4; i < s_count[0]; i += 16)
+    for (uint32_t t = s_first[i] + (threadIdx.x & 15u); t < s_last[i]; t += 16) tile_seg[t] = s_seg[i];
+  for (uint32_t i = 256u - s_count[1]; i < 256u; ++i)
     for (uint32_t t = s_first[i] + threadIdx.x; t < s_last[i]; t += 256) tile_seg[t] = s_seg[i];
 }
 
@@ -1135,15 +1142,21 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
 //           < 12 MiB: 1024 x 2;  < 64 MiB: 1024 x 4;  n < 2^26: 512 x 8;
 //           otherwise 1024 x 8
 //   reduce: n < 2^16: 128 x 2;  n < 2^20: 256 x 2;  < 20 MiB: 1024 x 2;
-//           < 48 MiB: 1024 x 4;  otherwise 256 x 4 (8-byte: 512 x 4)
+//           < 48 MiB: 1024 x 4;  otherwise 256 x 4 (8-byte: 512 x 4), but
+//           with at most one segment per 2^14 elements 1024 x 4 (60M int32 in
+//           1000 segments 46.3 and 42.1 us, in 300 44.4 and 44.8 us, in 20000
+//           42.4 and 51.6 us), and 512 x 2 from 320 MiB (204M int32 in 300
+//           segments 137.0 and 130.0 us, in 3977 140.1 and 134.7 us, in
+//           100,000 139.0 and 158.1 us)
 // 2-row scans of up to max_search_tiles tiles and reductions of as many
 // tiles need one launch less, so the tiles grow with the input as long as
 // they stay below that (2^20 fp32 scan: 8.5 us at 1024 x 2, 11.6 us at 512 x
 // 8; 2^23 fp32 reduction: 11.9 us at 1024 x 4, 14.7 us at 1024 x 2).  Large
 // scans take 8-row tiles (two 512-wide or one 1024-wide group per CU, 123
-// VGPRs for int64); large reductions take 4-row tiles, which leave room for
+// VGPRs for int64); large reductions take 2- or 4-row tiles, which leave room for
 // several groups per CU (the reduction's groups never wait for each other).
-inline void default_tile(bool reduce, uint64_t total, int elem_bytes, uint32_t &wg, int &rows) {
+inline void default_tile(bool reduce, uint64_t total, uint64_t num_segments, int elem_bytes, uint32_t &wg,
+                         int &rows) {
   const bool wide = elem_bytes == 8;
   const uint64_t mib = total * elem_bytes >> 20;
   if (total < (1ull << 20)) {
@@ -1155,6 +1168,10 @@ inline void default_tile(bool reduce, uint64_t total, int elem_bytes, uint32_t &
   } else if (reduce) {
     rows = mib < 20 ? 2 : 4;
     wg = mib < 48 ? 1024 : (wide ? 512 : 256);
+    if (mib >= 48 && num_segments <= total >> 14) {
+      wg = mib < 320 ? 1024 : 512;
+      rows = mib < 320 ? 4 : 2;
+    }
   } else {
     rows = mib < 12 ? 2 : mib < 64 ? 4 : 8;
     wg = (mib < 64 || total >= (1ull << 26)) ? 1024 : 512;
@@ -1213,7 +1230,7 @@ struct call : prepared {
     if (st != ACPP_SUCCESS) return st;
     device = group_device(g);
     reduce = is_reduce;
-    default_tile(reduce, total, static_cast<int>(sizeof(T)), wg, rows);
+    default_tile(reduce, total, num_segments, static_cast<int>(sizeof(T)), wg, rows);
     if (cfg && cfg->work_group_size) wg = cfg->work_group_size;
     if (!valid_work_group_size(wg))
       return set_error(ACPP_ERROR_INVALID_ARGUMENT, std::string(name) + ": bad work_group_size");

@@ -50,9 +50,10 @@ CONFIGS = [(wg, r) for wg in WORK_GROUP_SIZES for r in ROWS]
 DEFAULT_CONFIG = (512, 4)
 
 
-def default_config(kind: str, n: int, dtype: str = "i32") -> tuple:
+def default_config(kind: str, n: int, dtype: str = "i32", segments: int | None = None) -> tuple:
     """The library's own choice when no configuration is given: the size
-    and element-size rule of segmented.hip (default_tile)."""
+    and element-size rule of segmented.hip (default_tile).  Without
+    `segments`: the choice for many."""
     width = DTYPES.get(dtype, 4)
     mib = n * width >> 20
     if n < (1 << 16):
@@ -62,6 +63,8 @@ def default_config(kind: str, n: int, dtype: str = "i32") -> tuple:
     if kind == "reduce":
         if mib < 48:
             return (1024, 2) if mib < 20 else (1024, 4)
+        if segments is not None and segments <= n >> 14:
+            return (1024, 4) if mib < 320 else (512, 2)
         return (512, 4) if width == 8 else (256, 4)
     if mib < 64:
         return (1024, 2) if mib < 12 else (1024, 4)

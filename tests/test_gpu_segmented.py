@@ -349,3 +349,21 @@ def test_plan_launched_eagerly_and_in_a_graph(gpu, n):
     red.close()
     scratch.close()
     cache.close()
+
+
+# Large reductions: few segments and one more than few (the tile differs), and
+# segments of very different lengths, whose tiles one work-item, 16 lanes or
+# the whole group write.
+@pytest.mark.parametrize("segments", [1, 5, 767, 768, 769, 4000])
+def test_segmented_reduce_tiles_by_segments(gpu, q, scratch, segments):
+    torch, _ = gpu
+    n = 768 << 14  # 48 MiB of int32
+    gen = torch.Generator().manual_seed(segments)
+    cuts = (torch.rand(segments - 1, generator=gen).double() ** 3 * n).long().sort().values
+    offsets = torch.cat([torch.tensor([0]), cuts, torch.tensor([n])])
+    x = torch.randint(-1000, 1000, (n,), dtype=torch.int32, generator=gen)
+    sums = torch.cat([torch.tensor([0]), x.long().cumsum(0)])[offsets]
+    out = torch.zeros(segments, dtype=torch.int32, device="cuda")
+    acpp.segmented_reduce(q, scratch, x.cuda(), offsets.cuda().view(torch.uint64), out)
+    q.wait()
+    assert torch.equal(out.cpu().long(), sums[1:] - sums[:-1])
