@@ -1143,11 +1143,12 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
 //           otherwise 1024 x 8
 //   reduce: n < 2^16: 128 x 2;  n < 2^20: 256 x 2;  < 20 MiB: 1024 x 2;
 //           < 48 MiB: 1024 x 4;  otherwise 256 x 4 (8-byte: 512 x 4), but
-//           with at most one segment per 2^14 elements 1024 x 4 (60M int32 in
-//           1000 segments 46.3 and 42.1 us, in 300 44.4 and 44.8 us, in 20000
-//           42.4 and 51.6 us), and 512 x 2 from 320 MiB (204M int32 in 300
-//           segments 137.0 and 130.0 us, in 3977 140.1 and 134.7 us, in
-//           100,000 139.0 and 158.1 us)
+//           with one segment per 2^14 to 2^17 elements 1024 x 4 (the tiles are
+//           then few enough for the segments to write their table: 60M int32
+//           in 1000 segments 46.3 and 42.1 us, in 48 40.5 and 42.8 us, in
+//           20000 42.4 and 51.6 us), and 512 x 2 from 320 MiB with at most one
+//           per 2^14 (204M int32 in 300 segments 137.0 and 130.0 us, in 3977
+//           140.1 and 134.7 us, in 100,000 139.0 and 158.1 us)
 // 2-row scans of up to max_search_tiles tiles and reductions of as many
 // tiles need one launch less, so the tiles grow with the input as long as
 // they stay below that (2^20 fp32 scan: 8.5 us at 1024 x 2, 11.6 us at 512 x
@@ -1168,9 +1169,12 @@ inline void default_tile(bool reduce, uint64_t total, uint64_t num_segments, int
   } else if (reduce) {
     rows = mib < 20 ? 2 : 4;
     wg = mib < 48 ? 1024 : (wide ? 512 : 256);
-    if (mib >= 48 && num_segments <= total >> 14) {
-      wg = mib < 320 ? 1024 : 512;
-      rows = mib < 320 ? 4 : 2;
+    const bool few = num_segments <= total >> 14;
+    if (mib >= 320 && few) {
+      wg = 512;
+      rows = 2;
+    } else if (mib >= 48 && few && num_segments >= total >> 17) {
+      wg = 1024;
     }
   } else {
     rows = mib < 12 ? 2 : mib < 64 ? 4 : 8;

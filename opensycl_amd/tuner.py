@@ -64,7 +64,10 @@ def default_config(kind: str, n: int, dtype: str = "i32", segments: int | None =
         if mib < 48:
             return (1024, 2) if mib < 20 else (1024, 4)
         if segments is not None and segments <= n >> 14:
-            return (1024, 4) if mib < 320 else (512, 2)
+            if mib >= 320:
+                return (512, 2)
+            if segments >= n >> 17:
+                return (1024, 4)
         return (512, 4) if width == 8 else (256, 4)
     if mib < 64:
         return (1024, 2) if mib < 12 else (1024, 4)

@@ -354,7 +354,7 @@ def test_plan_launched_eagerly_and_in_a_graph(gpu, n):
 # Large reductions: few segments and one more than few (the tile differs), and
 # segments of very different lengths, whose tiles one work-item, 16 lanes or
 # the whole group write.
-@pytest.mark.parametrize("segments", [1, 5, 767, 768, 769, 4000])
+@pytest.mark.parametrize("segments", [1, 5, 95, 96, 768, 769, 4000])
 def test_segmented_reduce_tiles_by_segments(gpu, q, scratch, segments):
     torch, _ = gpu
     n = 768 << 14  # 48 MiB of int32
