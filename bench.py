@@ -19,7 +19,7 @@ Other fields:
                    (profiles/traffic.json) when present;
   segmented     -- 65,536 segments with log-normal lengths (median 512,
                    sigma 2, clipped to [1, 2^20]): int64 segmented inclusive
-                   scan and fp32 segmented reduce, one hipGraph plan launch
+                   scan and fp32 segmented reduce, one plan launch
                    (and one direct launch) against one plain call per segment
                    issued from native code;
   other_configs -- compensated / plain fp32 and bf16 sums and dot products
@@ -258,7 +258,7 @@ def main():
 
 
 def segmented_leg(acpp, q, cache, per_segment=True):
-    """65,536 log-normal segments: batched (graph plan / direct) against one
+    """65,536 log-normal segments: batched (plan / direct) against one
     plain call per segment from native code (opensycl_amd/lib/libacpp_bench.so)."""
     import numpy as np
     import torch
