@@ -333,10 +333,16 @@ __device__ __forceinline__ void cas_select(T *p, T v, Cmp keep_old) {
   }
 }
 
+// identity() and apply() fold the elements of a slot before the one atomic on
+// it.  A NaN stays in the fold of min and max: as the last of the folded
+// elements it takes the target's place, as it does where every element has
+// an atomic of its own.  (By the atomics' rule a later element would replace
+// it in the fold, or the identity of a lane without elements, and the target
+// would never see it.)
 template <class T>
 struct rmw_min {
   __device__ static T identity() { return ops::minimum<T, T>::identity(); }
-  __device__ static T apply(T a, T b) { return ops::minimum<T, T>::apply(a, b); }
+  __device__ static T apply(T a, T b) { return (a < b || a != a) ? a : b; }
   template <int Scope>
   __device__ static void atomic(T *p, T v) {
     if constexpr (std::is_floating_point_v<T>)
@@ -349,7 +355,7 @@ struct rmw_min {
 template <class T>
 struct rmw_max {
   __device__ static T identity() { return ops::maximum<T, T>::identity(); }
-  __device__ static T apply(T a, T b) { return ops::maximum<T, T>::apply(a, b); }
+  __device__ static T apply(T a, T b) { return (a > b || a != a) ? a : b; }
   template <int Scope>
   __device__ static void atomic(T *p, T v) {
     if constexpr (std::is_floating_point_v<T>)
@@ -361,7 +367,7 @@ struct rmw_max {
 
 template <class T>
 struct rmw_add {
-  __device__ static T identity() { return T(0); }
+  __device__ static T identity() { return ops::plus<T, T>::identity(); }
   __device__ static T apply(T a, T b) { return ops::wrap_add(a, b); }
   template <int Scope>
   __device__ static void atomic(T *p, T v) {
@@ -437,9 +443,14 @@ __global__ __launch_bounds__(1024) void strided_strip_kernel(const T *__restrict
 #pragma unroll
   for (int k = 0; k < VEC; ++k) lds[threadIdx.x * VEC + k] = acc[k];
   __syncthreads();
-  // Values e, e + num_slots, ... of every row of the strip meet one slot.
+  // Values e, e + num_slots, ... of every row of the strip meet one slot.  Only
+  // slots that met an element go on to the atomics (a NaN in the target gives
+  // way to any value): those of the vectors in the group's first row.
   const uint32_t values = width * VEC;
-  const uint64_t in_row = ((p.columns < p.gm.nvec ? p.columns : p.gm.nvec) - first_column) * VEC;
+  const uint64_t first_vec = row_group * rows * p.columns + first_column;
+  const uint64_t left_in_row = p.columns - first_column;
+  const uint64_t left = p.gm.nvec > first_vec ? p.gm.nvec - first_vec : 0;
+  const uint64_t in_row = (left < left_in_row ? left : left_in_row) * VEC;
   const uint32_t used = in_row < values ? static_cast<uint32_t>(in_row) : values;
   const uint32_t slots = p.num_slots < used ? static_cast<uint32_t>(p.num_slots) : used;
   for (uint32_t e = threadIdx.x; e < used; e += blockDim.x) {
@@ -450,17 +461,17 @@ __global__ __launch_bounds__(1024) void strided_strip_kernel(const T *__restrict
   __syncthreads();
   // Four to one per step: with 18 slots a chain of 57 LDS reads took 2.5 us
   // at the end of every launch.
-  for (uint32_t left = used; left > slots;) {
-    const uint32_t next = (left + 4 * slots - 1) / (4 * slots) * slots;  // whole periods
+  for (uint32_t count = used; count > slots;) {
+    const uint32_t next = (count + 4 * slots - 1) / (4 * slots) * slots;  // whole periods
     for (uint32_t e = threadIdx.x; e < next; e += blockDim.x) {
       T x = lds[e];
 #pragma unroll
       for (uint32_t j = 1; j < 4; ++j)
-        if (e + j * next < left) x = R::apply(x, lds[e + j * next]);
+        if (e + j * next < count) x = R::apply(x, lds[e + j * next]);
       lds[e] = x;
     }
     __syncthreads();
-    left = next;
+    count = next;
   }
   for (uint32_t e = threadIdx.x; e < slots; e += blockDim.x)
     R::template atomic<scope_dev>(&target[(p.gm.head + first_column * VEC + e) % p.num_slots], lds[e]);

@@ -260,3 +260,53 @@ def test_histogram_direct_flush_whole_waves(gpu, q, scratch, num_bins):
         q.wait()
         exp = torch.bincount(keys.long(), minlength=num_bins)[:num_bins] + 9
         assert torch.equal(bins.long(), exp), n
+
+
+def _order_dependent(got, start, v, idx, num_slots, op):
+    """Float fetch_min / fetch_max: slots without a NaN hold the exact result;
+    in a slot with one, whatever the order of its elements, the result is that
+    NaN or one of the slot's numbers (numbers before the NaN, the start value
+    among them, do not survive it)."""
+    exp = np.where(np.isnan(start) & (np.arange(num_slots) < len(v)), -np.inf if op == "max" else np.inf, start)
+    with np.errstate(invalid="ignore"):
+        (np.maximum if op == "max" else np.minimum).at(exp, idx, v)  # propagates NaN
+    clean = ~np.isnan(exp)
+    assert np.array_equal(got[clean], exp[clean]), op
+    for s in np.flatnonzero(~clean):
+        assert np.isnan(got[s]) or got[s] in v[idx == s], (op, s, got[s])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n, num_slots", [(5, 3), (70, 64), (1500, 1000), (5000, 4093), (100003, 70000),
+                                          ((1 << 16) + 3, 7), ((1 << 20) + 1, 600)])
+def test_strided_fetch_min_max_nan_and_infinities(gpu, q, scratch, dtype, n, num_slots):
+    # A NaN as the last element of a slot, in slots of one and of many
+    # elements; infinities of both signs; slots of the operator's worst values.
+    torch, _ = gpu
+    v = np.round(rand(np.float64, n, seed=n) * 4).astype(dtype)
+    idx = (np.arange(n) % num_slots).astype(np.uint32)
+    last = n - 1 - (n - 1 - np.arange(min(num_slots, n))) % num_slots
+    v[last[::3]] = np.nan
+    v[np.arange(1, n, 7)] = np.inf
+    v[np.arange(2, n, 11)] = -np.inf
+    for op, worst in (("max", -np.inf), ("min", np.inf)):
+        for offset in (0, 1):
+            w = v.copy()
+            w[idx == 1] = worst  # nothing but the identity
+            start = np.full(num_slots, 1e30 if op == "max" else -1e30, dtype=dtype)
+            start[1] = worst
+            start[2::5] = np.nan  # gives way to the slot's elements
+            t = dev(torch, start)
+            buf = dev(torch, np.concatenate([np.zeros(offset, dtype=dtype), w]))[offset:]
+            acpp.atomic_fetch_strided(q, scratch, op, buf, t)
+            q.wait()
+            _order_dependent(host(t), start, w, idx, num_slots, op)
+
+
+def test_strided_fetch_add_keeps_negative_zero(gpu, q, scratch):
+    torch, _ = gpu
+    for n, num_slots in ((10, 3), (5000, 64), (100003, 70000)):
+        t = torch.full((num_slots,), -0.0, device="cuda")
+        acpp.atomic_fetch_strided(q, scratch, "add", torch.full((n,), -0.0, device="cuda"), t)
+        q.wait()
+        assert bool(torch.signbit(t).all()), (n, num_slots)
