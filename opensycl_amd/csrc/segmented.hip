@@ -810,7 +810,7 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
 // segment, keeps the results coalesced and costs no search: a binary search
 // for the segment of every last element ran in almost every step of the
 // unrolled rows once segments are short (2^26 fp32 in 1.3 million segments: 186
-// -> 67 us).  A tile in which at most three segments start takes plain folds
+// -> 67 us).  A whole tile in which at most three segments start takes plain folds
 // without any scan (2^28 fp32 in 40 segments: 514 -> 180 us with the fix-up
 // below, in 89,479 segments 184 -> 179 us).
 // --------------------------------------------------------------------------
@@ -825,6 +825,35 @@ struct reduce_parts {
 
 using constant_u32 = const __attribute__((address_space(4))) uint32_t *;
 using constant_u64 = const __attribute__((address_space(4))) uint64_t *;
+
+// Op for folds in which some lanes or accumulators hold no element but the
+// identity, to the right of others' elements too: it leaves those alone.  For
+// min and max of floating-point numbers the identity is none there:
+// max(NaN, -inf) is -inf, and the NaN would be lost.
+template <class Op, class W>
+struct skip_identity {
+  static constexpr bool needed =
+      std::is_floating_point_v<W> && (Op::id == ops::op_min || Op::id == ops::op_max);
+  __device__ static W identity() { return Op::identity(); }
+  __device__ static W apply(W a, W b) {
+    if constexpr (needed)
+      return b == Op::identity() ? a : Op::apply(a, b);
+    else
+      return Op::apply(a, b);
+  }
+};
+
+// The fold of a wave's lanes, some of which may hold the identity; uniform.
+// Every fold by Op is one of the folded values, so only the identity itself
+// can be wrong: the longer chain of skip_identity follows then alone.
+template <class Op, class W>
+__device__ __forceinline__ W fold_lanes(W x) {
+  W y = wave::reduce_full<Op>(x);
+  if constexpr (skip_identity<Op, W>::needed) {
+    if (y == Op::identity() && wave::ballot(!(x == Op::identity()))) y = wave::reduce_full<skip_identity<Op, W>>(x);
+  }
+  return y;
+}
 
 template <class T, class Op, int R>
 __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
@@ -897,7 +926,8 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
   };
   auto load_off = [&](uint32_t i) { return in_tile(p.offsets[static_cast<uint64_t>(lo) + i]); };
   const bool off_in_lds = owned + 1 <= off_cap;
-  const bool few = owned < max_pieces;
+  // (a tile cut short by the end of the input has no element in some lanes)
+  const bool few = owned < max_pieces && in_range == tile_elems;
   if (!few) {
     for (uint32_t i = tid; i < (tile_elems >> 5); i += B) s_heads[i] = 0;
     if (off_in_lds)
@@ -952,14 +982,14 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
         for (int k = 0; k < VEC; ++k) {
           const uint32_t mine = piece_of(c + lane * VEC + k);
 #pragma unroll
-          for (uint32_t j = 0; j < max_pieces; ++j) acc[j] = Op::apply(acc[j], mine == j ? v[r][k] : id);
+          for (uint32_t j = 0; j < max_pieces; ++j) acc[j] = mine == j ? Op::apply(acc[j], v[r][k]) : acc[j];
         }
       }
     }
 #pragma unroll
     for (uint32_t j = 0; j < max_pieces; ++j) {
       if (j <= owned) {
-        const W x = wave::reduce_full<Op>(acc[j]);
+        const W x = fold_lanes<Op>(acc[j]);
         if (lane == 0) s_piece[j][w] = x;
       }
     }
@@ -969,7 +999,7 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
 #pragma unroll
       for (uint32_t j = 0; j < max_pieces; ++j) {
         if (j <= owned) {
-          const W x = wave::reduce_full<Op>(lane < nw ? s_piece[j][lane] : id);
+          const W x = fold_lanes<Op>(lane < nw ? s_piece[j][lane] : id);
           if (j == 0) {
             if (lane == 0) parts.head[tile] = x;
           } else {
@@ -1060,6 +1090,7 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
                                                                reduce_parts<typename elem_traits<T>::work> parts,
                                                                uint64_t tile_elems) {
   using W = typename elem_traits<T>::work;
+  using Fold = skip_identity<Op, W>;
   constexpr uint32_t serial_span = 16;
   constexpr uint32_t wave_span = 1024;
   constexpr uint32_t max_list = 64;  // a group's tiles start at most 61 such segments
@@ -1107,7 +1138,7 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
       for (int j = 0; j < 4; ++j) acc[j] = Op::apply(acc[j], parts.head[u + static_cast<uint64_t>(j) * lanes]);
     }
     for (; u <= tl; u += lanes) acc[0] = Op::apply(acc[0], parts.head[u]);
-    return wave::reduce_full<Op>(Op::apply(Op::apply(acc[0], acc[1]), Op::apply(acc[2], acc[3])));
+    return fold_lanes<Op>(Fold::apply(Fold::apply(acc[0], acc[1]), Fold::apply(acc[2], acc[3])));
   };
   auto finish = [&](uint32_t tb, W rest) {
     p.out[parts.tail_seg[tb]] = static_cast<T>(Op::apply(p.init, Op::apply(parts.tail[tb], rest)));
@@ -1124,7 +1155,7 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
     if (lane == 0) s_red[w] = x;
     __syncthreads();
     if (w == 0) {
-      x = wave::reduce_full<Op>(lane < static_cast<int>(blockDim.x >> 6) ? s_red[lane] : id);
+      x = fold_lanes<Op>(lane < static_cast<int>(blockDim.x >> 6) ? s_red[lane] : id);
       if (lane == 0) finish(s_tile[i], x);
     }
   }

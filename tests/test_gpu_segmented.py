@@ -367,3 +367,31 @@ def test_segmented_reduce_tiles_by_segments(gpu, q, scratch, segments):
     acpp.segmented_reduce(q, scratch, x.cuda(), offsets.cuda().view(torch.uint64), out)
     q.wait()
     assert torch.equal(out.cpu().long(), sums[1:] - sums[:-1])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1], [3, 70, 1], [200, 1, 900], [5000, 2, 3000], [100000, 50001, 1],
+                                  [1 << 22, 77], [9] * 3000], ids=lambda l: f"{len(l)}x{l[0]}")
+def test_segmented_min_max_nan_and_infinities(gpu, q, scratch, dtype, lens):
+    # A NaN as the last element of every other segment, and infinities.  Whatever
+    # the order of its elements, a segment with a NaN gives that NaN or one of
+    # the segment's numbers; the others give the exact result.
+    torch, _ = gpu
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    n, S = int(off[-1]), len(lens)
+    first, last = off[:-1].astype(np.int64), off[1:].astype(np.int64) - 1
+    for op, init, worst in ((acpp.MAX, -np.inf, -np.inf), (acpp.MIN, np.inf, np.inf)):
+        x = np.round(rand(np.float64, n, seed=S) * 100).astype(dtype)
+        x[np.arange(1, n, 1013)] = -worst
+        x[first[1::4]] = worst
+        x[last[::2]] = np.nan
+        out = torch.zeros(S, dtype=torch.float32 if dtype == np.float32 else torch.float64, device="cuda")
+        acpp.segmented_reduce(q, scratch, dev(torch, x), dev(torch, off), out, init, op)
+        q.wait()
+        got = host(out)
+        for s in range(S):
+            seg = x[first[s]:last[s] + 1]
+            if s % 2 == 0:
+                assert np.isnan(got[s]) or got[s] in seg, (op, s, got[s])
+            else:
+                assert got[s] == (seg.max() if op == acpp.MAX else seg.min()), (op, s, got[s])
