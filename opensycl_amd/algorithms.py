@@ -160,10 +160,12 @@ class AllocationCache:
         check(lib.acpp_allocation_cache_create(allocation_type, ctypes.byref(h)))
         self._h = h
         self._groups: dict = {}  # device -> handles of closed (empty) groups, for new ones
+        self._alive: dict = {}   # the library's groups on this cache, open or in _groups
+        self._closing = False
 
     @property
     def handle(self):
-        return self._h
+        return None if self._closing else self._h
 
     def purge(self) -> None:
         self._destroy_groups()
@@ -172,13 +174,28 @@ class AllocationCache:
     def _destroy_groups(self) -> None:
         for pool in self._groups.values():
             while pool:
-                _abi.load().acpp_allocation_group_destroy(pool.pop())
+                self._destroy_group(pool.pop())
 
-    def close(self) -> None:
-        if self._h:
-            self._destroy_groups()
+    def _destroy_group(self, h) -> int:
+        st = _abi.load().acpp_allocation_group_destroy(h)
+        self._alive.pop(h.value, None)
+        if self._closing:
+            self._destroy()
+        return st
+
+    def _destroy(self) -> None:
+        if self._h and not self._alive:
             h, self._h = self._h, None
             check(_abi.load().acpp_allocation_cache_destroy(h))
+
+    def close(self) -> None:
+        """Free the cache.  Groups that are still open return their regions to
+        it: it is freed with the last of them (the garbage collector may
+        finalise a cache before its groups)."""
+        if self._h and not self._closing:
+            self._destroy_groups()
+            self._closing = True
+            self._destroy()
 
     def __del__(self):
         try:
@@ -197,6 +214,7 @@ class AllocationGroup:
         except (AttributeError, IndexError):
             h = ctypes.c_void_p()
             check(_abi.load().acpp_allocation_group_create(cache.handle, device, ctypes.byref(h)))
+            cache._alive[h.value] = None
             pool = cache._groups.setdefault(device, [])
         self._h = h
         self._cache = cache
@@ -241,11 +259,11 @@ class AllocationGroup:
         if self._h:
             h, self._h = self._h, None
             # emptied even when it reports an asynchronous error
-            if self._cache._h and len(self._pool) < 16:
+            if not self._cache._closing and len(self._pool) < 16:
                 st = _abi.load().acpp_allocation_group_release(h)
                 self._pool.append(h)
             else:
-                st = _abi.load().acpp_allocation_group_destroy(h)
+                st = self._cache._destroy_group(h)
             if st:
                 check(st)
 

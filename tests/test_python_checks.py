@@ -12,6 +12,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 import opensycl_amd as acpp  # noqa: E402
+from opensycl_amd import algorithms  # noqa: E402
 
 
 def t(n, dtype=torch.int32):
@@ -121,3 +122,44 @@ def test_closed_groups_are_kept_for_new_ones(groups):
     late.close()
     cache.close()
     assert not cache_handles
+
+
+class _Log:
+    """The library with every call's name noted."""
+
+    def __init__(self, lib, names):
+        self._lib, self._names = lib, names
+
+    def __getattr__(self, name):
+        fn = getattr(self._lib, name)
+
+        def call(*args):
+            self._names.append(name)
+            return fn(*args)
+        return call
+
+
+@pytest.mark.parametrize("groups", [1, 20])
+def test_cache_outlives_its_open_groups(monkeypatch, groups):
+    # a group's regions go back to its cache: a cache closed first (or
+    # finalised first, as the garbage collector may do with a cycle) is
+    # destroyed after its last group
+    cache = acpp.AllocationCache()
+    acpp.AllocationGroup(cache).close()  # one handle kept for new groups
+    opened = [acpp.AllocationGroup(cache) for _ in range(groups)]
+    names = []
+    lib = algorithms._abi.load()
+    monkeypatch.setattr(algorithms._abi, "load", lambda: _Log(lib, names))
+    cache.close()
+    cache.close()
+    assert "acpp_allocation_cache_destroy" not in names
+    with pytest.raises(acpp.AcppError):
+        acpp.AllocationGroup(cache)
+    for g in opened:
+        g.close()
+    assert names.count("acpp_allocation_group_destroy") == groups
+    assert names.count("acpp_allocation_cache_destroy") == 1
+    assert names[-1] == "acpp_allocation_cache_destroy"
+    called = len(names)
+    cache.close()
+    assert len(names) == called
