@@ -172,9 +172,12 @@ class AllocationCache:
         check(_abi.load().acpp_allocation_cache_purge(self._h))
 
     def _destroy_groups(self) -> None:
-        for pool in self._groups.values():
-            while pool:
-                self._destroy_group(pool.pop())
+        for pool in list(self._groups.values()):
+            try:
+                while True:
+                    self._destroy_group(pool.pop())
+            except IndexError:  # empty, maybe because another thread took the last one
+                pass
 
     def _destroy_group(self, h) -> int:
         st = _abi.load().acpp_allocation_group_destroy(h)

@@ -163,3 +163,15 @@ def test_cache_outlives_its_open_groups(monkeypatch, groups):
     called = len(names)
     cache.close()
     assert len(names) == called
+
+
+def test_purge_beside_a_thread_that_takes_the_last_handle():
+    class Taken(list):  # not empty when looked at, empty when popped from
+        def __len__(self):
+            return 1
+
+    cache = acpp.AllocationCache()
+    cache._groups[0] = Taken()
+    cache.purge()
+    cache._groups[0] = []
+    cache.close()
