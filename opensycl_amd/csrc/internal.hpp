@@ -171,6 +171,8 @@ struct region_state {
 
 // Obtain ordinary scratch from the group.
 acpp_status group_obtain(acpp_allocation_group *g, size_t bytes, void **out);
+// The same from what the cache holds, without an allocation; false: nothing.
+bool group_obtain_cached(acpp_allocation_group *g, size_t bytes, void **out);
 // Epoch and ticket base of one launch on a sync region.  Eager launches
 // continue the region's host-side count.  Under stream capture the graph may
 // be replayed any number of times, so the captured work clears the region

@@ -231,6 +231,14 @@ acpp_status group_obtain(acpp_allocation_group *g, size_t bytes, void **out) {
   return ACPP_SUCCESS;
 }
 
+bool group_obtain_cached(acpp_allocation_group *g, size_t bytes, void **out) {
+  allocation a;
+  if (!g->parent->find(round_request(bytes), 256, g->dev, false, a)) return false;
+  g->held.push_back(a);
+  *out = a.ptr;
+  return true;
+}
+
 namespace {
 // `stream`: where a fresh region is cleared; NULL: by its first launch.
 acpp_status obtain_sync(acpp_allocation_group *g, size_t bytes, const hipStream_t *stream, void **out,

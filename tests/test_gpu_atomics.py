@@ -4,6 +4,8 @@ Final contents must be bit-exact against the oracle's serial fold
 (order-independent operations) for both the privatized and the global
 strategy.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -310,3 +312,43 @@ def test_strided_fetch_add_keeps_negative_zero(gpu, q, scratch):
         acpp.atomic_fetch_strided(q, scratch, "add", torch.full((n,), -0.0, device="cuda"), t)
         q.wait()
         assert bool(torch.signbit(t).all()), (n, num_slots)
+
+
+def _graph_nodes(graph):
+    hip = ctypes.CDLL("libamdhip64.so")
+    nodes = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    return nodes.value
+
+
+@pytest.mark.parametrize("warm", [True, False])
+@pytest.mark.parametrize("num_bins, n", [(40000, 1 << 24), (65536, 1 << 24), (65537, 1 << 22), (200000, 1 << 22)])
+def test_captured_histogram_takes_cached_partials(gpu, q, num_bins, n, warm):
+    # Where the cache holds the scratch of an earlier call, a captured call of
+    # bins that fit one LDS goes through partials as that one did (a counting
+    # and a combining kernel); else, and with more bins, it needs no scratch (the
+    # counting kernel alone).
+    torch, _ = gpu
+    keys = rand(np.uint32, n, seed=num_bins) % np.uint32(num_bins)
+    kd = dev(torch, keys)
+    cache = acpp.AllocationCache()
+    scratch = acpp.AllocationGroup(cache)
+    bins = torch.zeros(num_bins, dtype=torch.int32, device="cuda").view(torch.uint32)
+    if warm:
+        acpp.histogram(q, scratch, kd, bins)
+        q.wait()
+        scratch.release()
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=s):
+        acpp.histogram(acpp.Queue(), scratch, kd, bins)
+    assert _graph_nodes(graph) == (2 if warm and num_bins <= 65536 else 1)
+    graph.instantiate()
+    once = O.histogram(keys, num_bins).astype(np.uint64)
+    for calls in (1, 2, 3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(host(bins), (once * (calls + warm)).astype(np.uint32))
+    del graph
+    scratch.close()
+    cache.close()
