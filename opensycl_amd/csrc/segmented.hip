@@ -810,7 +810,7 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
 // segment, keeps the results coalesced and costs no search: a binary search
 // for the segment of every last element ran in almost every step of the
 // unrolled rows once segments are short (2^26 fp32 in 1.3 million segments: 186
-// -> 67 us).  A whole tile in which at most three segments start takes plain folds
+// -> 67 us).  A tile in which at most three segments start takes plain folds
 // without any scan (2^28 fp32 in 40 segments: 514 -> 180 us with the fix-up
 // below, in 89,479 segments 184 -> 179 us).
 // --------------------------------------------------------------------------
@@ -926,8 +926,9 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
   };
   auto load_off = [&](uint32_t i) { return in_tile(p.offsets[static_cast<uint64_t>(lo) + i]); };
   const bool off_in_lds = owned + 1 <= off_cap;
-  // (a tile cut short by the end of the input has no element in some lanes)
-  const bool few = owned < max_pieces && in_range == tile_elems;
+  // (a tile cut short by the end of the input has only the identity in some lanes)
+  constexpr bool ordered = skip_identity<Op, W>::needed;
+  const bool few = owned < max_pieces && (!ordered || in_range == tile_elems);
   if (!few) {
     for (uint32_t i = tid; i < (tile_elems >> 5); i += B) s_heads[i] = 0;
     if (off_in_lds)
@@ -982,7 +983,12 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
         for (int k = 0; k < VEC; ++k) {
           const uint32_t mine = piece_of(c + lane * VEC + k);
 #pragma unroll
-          for (uint32_t j = 0; j < max_pieces; ++j) acc[j] = mine == j ? Op::apply(acc[j], v[r][k]) : acc[j];
+          for (uint32_t j = 0; j < max_pieces; ++j) {
+            if constexpr (ordered)
+              acc[j] = mine == j ? Op::apply(acc[j], v[r][k]) : acc[j];
+            else
+              acc[j] = Op::apply(acc[j], mine == j ? v[r][k] : id);
+          }
         }
       }
     }
