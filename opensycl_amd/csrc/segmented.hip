@@ -255,23 +255,115 @@ __device__ __forceinline__ uint64_t clamp_off(const uint64_t *offsets, uint64_t 
   return o < total ? o : total;
 }
 
-// The number of offsets[0 .. n) below key (offsets sorted), found by a whole
-// wave: 64 probes a round shrink the range 65 times, so 65,536 offsets take
-// three dependent loads and 2^26 five.  Unsorted offsets give some value in
-// [0, n].  The result is uniform.
-__device__ __forceinline__ uint64_t wave_lower_bound(const uint64_t *offsets, uint64_t n, uint64_t key) {
+// The number of leading positions of [0, n) that `below` holds for, found by a
+// whole wave: 64 probes a round shrink the range 65 times, so 65,536 positions
+// take three dependent loads and 2^26 five.  Where `below` does not hold for a
+// prefix (unsorted offsets), some value in [0, n].  The result is uniform.
+template <class Below>
+__device__ __forceinline__ uint64_t wave_partition_point(uint64_t n, Below below) {
   const uint64_t lane = threadIdx.x & 63;
   uint64_t lo = 0, hi = n;
   while (lo < hi) {
     const uint64_t step = (hi - lo + 64) / 65;
     const uint64_t at = lo + (lane + 1) * step - 1;
-    const bool below = at < hi && offsets[at] < key;
-    const uint64_t c = static_cast<uint64_t>(__builtin_popcountll(wave::ballot(below)));
+    const uint64_t c = static_cast<uint64_t>(__builtin_popcountll(wave::ballot(at < hi && below(at))));
     if (c < 64) hi = min(hi, lo + (c + 1) * step - 1);
     lo += c * step;
   }
   return lo;
 }
+
+// The number of offsets[0 .. n) below key.
+__device__ __forceinline__ uint64_t wave_lower_bound(const uint64_t *offsets, uint64_t n, uint64_t key) {
+  return wave_partition_point(n, [&](uint64_t i) { return offsets[i] < key; });
+}
+
+// Sets bit `at` of s_heads; none for no_head.  Lanes that follow one with the
+// same bit leave it to that one: the starts of a run of empty segments are
+// one address, and their atomics would go one after the other.
+constexpr uint32_t no_head = 0xffffffffu;
+__device__ __forceinline__ void mark_head(uint32_t *s_heads, uint32_t at) {
+  const uint32_t before = wave::dpp<wave::wave_shr1, 0xf, 0xf>(no_head, at);
+  if (at != no_head && at != before) atomicOr(&s_heads[at >> 5], 1u << (at & 31));
+}
+
+// Segments that a work-group walks one by one.  Where more start in its tile,
+// most of them are empty, and it looks the tile's starts up by element instead
+// (tile_starts): 30,000 empty segments in one place of 2^26 int32, 256 x 4 tiles,
+// 113 us of reduce kernel walked and 63 us looked up; but two starts per element
+// everywhere (2^23 int32, 1024 x 4 tiles) 111 us a call walked and 260 us
+// looked up.
+__host__ __device__ constexpr uint32_t max_walk_segments(uint32_t work_group) {
+  return work_group > 256 ? 64u * work_group : 16384u;
+}
+// Calls with at most this many segments have kernels without that: a walk of
+// 16 rounds is the worst that can happen to them.
+__host__ __device__ constexpr uint32_t max_few_segments(uint32_t work_group) { return 16u * work_group; }
+
+// The starts offsets[lo .. lo + count) of a tile whose first element is `base`,
+// however many: one binary search finds, for each of the wave's blocks of 64
+// elements, the starts in it; a second one inside the block finds each
+// element's.
+struct tile_starts {
+  const uint64_t *starts;
+  uint64_t base;
+  uint32_t in_range;  // elements of the tile
+  uint32_t b0, b1;    // the wave's blocks (at most 32)
+  uint32_t bound;     // lane i: the starts before block b0 + i (search)
+
+  __device__ __forceinline__ tile_starts(const uint64_t *offsets, uint64_t lo, uint64_t base_, uint32_t in_range_,
+                                         uint32_t bound_ = 0)
+      : starts(offsets + lo), base(base_), in_range(in_range_), bound(bound_) {
+    const uint32_t waves = blockDim.x >> 6;
+    const uint32_t blocks = (in_range + 63) / 64;
+    const uint32_t each = (blocks + waves - 1) / waves;
+    b0 = min((threadIdx.x >> 6) * each, blocks);
+    b1 = min(b0 + each, blocks);
+  }
+
+  __device__ __forceinline__ void search(uint32_t count) {
+    const uint64_t key = base + (b0 + (threadIdx.x & 63)) * 64ull;
+    uint32_t l = 0, h = count;
+    while (l < h) {
+      const uint32_t mid = l + (h - l) / 2;
+      if (starts[mid] < key)
+        l = mid + 1;
+      else
+        h = mid;
+    }
+    bound = l;
+  }
+
+  // f(e, i, found) for the elements e of the blocks in which segments start, by
+  // whole waves: found, if a segment starts at e, with the last one that does,
+  // lo + i (the only one of them that can hold elements).
+  template <class F>
+  __device__ __forceinline__ void for_each(F f) const {
+    for (uint32_t b = b0; b < b1; ++b) {
+      const uint32_t first = wave::read_lane(bound, static_cast<int>(b - b0));
+      const uint32_t last = wave::read_lane(bound, static_cast<int>(b - b0) + 1);
+      if (last <= first) continue;
+      const uint32_t e = b * 64 + (threadIdx.x & 63);
+      uint32_t l = first, h = last;
+      while (l < h) {
+        const uint32_t mid = l + (h - l) / 2;
+        if (starts[mid] <= base + e)
+          l = mid + 1;
+        else
+          h = mid;
+      }
+      f(e, l - 1, e < in_range && l > first && starts[l - 1] == base + e);
+    }
+  }
+
+  // The head bits of the blocks in which segments start.
+  __device__ __forceinline__ void mark(uint32_t *s_heads) const {
+    for_each([&](uint32_t e, uint32_t, bool found) {
+      const uint64_t bits = wave::ballot(found);
+      if ((e & 31u) == 0) s_heads[e >> 5] = static_cast<uint32_t>(bits >> (e & 32u));
+    });
+  }
+};
 
 // The segments whose start lies in [first, last) (all from the first one on
 // when to_end): found by the work-group's first and last wave, returned to
@@ -375,32 +467,70 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(const uint64_t *__res
 }
 
 // The head bitmap of the scans: bit b for every segment start b < total (the
-// start of an empty segment is that of the next one that is not empty).  A
-// work-group marks 32 x WORDS elements in LDS from the offsets inside its
-// range and writes the words once: the bitmap needs no clearing and no global
-// atomics.  (A fill, then one global atomicOr per segment: 2^26 elements in
-// 13.4 million segments took 450 us of 558.)
-template <uint32_t WORDS>
+// start of an empty segment is that of the next one that is not empty).  The
+// starts and the words are merged, a word behind the starts in it, and every
+// work-group takes `part` of that order, a start counting 1 and a word
+// word_weight: the work does not depend on where the empty segments are (by
+// words alone, 10 million in one place of 2^23 elements took 11.7 ms).  A group
+// marks the words that end in its part in LDS and writes them once: the bitmap
+// needs no clearing and no global atomics.  (A fill, then one global atomicOr
+// per segment: 2^26 elements in 13.4 million segments took 450 us of 558.)
+constexpr uint32_t word_weight = 8;
 __global__ __launch_bounds__(256) void head_bitmap_kernel(const uint64_t *__restrict__ offsets, uint64_t num_segments,
-                                                          uint64_t total, uint64_t head_words, uint32_t *heads) {
-  __shared__ uint32_t s_words[WORDS];
-  __shared__ uint64_t s_range[2];
-  const uint64_t base = blockIdx.x * 32ull * WORDS;
-  const uint64_t end = min(base + 32ull * WORDS, total);
-  find_segments(offsets, num_segments, base, end, false, s_range);
-  for (uint32_t i = threadIdx.x; i < WORDS; i += 256) s_words[i] = 0;
-  __syncthreads();
-  const uint64_t hi = s_range[1];
-#pragma unroll 4
-  for (uint64_t i = s_range[0] + threadIdx.x; i < hi; i += 256) {
-    const uint64_t b = offsets[i];
-    if (b >= base && b < end) atomicOr(&s_words[(b - base) >> 5], 1u << (b & 31));
+                                                          uint64_t total, uint64_t head_words, uint32_t part,
+                                                          uint32_t *heads) {
+  extern __shared__ uint32_t s_words[];  // part / word_weight
+  __shared__ uint64_t s_start[2];  // first start of the group's part, and of the next
+  __shared__ uint32_t s_deep;
+  const uint64_t all = num_segments + head_words * word_weight;
+  const uint64_t d0 = static_cast<uint64_t>(blockIdx.x) * part;
+  const uint64_t d1 = min(d0 + part, all);
+  const uint32_t tid = threadIdx.x;
+  auto word_of = [&](uint64_t i) { return clamp_off(offsets, i, total) >> 5; };
+  if (tid < 64 || tid >= 192) {
+    const uint64_t d = tid < 64 ? d0 : d1;
+    const uint64_t i = wave_partition_point(num_segments, [&](uint64_t i) { return i + word_of(i) * word_weight < d; });
+    if ((tid & 63) == 0) s_start[tid < 64 ? 0 : 1] = i;
   }
+  for (uint32_t i = tid; i < part / word_weight; i += 256) s_words[i] = 0;
+  if (tid == 0) s_deep = 0;
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < WORDS; i += 256) {
-    const uint64_t w = blockIdx.x * static_cast<uint64_t>(WORDS) + i;
-    if (w < head_words) heads[w] = s_words[i];
+  const uint64_t i0 = s_start[0], i1 = s_start[1];
+  // the words before the part are those whose weight is left of d0
+  const uint64_t w0 = min(head_words, (d0 > i0 ? d0 - i0 : 0) / word_weight);
+  const uint64_t w1 = min(head_words, (d1 > i1 ? d1 - i1 : 0) / word_weight);
+  if (w1 <= w0) return;  // a part of a run of empty segments
+  const uint32_t words = static_cast<uint32_t>(min(w1 - w0, static_cast<uint64_t>(part / word_weight)));
+  const uint64_t base = w0 << 5;
+  const uint64_t end = min(static_cast<uint64_t>(words) << 5, total > base ? total - base : 0);
+  auto mark = [&](uint64_t b) { mark_head(s_words, b - base < end ? static_cast<uint32_t>(b - base) : no_head); };
+  // The first word can hold starts of the parts before, too: the last 256 of
+  // them, and if those all lie in it (or at the end of the input in it),
+  // whatever there is, bit by bit (below).
+  if (tid < i0) {
+    const uint64_t b = offsets[i0 - 1 - tid];
+    mark(b);
+    if (tid == 255 && min(b, total) >> 5 == w0) s_deep = 1;
   }
+#pragma unroll 8
+  for (uint64_t i = i0 + tid; i < i1; i += 256) mark(offsets[i]);
+  __syncthreads();
+  if (s_deep) {
+    if (tid < 32) {
+      const uint64_t key = base + tid;
+      uint64_t lo = 0, hi = i0;
+      while (lo < hi) {
+        const uint64_t mid = lo + (hi - lo) / 2;
+        if (offsets[mid] < key)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      if (lo < i0 && offsets[lo] == key && key < total) atomicOr(&s_words[0], 1u << tid);
+    }
+    __syncthreads();
+  }
+  for (uint32_t i = tid; i < words; i += 256) heads[w0 + i] = s_words[i];
 }
 
 // 32-bit words of a reduction tile's head bits, rounded up so that the values
@@ -464,7 +594,8 @@ __device__ __forceinline__ uint32_t fold_wave_prefixes(uint32_t fm, W (&v)[R][VE
 
 // MARK: the tile marks its segment starts from the offsets itself instead of
 // reading the bitmap (small inputs: one launch instead of two).
-template <class T, class Op, int R, bool MARK>
+// RUNS: more segments than max_few_segments.
+template <class T, class Op, int R, bool MARK, bool RUNS = false>
 __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
   using W = typename elem_traits<T>::work;
   using SIO = seg_status<W>;
@@ -573,10 +704,17 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
       s_heads[tid + B] = hword1 & hmask1;
       __syncthreads();
       if constexpr (MARK) {
-        const uint64_t hi = s_range[1];
-        for (uint64_t i = s_range[0] + tid; i < hi; i += B) {
-          const uint64_t b = p.offsets[i];
-          if (b >= base && b - base < in_range) atomicOr(&s_heads[(b - base) >> 5], 1u << (b & 31));
+        const uint64_t lo = s_range[0], hi = s_range[1];
+        if (RUNS && hi > lo && hi - lo > max_walk_segments(B)) {
+          tile_starts starts(p.offsets, lo, base, in_range);
+          starts.search(static_cast<uint32_t>(hi - lo));
+          starts.mark(s_heads);
+        } else {
+#pragma unroll 4
+          for (uint64_t i = lo + tid; i < hi; i += B) {
+            const uint64_t b = p.offsets[i];
+            mark_head(s_heads, b >= base && b - base < in_range ? static_cast<uint32_t>(b - base) : no_head);
+          }
         }
         __syncthreads();
       }
@@ -816,6 +954,14 @@ __global__ __launch_bounds__(1024) void segmented_kernel(params<T> p) {
 // --------------------------------------------------------------------------
 constexpr uint32_t no_segment = 0xffffffffu;
 
+// Where the segments of such a run (those from a multiple of empty_run up to
+// the next one) all start in one tile, the fix-up kernel writes init to its
+// empty ones: empty_runs runs a work-group, so that millions of empty segments
+// in one place are spread over the chip.
+constexpr uint32_t empty_run = 8192;
+constexpr uint32_t empty_runs = 2;
+static_assert(2 * empty_run <= max_walk_segments(64) && 16 % empty_runs == 0, "a tile that does not walk its segments holds a whole run");
+
 template <class W>
 struct reduce_parts {
   W *head;
@@ -855,8 +1001,12 @@ __device__ __forceinline__ W fold_lanes(W x) {
   return y;
 }
 
-template <class T, class Op, int R>
-__global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
+// RUNS: more segments than max_few_segments (a kernel of its own: with that code
+// in it the other one takes 72 -> 80 us for 120M fp32 in 40 segments, 512 x 2
+// tiles).
+// At most 64 registers for 2 and 4 rows: two 1024-wide groups on a CU.
+template <class T, class Op, int R, bool RUNS>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(R == 8 ? 4 : 8))) void segmented_reduce_kernel(params<T> p,
                                                                 reduce_parts<typename elem_traits<T>::work> parts) {
   using W = typename elem_traits<T>::work;
   constexpr int VEC = 16 / sizeof(T);
@@ -1025,10 +1175,20 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
     return;
   }
 
+  const bool walk = !RUNS || owned <= max_walk_segments(B);
+  uint32_t bound = 0;
   __syncthreads();
-  for (uint32_t i = tid; i < owned; i += B) {
-    const uint32_t b = off(i);
-    if (b < in_range) atomicOr(&s_heads[b >> 5], 1u << (b & 31));
+  auto mark = [&](uint32_t b) { mark_head(s_heads, b < in_range ? b : no_head); };
+  if (RUNS && !off_in_lds && walk) {
+#pragma unroll 4
+    for (uint32_t i = tid; i < owned; i += B) mark(load_off(i));
+  } else if (walk) {
+    for (uint32_t i = tid; i < owned; i += B) mark(off(i));
+  } else {
+    tile_starts starts(p.offsets, lo, base, in_range);
+    starts.search(owned);
+    starts.mark(s_heads);
+    bound = starts.bound;
   }
   __syncthreads();
 
@@ -1068,14 +1228,29 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
     reinterpret_cast<u32x4 *>(s_val)[r * B + tid] = qv;
   }
   __syncthreads();
-  for (uint32_t i = tid; i < owned; i += B) {
-    const uint32_t b = off(i);
-    const uint32_t e = off(i + 1);
+  auto result = [&](uint32_t i, uint32_t b, uint32_t e) {
     const uint64_t s = static_cast<uint64_t>(lo) + i;
     if (e <= b)
       p.out[s] = static_cast<T>(p.init);
     else if (e <= in_range)
       p.out[s] = static_cast<T>(Op::apply(p.init, s_val[e - 1]));
+  };
+  if (RUNS && !off_in_lds) {
+    // A tile that is not walked: the segments with elements, and the empty ones
+    // outside of the runs that the fix-up kernel fills.
+    uint32_t filled = owned, end = owned;
+    if (!walk) {
+      tile_starts(p.offsets, lo, base, in_range, bound).for_each([&](uint32_t, uint32_t i, bool found) {
+        if (found) result(i, load_off(i), load_off(i + 1));
+      });
+      filled = (empty_run - lo % empty_run) % empty_run;  // from here on
+      end = (hi - 1) / empty_run * empty_run - lo;        // up to here
+    }
+#pragma unroll 4
+    for (uint32_t i = tid; i < filled; i += B) result(i, load_off(i), load_off(i + 1));
+    for (uint32_t i = end + tid; i < owned; i += B) result(i, load_off(i), load_off(i + 1));
+  } else {
+    for (uint32_t i = tid; i < owned; i += B) result(i, off(i), off(i + 1));
   }
   if (tid == 0) {
     const uint32_t first = off(0);
@@ -1089,12 +1264,13 @@ __global__ __launch_bounds__(1024) void segmented_reduce_kernel(params<T> p,
 // op(init, tail[tb] . head[tb+1] . ... . head[tl]) for every segment that
 // continues from tile tb to tile tl > tb: one work-item per tile tb, a wave
 // for a segment of more than serial_span tiles, the whole group above
-// wave_span.  (One work-item per segment and eight partials in flight: 18 us
+// wave_span.  The work-groups past the first fix_groups fill the runs of empty
+// segments.  (One work-item per segment and eight partials in flight: 18 us
 // for 48 segments of 250 tiles, 3.1 ms for one segment of 65,536.)
 template <class T, class Op>
 __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
                                                                reduce_parts<typename elem_traits<T>::work> parts,
-                                                               uint64_t tile_elems) {
+                                                               uint64_t tile_elems, uint32_t fix_groups) {
   using W = typename elem_traits<T>::work;
   using Fold = skip_identity<Op, W>;
   constexpr uint32_t serial_span = 16;
@@ -1107,6 +1283,27 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
   const W id = Op::identity();
   const int w = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
+  if (blockIdx.x >= fix_groups) {
+    const uint64_t first = (blockIdx.x - fix_groups) * static_cast<uint64_t>(empty_runs) * empty_run;
+    if (threadIdx.x <= empty_runs) {
+      const uint64_t s = first + threadIdx.x * empty_run;
+      s_tile[threadIdx.x] =
+          s < p.num_segments ? static_cast<uint32_t>(min(clamp_off(p.offsets, s, p.total) / tile_elems,
+                                                         static_cast<uint64_t>(p.num_tiles - 1)))
+                             : no_segment;
+    }
+    __syncthreads();
+    constexpr uint32_t lanes = 1024 / empty_runs;  // work-items for a run
+    const uint32_t j = threadIdx.x / lanes;
+    if (s_tile[j] == no_segment || s_tile[j] != s_tile[j + 1]) return;
+#pragma unroll 8
+    for (uint32_t i = threadIdx.x % lanes; i < empty_run; i += lanes) {
+      const uint64_t s = first + j * empty_run + i;
+      const uint64_t b = p.offsets[s], e = p.offsets[s + 1];
+      if (e <= b) p.out[s] = static_cast<T>(p.init);
+    }
+    return;
+  }
   if (threadIdx.x == 0) s_count = 0;
   __syncthreads();
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1376,6 +1573,7 @@ struct call : prepared {
 
   template <class F>
   acpp_status with_scan_kernel(F &&f) {
+    if (mark && p.num_segments > max_few_segments(wg)) return f(segmented_kernel<T, Op, 2, true, true>);
     if (mark) return f(segmented_kernel<T, Op, 2, true>);
     if (rows == 2) return f(segmented_kernel<T, Op, 2, false>);
     if (rows == 4) return f(segmented_kernel<T, Op, 4, false>);
@@ -1399,23 +1597,36 @@ struct call : prepared {
       st = check_launch(name);
       if (st != ACPP_SUCCESS) return st;
     }
-    if (rows == 2)
-      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 2>), dim3(grid), dim3(wg), lds, stream, p, parts);
-    else if (rows == 4)
-      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 4>), dim3(grid), dim3(wg), lds, stream, p, parts);
-    else
-      hipLaunchKernelGGL((segmented_reduce_kernel<T, Op, 8>), dim3(grid), dim3(wg), lds, stream, p, parts);
+    auto kernel = [&](auto runs) {
+      constexpr bool RUNS = decltype(runs)::value;
+      return rows == 2   ? segmented_reduce_kernel<T, Op, 2, RUNS>
+             : rows == 4 ? segmented_reduce_kernel<T, Op, 4, RUNS>
+                         : segmented_reduce_kernel<T, Op, 8, RUNS>;
+    };
+    const bool few = num_segments <= max_few_segments(wg);
+    hipLaunchKernelGGL(few ? kernel(std::false_type{}) : kernel(std::true_type{}), dim3(grid), dim3(wg), lds, stream, p,
+                       parts);
     st = check_launch(name);
-    if (st != ACPP_SUCCESS || num_tiles == 1) return st;
-    hipLaunchKernelGGL((segmented_fixup_kernel<T, Op>), dim3(static_cast<uint32_t>(ceil_div(num_tiles, 1024))),
-                       dim3(1024), 0, stream, p, parts, tile_elems);
+    const bool walked = num_segments <= max_walk_segments(wg);  // whatever tiles they start in
+    if (st != ACPP_SUCCESS || (num_tiles == 1 && walked)) return st;
+    const uint32_t fix_groups = static_cast<uint32_t>(ceil_div(num_tiles, 1024));
+    const uint64_t fill_groups = walked ? 0 : ceil_div(num_segments, static_cast<uint64_t>(empty_runs) * empty_run);
+    hipLaunchKernelGGL((segmented_fixup_kernel<T, Op>), dim3(fix_groups + static_cast<uint32_t>(fill_groups)),
+                       dim3(1024), 0, stream, p, parts, tile_elems, fix_groups);
     return check_launch(name);
   }
 
-  template <uint32_t WORDS>
+  // Parts small enough to occupy the chip, large enough that the searches do
+  // not count (2^28 fp32 in 89,479 segments: 411 us with 1024 words, 404 us with
+  // 4096; 2^23 in 1.7 million: 31 and 56 us), with the starts that go with
+  // the words, up to one in four elements.
   acpp_status mark_heads(hipStream_t stream) {
-    hipLaunchKernelGGL(head_bitmap_kernel<WORDS>, dim3(static_cast<uint32_t>(ceil_div(head_words, WORDS))), dim3(256),
-                       0, stream, p.offsets, p.num_segments, p.total, head_words, heads);
+    const uint64_t words = p.total >= (1ull << 27) ? 4096 : p.total >= (1ull << 23) ? 1024 : 256;
+    const uint64_t all = p.num_segments + head_words * word_weight;
+    const uint64_t even = ceil_div(ceil_div(all, ceil_div(head_words, words)), word_weight) * word_weight;
+    const uint32_t part = static_cast<uint32_t>(std::min(even, 2 * words * word_weight));
+    hipLaunchKernelGGL(head_bitmap_kernel, dim3(static_cast<uint32_t>(ceil_div(all, part))), dim3(256),
+                       part / word_weight * 4, stream, p.offsets, p.num_segments, p.total, head_words, part, heads);
     return check_launch(name);
   }
 
@@ -1425,13 +1636,7 @@ struct call : prepared {
     if (st != ACPP_SUCCESS) return st;
     p.epoch = rl.epoch;
     p.ticket_base = rl.ticket_base;
-    // Chunks small enough to occupy the chip, large enough that the searches
-    // do not count (2^28 fp32 in 89,479 segments: 411 us with 1024 words, 404
-    // us with 4096; 2^23 in 1.7 million: 31 and 56 us).
-    if (!mark)
-      st = p.total >= (1ull << 27) ? mark_heads<4096>(stream)
-           : p.total >= (1ull << 23) ? mark_heads<1024>(stream)
-                                     : mark_heads<256>(stream);
+    if (!mark) st = mark_heads(stream);
     if (st == ACPP_SUCCESS)
       st = with_scan_kernel([&](auto kernel) -> acpp_status {
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(wg), lds, stream, p);

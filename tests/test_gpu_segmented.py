@@ -395,3 +395,94 @@ def test_segmented_min_max_nan_and_infinities(gpu, q, scratch, dtype, lens):
                 assert np.isnan(got[s]) or got[s] in seg, (op, s, got[s])
             else:
                 assert got[s] == (seg.max() if op == acpp.MAX else seg.min()), (op, s, got[s])
+
+
+def _empty_run_layouts():
+    """Runs of empty segments from a few to far more than a work-group walks, in
+    front, inside a tile, at a tile's edge and behind the last element, and
+    segments that are empty nearly everywhere."""
+    rng = np.random.default_rng(17)
+    for n in (0, 5, 1000, 70001, (1 << 20) + 13, 1 << 20, (1 << 23) + 77):
+        lens = np.bincount(rng.integers(0, 40, n), minlength=40) if n else np.zeros(0, dtype=np.int64)
+        for run in (300, 16384, 16385, 40000, 200001):
+            for at in sorted({0, len(lens) // 2, len(lens)}):
+                yield f"{run} at {at} of {n}", np.concatenate([lens[:at], np.zeros(run, dtype=np.int64), lens[at:]])
+        if n:
+            # runs at single elements, next to each other and at round positions
+            pos = np.unique(np.concatenate([[0, 1, 2, 31, 32, 33, 4096, 8191, 8192], rng.integers(0, n, 5), [n - 1, n]]))
+            off = np.sort(np.concatenate([np.repeat(pos[pos <= n], 20000), [0, n]]))
+            yield f"many runs in {n}", np.diff(off)
+            yield f"sparse in {n}", np.bincount(rng.integers(0, 300000, n), minlength=300000)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.float64])
+def test_runs_of_empty_segments(gpu, q, scratch, dtype):
+    torch, _ = gpu
+    for name, lens in _empty_run_layouts():
+        off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+        n, S = int(off[-1]), len(lens)
+        xi = exact_ints(torch, n, n % 1000)
+        xh = host(xi).astype(np.int64)
+        xd, od = xi.to(torch.int32 if dtype == np.int32 else torch.float64), dev(torch, off)
+        if n:
+            yd = torch.zeros_like(xd)
+            acpp.segmented_inclusive_scan(q, scratch, xd, yd, od)
+            q.wait()
+            assert np.array_equal(host(yd).astype(np.int64), O.segmented_inclusive_scan(xh, off)), name
+        out = torch.full((S,), -7, dtype=xd.dtype, device="cuda")
+        acpp.segmented_reduce(q, scratch, xd, od, out, 3)
+        q.wait()
+        assert np.array_equal(host(out).astype(np.int64), O.segmented_reduce(xh, off, np.int64(3))), name
+        scratch.release()
+
+
+@pytest.mark.parametrize("cfg", [(64, 2), (128, 8), (1024, 2), (1024, 8)])
+def test_runs_of_empty_segments_tile_sizes(gpu, q, scratch, cfg):
+    # the same with every tile size from the smallest to the largest
+    torch, _ = gpu
+    n = 300007
+    rng = np.random.default_rng(23)
+    pos = np.concatenate([np.repeat([0, 511, 512, 32767, 32768, 150000, n], 40000), rng.integers(0, n, 30000), [0, n]])
+    off = np.sort(pos).astype(np.uint64)
+    xi = exact_ints(torch, n, 1)
+    xh = host(xi).astype(np.int64)
+    config = {"work_group_size": cfg[0], "items_per_thread": cfg[1]}
+    yd = torch.zeros_like(xi)
+    out = torch.full((len(off) - 1,), -7, dtype=xi.dtype, device="cuda")
+    acpp.segmented_inclusive_scan(q, scratch, xi, yd, dev(torch, off), config=config)
+    acpp.segmented_reduce(q, scratch, xi, dev(torch, off), out, 3, config=config)
+    q.wait()
+    assert np.array_equal(host(yd).astype(np.int64), O.segmented_inclusive_scan(xh, off))
+    assert np.array_equal(host(out).astype(np.int64), O.segmented_reduce(xh, off, np.int64(3)))
+
+
+@pytest.mark.parametrize("kind", ["scan", "reduce"])
+@pytest.mark.parametrize("n", [1 << 20, 1 << 23])
+def test_runs_of_empty_segments_cost_what_spread_ones_cost(gpu, q, scratch, kind, n):
+    # 4 million empty segments in one place against as many spread over the
+    # input: one work-group that walks the run alone takes 50 times as long
+    torch, _ = gpu
+    S = 4_000_000
+    spread = np.sort(np.random.default_rng(1).integers(0, n, S + 1))
+    spread[0], spread[-1] = 0, n
+    one = np.concatenate([np.linspace(0, n // 2, 500), np.full(S - 999, n // 2), np.linspace(n // 2, n, 500)])
+    x = torch.ones(n, dtype=torch.int32, device="cuda")
+    d = torch.empty(n if kind == "scan" else S, dtype=torch.int32, device="cuda")
+    times = []
+    for off in (spread, one):
+        od = dev(torch, off.astype(np.uint64))
+        assert od.numel() == S + 1
+        samples = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            if kind == "scan":
+                acpp.segmented_inclusive_scan(q, scratch, x, d, od)
+            else:
+                acpp.segmented_reduce(q, scratch, x, od, d, 0)
+            b.record()
+            b.synchronize()
+            scratch.release()
+            samples.append(a.elapsed_time(b))
+        times.append(min(samples))
+    assert times[1] < 5 * times[0], times
