@@ -400,7 +400,7 @@ def regret(db: list, picks: list) -> dict:
         best = min(t.values())
         tp = t[_key(pick)]
         sh = rec.get("shape", {})
-        dflt = (default_config(sh["kind"], sh["n"], sh.get("dtype", "i32"))
+        dflt = (default_config(sh["kind"], sh["n"], sh.get("dtype", "i32"), sh.get("num_segments"))
                 if "kind" in sh and "n" in sh else DEFAULT_CONFIG)
         td = t[_key(dflt)]
         tf = t[_key(DEFAULT_CONFIG)]

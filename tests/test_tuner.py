@@ -114,3 +114,20 @@ def test_library_default_rule_on_committed_timings():
     assert T.default_config("reduce", 1 << 28, "f32") == (256, 4)
     assert T.default_config("reduce", 1 << 28, "f64") == (512, 4)
     assert T.default_config("reduce", 1000) == (128, 2)
+
+
+def test_library_default_rule_by_segment_count():
+    # reductions of few segments have tiles of their own (default_tile)
+    assert T.default_config("reduce", 204_000_000, "i32", segments=300) == (512, 2)
+    assert T.default_config("reduce", 204_000_000, "i32", segments=100_000) == (256, 4)
+    assert T.default_config("reduce", 60_000_000, "i32", segments=1000) == (1024, 4)
+    assert T.default_config("reduce", 60_000_000, "i32", segments=48) == (256, 4)
+    assert T.default_config("reduce", 60_000_000, "i32", segments=20_000) == (256, 4)
+    assert T.default_config("reduce", 30_000_000, "f64", segments=1000) == (1024, 4)
+    # and the regret of the default is that of the tile that the library launches
+    times = {T._key(c): 100.0 for c in T.CONFIGS}
+    times[T._key((512, 2))] = 80.0
+    rec = {"shape": {"kind": "reduce", "n": 204_000_000, "dtype": "i32", "num_segments": 300}, "times_us": times}
+    assert T.regret([rec], [(512, 2)])["default_mean_regret"] == 0.0
+    rec["shape"]["num_segments"] = 100_000
+    assert T.regret([rec], [(512, 2)])["default_mean_regret"] == pytest.approx(0.25)
