@@ -258,3 +258,48 @@ def test_look_back_kernels_share_scratch_regions(gpu, q):
             k = int(host(cnt)[0])
             assert k == exp_k and np.array_equal(host(sel)[:k], exp_sel), rep
             g.close()
+
+
+@pytest.mark.parametrize("wg", [256, 512, 1024])
+@pytest.mark.parametrize("dtype", [np.int8, np.uint8, np.int16, np.int32, np.int64])
+def test_scan_misaligned_output_and_its_surroundings(gpu, q, scratch, dtype, wg):
+    # Input and output each off 16-byte alignment by itself, also in place in an
+    # offset view: whole vectors at any address, and the vector that the end of
+    # the input cuts.  The elements around the output stay as they were.  Sizes
+    # around a vector, a wave's row, a group's row and tiles of 4 and 8 rows;
+    # int8 takes the packed 8-row kernel by default and 4 rows on request.
+    torch, _ = gpu
+    vec = 16 // np.dtype(dtype).itemsize
+    tiles = [wg * vec * r for r in (1, 4, 8)]
+    sizes = sorted({1, vec - 1 or 1, vec, vec + 1, 64 * vec - 1, 64 * vec + 1,
+                    *(t + d for t in tiles for d in (-1, 0, 1)), tiles[-1] + 64 * vec + 5})
+    pad = 40
+    top = sizes[-1]
+    x = rand(dtype, top + pad, seed=wg)
+    xd = dev(torch, x)
+    clean = dev(torch, np.full(top + 2 * pad, 77, dtype=dtype))
+    init = dtype(5)
+    rows = [0, 4] if dtype in (np.int8, np.uint8) else [0]
+    for n in sizes:
+        for i_off, o_off in ((0, 1), (1, 0), (2, 3), (3, 2), (1, 1), (13, 9)):
+            want = [O.inclusive_scan(x[i_off:i_off + n]), O.exclusive_scan(x[i_off:i_off + n], init),
+                    O.transform_inclusive_scan(x[i_off:i_off + n], O.MAX, O.ABS)]
+            xin = xd[i_off:i_off + n]
+            for r in rows:
+                cfg = (wg, r)
+                for k, run in enumerate((
+                        lambda a, b: acpp.inclusive_scan(q, scratch, a, b, config=cfg),
+                        lambda a, b: acpp.exclusive_scan(q, scratch, a, b, init, config=cfg),
+                        lambda a, b: acpp.transform_inclusive_scan(q, scratch, a, b, acpp.MAX, acpp.ABS, config=cfg))):
+                    lo = pad + o_off
+                    buf = clean.clone()
+                    run(xin, buf[lo:lo + n])
+                    place = clean.clone()
+                    place[lo:lo + n] = xin
+                    run(place[lo:lo + n], place[lo:lo + n])
+                    q.wait()
+                    for got in (host(buf), host(place)):
+                        assert np.array_equal(got[lo:lo + n], want[k]), (n, i_off, o_off, r, k)
+                        assert np.all(got[:lo] == 77) and np.all(got[lo + n:] == 77), (n, i_off, o_off, r, k)
+            scratch.release()
+    assert scratch.watchdog_trips() == 0
