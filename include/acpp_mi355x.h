@@ -364,7 +364,7 @@ acpp_status acpp_exclusive_scan_i32(acpp_allocation_group *scratch, acpp_stream_
 /* No counterpart in the reference.  acpp_exclusive_scan_i32 for callers
    that cannot allocate (code under hipGraph capture, tight serving loops,
    harnesses that forbid hipMalloc): no allocation group; the scan's sync
-   region (256-byte header + 2 MiB of tile status lines) is a static device
+   region (2304-byte header + 2 MiB of tile status lines) is a static device
    array of the library, one per GPU, set up on the first call on each
    device.  At most 16384 tiles (2^29 elements with the default 1024 x 8-row
    tiles); larger inputs are rejected with ACPP_ERROR_INVALID_ARGUMENT.

@@ -240,7 +240,7 @@ class AllocationGroup:
         SegmentedPlan made from this group is alive: it still
         uses them, and replays would corrupt whichever call got them next."""
         if self._plans > 0:
-            raise RuntimeError("AllocationGroup.release: a SegmentedPlan captured from this group is alive; "
+            raise RuntimeError("AllocationGroup.release: a SegmentedPlan made from this group is alive; "
                                "close the plan first")
         check(_abi.load().acpp_allocation_group_release(self._h))
 

@@ -192,13 +192,12 @@ acpp_status begin_region_launch_flag(uint32_t *trip_flag, void *region, size_t u
                                      region_state *rs, hipStream_t stream, region_launch *out);
 
 // A sync region handed to a launcher instead of one from an allocation
-// group.  The caller makes its device current and knows its CU count.
+// group.  The caller makes its device current.
 struct fixed_region {
   void *ptr;            // device address
   size_t capacity;      // bytes
   region_state *rs;
   uint32_t *trip_flag;  // host trip flag of the device, or NULL
-  int compute_units;
 };
 // Record the launch: `tickets` tile tickets drawn; a failed launch makes the
 // region start over next time (it may or may not have run).

@@ -22,25 +22,21 @@ static __device__ __align__(256) unsigned char scratch[noalloc_bytes];
 
 struct noalloc_device {
   void *ptr = nullptr;  // this device's address of `scratch` (never the host-side name)
-  int compute_units = 0;
   region_state rs;
 };
 constexpr int noalloc_max_devices = 64;
 std::mutex g_noalloc_mutex;  // host bookkeeping of the calls (epoch, ticket base)
 noalloc_device g_noalloc[noalloc_max_devices];
 
-// Once per device, with that device current: the array's device address and
-// the CU count.  The region starts in "graph" mode, so the first launch
-// clears it with a kernel before use.
+// Once per device, with that device current: the array's device address.  The
+// region starts in "graph" mode, so the first launch clears it with a kernel
+// before use.
 acpp_status noalloc_setup(int dev, noalloc_device **out) {
   noalloc_device &d = g_noalloc[dev];
   if (!d.ptr) {
     void *p = nullptr;
     ACPP_CHECK_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     if (!p) return set_error(ACPP_ERROR_HIP, "hipGetSymbolAddress(scratch) returned NULL");
-    int cus = 0;
-    ACPP_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    d.compute_units = cus;
     d.rs.mode = region_state::graph;
     d.ptr = p;
   }
@@ -78,7 +74,7 @@ acpp_status acpp_exclusive_scan_i32_noalloc(acpp_stream_t stream, const int32_t 
   noalloc_device *d = nullptr;
   acpp_status st = noalloc_setup(dev, &d);
   if (st != ACPP_SUCCESS) return st;
-  const fixed_region region{d->ptr, noalloc_bytes, &d->rs, host_trip_flag_if_allocated(dev), d->compute_units};
+  const fixed_region region{d->ptr, noalloc_bytes, &d->rs, host_trip_flag_if_allocated(dev)};
   return with_op<int32_t, int32_t>(op, [&](auto opv) -> acpp_status {
     using Op = decltype(opv);
     if (n == 0) return clear_error();  // decoupled_lookback_scan.hpp:565-566

@@ -10,11 +10,11 @@
 // MI355X design:
 //   - the concatenated elements are cut into equal tiles, independent of the
 //     segment lengths, so log-normal segment lengths cost no load imbalance;
-//   - a setup kernel builds the device work queue: for every tile the first
-//     segment it touches (each non-empty segment writes the tiles whose first
-//     element it contains), and writes init into empty segments' results;
-//   - persistent work-groups (one wave of resident groups) draw tiles from
-//     a ticket counter in order; every tile marks its segment starts in an
+//   - a tile finds the segments that start in it by a search of the offsets
+//     (few tiles), or from a bitmap of the starts (scans) or a table of every
+//     tile's first segment (reductions) that a kernel before it wrote;
+//   - scans: persistent work-groups (one wave of resident groups) draw tiles
+//     from a ticket counter in order; every tile puts its segment starts in an
 //     LDS bitmap and runs a segmented scan over (head flag, value) pairs:
 //     (f1,v1) . (f2,v2) = (f1|f2, f2 ? v2 : v1 op v2), in registers, across
 //     each wave with DPP and across waves through LDS;
@@ -24,8 +24,8 @@
 //     segment start (its aggregate already discards everything before it),
 //     so it is short whenever segments are shorter than a tile;
 //   - scans write every element.  Reductions skip the look-back: each tile
-//     writes the totals of the segments it holds whole and two partial
-//     folds, and a fix-up kernel joins the partials of segments that span
+//     writes the totals of the segments it holds whole (init for empty ones)
+//     and two partial folds, and a fix-up kernel joins the partials of segments that span
 //     tiles (segmented_reduce_kernel below);
 //   - a plan keeps a call's scratch and parameters (acpp_segmented_plan_*).
 #include <memory>
