@@ -1382,7 +1382,10 @@ __global__ __launch_bounds__(1024) void segmented_fixup_kernel(params<T> p,
 //           in 1000 segments 46.3 and 42.1 us, in 48 40.5 and 42.8 us, in
 //           20000 42.4 and 51.6 us), and 512 x 2 from 320 MiB with at most one
 //           per 2^14 (204M int32 in 300 segments 137.0 and 130.0 us, in 3977
-//           140.1 and 134.7 us, in 100,000 139.0 and 158.1 us)
+//           140.1 and 134.7 us, in 100,000 139.0 and 158.1 us), 256 x 2 there
+//           up to one per 2^12 (120M int32 in 20,000 segments 87.7 and 84.7 us,
+//           300M int32 in 30,000 202.1 and 195.3 us, 150M fp64 in 15,000 207.5
+//           and 199.4 us; 204M int32 in 60,000 137.3 and 142.8 us)
 // 2-row scans of up to max_search_tiles tiles and reductions of as many
 // tiles need one launch less, so the tiles grow with the input as long as
 // they stay below that (2^20 fp32 scan: 8.5 us at 1024 x 2, 11.6 us at 512 x
@@ -1404,8 +1407,8 @@ inline void default_tile(bool reduce, uint64_t total, uint64_t num_segments, int
     rows = mib < 20 ? 2 : 4;
     wg = mib < 48 ? 1024 : (wide ? 512 : 256);
     const bool few = num_segments <= total >> 14;
-    if (mib >= 320 && few) {
-      wg = 512;
+    if (mib >= 320 && num_segments <= total >> 12) {
+      wg = few ? 512 : 256;
       rows = 2;
     } else if (mib >= 48 && few && num_segments >= total >> 17) {
       wg = 1024;

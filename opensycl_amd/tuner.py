@@ -63,11 +63,10 @@ def default_config(kind: str, n: int, dtype: str = "i32", segments: int | None =
     if kind == "reduce":
         if mib < 48:
             return (1024, 2) if mib < 20 else (1024, 4)
-        if segments is not None and segments <= n >> 14:
-            if mib >= 320:
-                return (512, 2)
-            if segments >= n >> 17:
-                return (1024, 4)
+        if segments is not None and mib >= 320 and segments <= n >> 12:
+            return (512, 2) if segments <= n >> 14 else (256, 2)
+        if segments is not None and n >> 17 <= segments <= n >> 14:
+            return (1024, 4)
         return (512, 4) if width == 8 else (256, 4)
     if mib < 64:
         return (1024, 2) if mib < 12 else (1024, 4)

@@ -119,10 +119,13 @@ def test_library_default_rule_on_committed_timings():
 def test_library_default_rule_by_segment_count():
     # reductions of few segments have tiles of their own (default_tile)
     assert T.default_config("reduce", 204_000_000, "i32", segments=300) == (512, 2)
-    assert T.default_config("reduce", 204_000_000, "i32", segments=100_000) == (256, 4)
+    assert T.default_config("reduce", 204_000_000, "i32", segments=40_000) == (256, 2)
+    assert T.default_config("reduce", 204_000_000, "i32", segments=60_000) == (256, 4)
     assert T.default_config("reduce", 60_000_000, "i32", segments=1000) == (1024, 4)
     assert T.default_config("reduce", 60_000_000, "i32", segments=48) == (256, 4)
     assert T.default_config("reduce", 60_000_000, "i32", segments=20_000) == (256, 4)
+    assert T.default_config("reduce", 120_000_000, "i32", segments=20_000) == (256, 2)
+    assert T.default_config("reduce", 60_000_000, "f64", segments=5000) == (256, 2)
     assert T.default_config("reduce", 30_000_000, "f64", segments=1000) == (1024, 4)
     # and the regret of the default is that of the tile that the library launches
     times = {T._key(c): 100.0 for c in T.CONFIGS}
