@@ -644,7 +644,10 @@ class SegmentedPlan:
     The plan holds raw pointers to the input, output and offsets
     tensors and to scratch regions of the allocation group, so the plan
     keeps references to all of them (and to the group's cache) for as long
-    as it lives: a replay never touches freed or reissued memory."""
+    as it lives: a launch never touches freed or reissued memory.  Launches
+    of one plan share that scratch: they have to be ordered on the device
+    (one stream, or events between streams); launches that may overlap need
+    plans of their own."""
 
     def __init__(self, handle, scratch, keep=()):
         self._h = handle
