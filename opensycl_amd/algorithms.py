@@ -159,6 +159,7 @@ class AllocationCache:
         h = ctypes.c_void_p()
         check(lib.acpp_allocation_cache_create(allocation_type, ctypes.byref(h)))
         self._h = h
+        self._owned = [h]        # until it is destroyed
         self._groups: dict = {}  # device -> handles of closed (empty) groups, for new ones
         self._alive: dict = {}   # the library's groups on this cache, open or in _groups
         self._closing = False
@@ -187,9 +188,14 @@ class AllocationCache:
         return st
 
     def _destroy(self) -> None:
-        if self._h and not self._alive:
-            h, self._h = self._h, None
-            check(_abi.load().acpp_allocation_cache_destroy(h))
+        if self._alive:
+            return
+        try:
+            h = self._owned.pop()  # (one step: two threads may close the last two groups)
+        except IndexError:
+            return
+        self._h = None
+        check(_abi.load().acpp_allocation_cache_destroy(h))
 
     def close(self) -> None:
         """Free the cache.  Groups that are still open return their regions to

@@ -175,3 +175,21 @@ def test_purge_beside_a_thread_that_takes_the_last_handle():
     cache.purge()
     cache._groups[0] = []
     cache.close()
+
+
+def test_last_groups_closed_by_two_threads_destroy_the_cache_once(monkeypatch):
+    class Raced(dict):  # another thread is through between a look at it and what follows
+        def __len__(self):
+            if not self.seen:
+                self.seen = True
+                cache._destroy()
+            return 0
+
+    cache = acpp.AllocationCache()
+    names = []
+    lib = algorithms._abi.load()
+    monkeypatch.setattr(algorithms._abi, "load", lambda: _Log(lib, names))
+    cache._alive = Raced()
+    cache._alive.seen = False
+    cache.close()
+    assert names.count("acpp_allocation_cache_destroy") == 1
