@@ -352,3 +352,56 @@ def test_captured_histogram_takes_cached_partials(gpu, q, num_bins, n, warm):
     del graph
     scratch.close()
     cache.close()
+
+
+class _Dim3(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_uint), ("y", ctypes.c_uint), ("z", ctypes.c_uint)]
+
+
+class _KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", _Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", _Dim3),
+                ("args", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+
+def _first_kernel(graph):
+    hip = ctypes.CDLL("libamdhip64.so")
+    g, count = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(8)
+    nodes = (ctypes.c_void_p * 8)()
+    assert hip.hipGraphGetNodes(g, nodes, ctypes.byref(count)) == 0 and count.value >= 1
+    params = _KernelNode()
+    assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(nodes[0]), ctypes.byref(params)) == 0
+    return params
+
+
+@pytest.mark.parametrize("num_bins, n, wg, lds, block, most_groups", [
+    (65537, 2048, 0, False, None, None),    # few keys, more bins than one LDS: one atomic per key
+    (1 << 22, 4096, 0, False, None, None),
+    (200000, 4097, 0, True, 1024, None),    # slices from here on
+    (65537, 2049, 0, True, 1024, None),
+    (300000, 1000, 64, False, 64, None),
+    (60000, 100000, 256, True, 256, None),
+])
+def test_histogram_forms(gpu, num_bins, n, wg, lds, block, most_groups):
+    torch, _ = gpu
+    keys = rand(np.uint32, n, seed=n) % np.uint32(num_bins + 3)
+    kd = dev(torch, keys)
+    bins = torch.zeros(num_bins, dtype=torch.int32, device="cuda").view(torch.uint32)
+    cache = acpp.AllocationCache()
+    scratch = acpp.AllocationGroup(cache)
+    s = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=s):
+        acpp.histogram(acpp.Queue(), scratch, kd, bins, config={"work_group_size": wg} if wg else None)
+    kernel = _first_kernel(graph)
+    assert (kernel.lds > 0) == lds
+    if block:
+        assert kernel.block.x == block
+    if most_groups:
+        assert kernel.grid.x in (most_groups * block, most_groups)  # in work-items or work-groups
+    graph.instantiate()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert np.array_equal(host(bins), O.histogram(keys, num_bins))
+    del graph
+    scratch.close()
+    cache.close()
