@@ -542,7 +542,9 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
   if (strat == strat_privatized && !fits16)
     return set_error(ACPP_ERROR_UNSUPPORTED,
                      "acpp_histogram_u32: more than 65536 bins do not fit the LDS; use the global strategy");
-  // More bins than one LDS holds are cut into slices.  Every slice visits
+  // More bins than one LDS holds are cut into slices, always by 1024-wide groups
+  // (128 KiB of counters to clear and to flush: 2M keys into 2.5M bins 610 us
+  // 64 wide).  Every slice visits
   // every key, so beyond max_slices one atomic per key is the better form.
   uint32_t slices_log2 = 0;
   while (!fits16 && slices_log2 < max_slices_log2 && ceil_div(num_bins, 1ull << slices_log2) > max_local_bins) ++slices_log2;
@@ -554,9 +556,10 @@ acpp_status histogram(acpp_allocation_group *g, hipStream_t stream, const uint32
   // in one bin, 2000 keys 30 us and 11 us).
   const bool few_keys = n <= 2048 || (n <= 4096 && num_bins > 2 * max_local_bins);
   if (strat == strat_auto) strat = (fits16 || (sliceable && !few_keys)) ? strat_privatized : strat_global;
-  const uint32_t wg = (cfg && cfg->work_group_size) ? cfg->work_group_size : 1024;
-  if (!valid_work_group_size(wg))
+  const uint32_t wg_given = (cfg && cfg->work_group_size) ? cfg->work_group_size : 1024;
+  if (!valid_work_group_size(wg_given))
     return set_error(ACPP_ERROR_INVALID_ARGUMENT, "acpp_histogram_u32: bad work_group_size");
+  const uint32_t wg = !fits16 && strat == strat_privatized ? 1024 : wg_given;
   const geom gm = make_geom(keys, n);
 
   if (strat == strat_global) {

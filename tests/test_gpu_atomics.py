@@ -378,6 +378,7 @@ def _first_kernel(graph):
     (1 << 22, 4096, 0, False, None, None),
     (200000, 4097, 0, True, 1024, None),    # slices from here on
     (65537, 2049, 0, True, 1024, None),
+    (300000, 100000, 64, True, 1024, None),  # slices are 1024 wide whatever is asked for
     (300000, 1000, 64, False, 64, None),
     (60000, 100000, 256, True, 256, None),
 ])
