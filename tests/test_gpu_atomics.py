@@ -381,6 +381,9 @@ def _first_kernel(graph):
     (300000, 100000, 64, True, 1024, None),  # slices are 1024 wide whatever is asked for
     (300000, 1000, 64, False, 64, None),
     (60000, 100000, 256, True, 256, None),
+    (150, 1_000_000, 0, True, 1024, 96),    # few bins: no more groups than flush in the time of the keys
+    (150, 300_000, 0, True, 1024, 74),
+    (8192, 3_000_000, 0, True, 1024, 245),
 ])
 def test_histogram_forms(gpu, num_bins, n, wg, lds, block, most_groups):
     torch, _ = gpu
