@@ -409,3 +409,21 @@ def test_histogram_forms(gpu, num_bins, n, wg, lds, block, most_groups):
     del graph
     scratch.close()
     cache.close()
+
+
+@pytest.mark.parametrize("num_bins", [8193, 9000, 12000, 20001, 32767, 32768, 32769, 40001, 65535, 65536, 65537, 200001])
+@pytest.mark.parametrize("wg", [0, 64, 192])
+def test_histogram_flushes_in_many_rounds(gpu, q, scratch, num_bins, wg):
+    # few keys straight to the bins, several words a round; every bin is hit
+    # and those next to the end are not
+    torch, _ = gpu
+    rng = np.random.default_rng(num_bins)
+    for n in (1, 5000, num_bins + 1, 130000):
+        keys = np.concatenate([np.arange(num_bins - 1, -1, -1), rng.integers(0, num_bins + 2, n)])[:n].astype(np.uint32)
+        bins = torch.full((num_bins + 64,), 9, dtype=torch.int32, device="cuda").view(torch.uint32)
+        acpp.histogram(q, scratch, dev(torch, keys), bins[:num_bins],
+                       config={"work_group_size": wg} if wg else None)
+        q.wait()
+        got = host(bins)
+        assert np.array_equal(got[:num_bins], O.histogram(keys, num_bins) + np.uint32(9)), n
+        assert np.all(got[num_bins:] == 9), n
