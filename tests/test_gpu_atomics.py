@@ -427,3 +427,33 @@ def test_histogram_flushes_in_many_rounds(gpu, q, scratch, num_bins, wg):
         got = host(bins)
         assert np.array_equal(got[:num_bins], O.histogram(keys, num_bins) + np.uint32(9)), n
         assert np.all(got[num_bins:] == 9), n
+
+
+@pytest.mark.parametrize("dtype, num_slots, wg, n, groups", [
+    (np.float64, 35982, 0, 2_000_000, 564),   # 282 strips on 256 CUs: two groups each
+    (np.float64, 35982, 0, 100_000, 71),      # a row and a bit, in wider strips
+    (np.int64, 200, 64, 8_000_000, 2040),     # eight narrow groups a CU
+    (np.int32, 200, 64, 8_000_000, 504),
+    (np.int64, 200, 512, 8_000_000, 250),
+])
+def test_strided_groups(gpu, dtype, num_slots, wg, n, groups):
+    torch, _ = gpu
+    v = rand(dtype, n, seed=n, lo=-1000, hi=1000) if np.issubdtype(dtype, np.integer) else \
+        np.round(rand(np.float64, n, seed=n) * 100)
+    vd = dev(torch, v)
+    t = dev(torch, np.full(num_slots, 3, dtype=dtype))
+    cache = acpp.AllocationCache()
+    scratch = acpp.AllocationGroup(cache)
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        acpp.atomic_fetch_strided(acpp.Queue(), scratch, "max", vd, t, config={"work_group_size": wg} if wg else None)
+    assert _first_kernel(graph).grid.x == groups
+    graph.instantiate()
+    graph.replay()
+    torch.cuda.synchronize()
+    exp = np.full(num_slots, 3, dtype=dtype)
+    np.maximum.at(exp, np.arange(n) % num_slots, v)
+    assert np.array_equal(host(t), exp)
+    del graph
+    scratch.close()
+    cache.close()
