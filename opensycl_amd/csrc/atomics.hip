@@ -371,7 +371,12 @@ __device__ __forceinline__ void cas_select(T *p, T v, Cmp keep_old) {
 template <class T>
 struct rmw_min {
   __device__ static T identity() { return ops::minimum<T, T>::identity(); }
-  __device__ static T apply(T a, T b) { return (a < b || a != a) ? a : b; }
+  __device__ static T apply(T a, T b) {
+    if constexpr (std::is_floating_point_v<T>)
+      return __builtin_elementwise_minimum(a, b);  // a NaN if either is
+    else
+      return ops::minimum<T, T>::apply(a, b);
+  }
   template <int Scope>
   __device__ static void atomic(T *p, T v) {
     if constexpr (std::is_floating_point_v<T>)
@@ -384,7 +389,12 @@ struct rmw_min {
 template <class T>
 struct rmw_max {
   __device__ static T identity() { return ops::maximum<T, T>::identity(); }
-  __device__ static T apply(T a, T b) { return (a > b || a != a) ? a : b; }
+  __device__ static T apply(T a, T b) {
+    if constexpr (std::is_floating_point_v<T>)
+      return __builtin_elementwise_maximum(a, b);
+    else
+      return ops::maximum<T, T>::apply(a, b);
+  }
   template <int Scope>
   __device__ static void atomic(T *p, T v) {
     if constexpr (std::is_floating_point_v<T>)
