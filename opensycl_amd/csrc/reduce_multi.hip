@@ -4,16 +4,15 @@
 // one parallel_for).
 //
 // One launch reduces up to four inputs of the same length, each with its
-// own operator and output: every work-group streams the distinct inputs one
-// after the other (16-byte loads, the operator switch outside the streaming
-// loop) and folds an array that several reductions share once for all of
-// them, with one uniform switch per operator and batch of loads.  It reduces
-// all values with DPP and one LDS exchange and publishes one partial per
-// reduction; the last work-group to finish (fence-free ticket, as in
-// reduce_common.hpp) folds all partials in a fixed order and writes the
-// results.  (An array shared by three reductions was streamed three times:
-// 2^28 fp32 460 us, now 160 us; arrays off 16-byte alignment went element
-// by element: 2573 us, now 159 us.)
+// own operator and output.  Every work-group streams the inputs one after the
+// other (16-byte loads, the operator switch outside the streaming loop), reduces
+// each with DPP and one LDS exchange and publishes one partial per reduction; the
+// last work-group to finish (fence-free ticket, as in reduce_common.hpp) folds
+// all partials in a fixed order and writes the results.  A large array that
+// several reductions share is read once and folded for all of them, with one
+// uniform switch per operator and batch of loads (2^28 fp32 in three reductions
+// 460 us one by one, 160 us so; arrays off 16-byte alignment went element by
+// element: 2573 us, now 159 us).
 #include "launch_util.hpp"
 #include "reduce_common.hpp"
 
@@ -235,21 +234,68 @@ __device__ void group_reduce(int waves, const params<T> &p, typename elem_traits
     });
 }
 
-// SHARED: several reductions read one array.
-template <class T, bool NT, bool SHARED>
+// Writes the result of reduction m, whose whole fold is r.
+template <class T, class Op>
+__device__ __forceinline__ void finish(const params<T> &p, int m, typename elem_traits<T>::work r) {
+  if (p.init_mode[m] == 0) r = Op::apply(elem_traits<T>::to_work(*p.out[m]), r);
+  else if (p.init_mode[m] == 2) r = Op::apply(p.identity[m], r);
+  *p.out[m] = static_cast<T>(r);
+}
+
+// One reduction after the other.  The loop stays a loop: a short call spends
+// its time fetching instructions (1000 int32 in two reductions 5.6 us, 6.5 us
+// with the code of shared_kernel, which has a copy for each reduction).
+template <class T, bool NT>
 __global__ __launch_bounds__(1024) void multi_kernel(params<T> p) {
+  using W = typename elem_traits<T>::work;
+  __shared__ W s_waves[max_waves];
+  __shared__ bool s_last;
+  const bool force = p.force_give_up != 0;
+  const bool alone = gridDim.x == 1 && !force;  // nothing to exchange
+  for (int k = 0; k < p.count; ++k) {
+    __syncthreads();  // s_waves of the previous reduction has been read
+    dispatch<W>(p.op[k], [&](auto opv) {
+      using Op = decltype(opv);
+      W v = stream_fold<T, Op, NT>(p.in[k], p.n);
+      v = reduce_detail::block_reduce<reduce_detail::plain_monoid<W, Op>>(v, s_waves);
+      if (threadIdx.x == 0) {
+        if (alone)
+          finish<T, Op>(p, k, v);
+        else
+          publish_partial(p.partials, static_cast<uint64_t>(k) * gridDim.x + blockIdx.x, p.epoch, v);
+      }
+    });
+  }
+  if (alone) return;
+  if (threadIdx.x == 0) s_last = reduce_detail::draw_last_ticket(p.sync);  // (the last group waits for each partial's tag)
+  __syncthreads();
+  if (!s_last) return;
+  for (int k = 0; k < p.count; ++k) {
+    __syncthreads();
+    dispatch<W>(p.op[k], [&](auto opv) {
+      using Op = decltype(opv);
+      W r = Op::identity();
+      for (uint32_t i = threadIdx.x; i < gridDim.x; i += blockDim.x)
+        r = Op::apply(r, wait_partial<W>(p.partials, static_cast<uint64_t>(k) * gridDim.x + i, p.epoch, p.sync, force,
+                                         Op::identity()));
+      r = reduce_detail::block_reduce<reduce_detail::plain_monoid<W, Op>>(r, s_waves);
+      if (threadIdx.x == 0) finish<T, Op>(p, k, r);
+    });
+  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&p.sync->done_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Large arrays that several reductions share are read once.
+template <class T, bool NT>
+__global__ __launch_bounds__(1024) void shared_kernel(params<T> p) {
   using W = typename elem_traits<T>::work;
   __shared__ W s_waves[max_inputs][max_waves];
   __shared__ bool s_last;
   W v[max_inputs];
 #pragma unroll
-  for (int k = 0; k < max_inputs; ++k) {
-    if (k >= p.count || p.first[k] != k) continue;
-    if constexpr (SHARED)
-      shared_fold<T, NT>(p, k, v);
-    else
-      dispatch<W>(p.op[k], [&](auto opv) { v[k] = stream_fold<T, decltype(opv), NT>(p.in[k], p.n); });
-  }
+  for (int k = 0; k < max_inputs; ++k)
+    if (k < p.count && p.first[k] == k) shared_fold<T, NT>(p, k, v);
   group_reduce(blockDim.x >> 6, p, v, s_waves, [&](int m, W x) {
     publish_partial(p.partials, static_cast<uint64_t>(m) * gridDim.x + blockIdx.x, p.epoch, x);
   });
@@ -271,14 +317,8 @@ __global__ __launch_bounds__(1024) void multi_kernel(params<T> p) {
                                            p.force_give_up != 0, Op::identity()));
         v[k] = r;
       });
-  group_reduce(1, p, v, s_waves, [&](int m, W r) {
-    dispatch<W>(p.op[m], [&](auto opv) {
-      using Op = decltype(opv);
-      if (p.init_mode[m] == 0) r = Op::apply(elem_traits<T>::to_work(*p.out[m]), r);
-      else if (p.init_mode[m] == 2) r = Op::apply(p.identity[m], r);
-      *p.out[m] = static_cast<T>(r);
-    });
-  });
+  group_reduce(1, p, v, s_waves,
+               [&](int m, W r) { dispatch<W>(p.op[m], [&](auto opv) { finish<T, decltype(opv)>(p, m, r); }); });
   if (threadIdx.x == 0)
     __hip_atomic_store(&p.sync->done_counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -352,8 +392,14 @@ acpp_status entry(acpp_allocation_group *g, hipStream_t stream, uint32_t count, 
   // Non-temporal loads once the inputs are larger than the 256 MiB
   // last-level cache, as for the plain reductions.
   const bool nt = static_cast<uint64_t>(arrays) * n * sizeof(T) >= (256ull << 20);
-  auto kernel = arrays < count ? (nt ? multi_kernel<T, true, true> : multi_kernel<T, false, true>)
-                               : (nt ? multi_kernel<T, true, false> : multi_kernel<T, false, false>);
+  // Arrays that the last-level cache holds are read again sooner than folded for
+  // all at once (int64 in three reductions, 32 MB 15.8 and 17.4 us, 400 MB 169
+  // and 77 us; int32 in two, 4 MB 8.2 and 9.0 us, 200 MB 57 and 37 us), and the
+  // fold of 1-byte elements costs more than a second read (2^28 int8 in two 82
+  // and 90 us, in four 165 and 144 us).
+  const bool shared = arrays < count && n * sizeof(T) >= (48ull << 20) && (sizeof(T) > 1 || count - arrays >= 2);
+  auto kernel = shared ? (nt ? shared_kernel<T, true> : shared_kernel<T, false>)
+                       : (nt ? multi_kernel<T, true> : multi_kernel<T, false>);
   int resident = 1;
   st = occupancy(kernel, static_cast<int>(wg), &resident);
   if (st != ACPP_SUCCESS) return st;

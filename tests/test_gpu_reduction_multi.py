@@ -137,3 +137,30 @@ def test_shared_arrays(gpu, q, scratch, dtype, offset):
                 x = (a, b)[i][offset:].astype(np.int64)
                 exp = {acpp.PLUS: x.sum(), acpp.MIN: x.min(), acpp.MAX: x.max()}[op]
                 assert host(out)[0] == np.array(exp).astype(dtype), (n, pick, op)
+
+
+@pytest.mark.parametrize("dtype", ["int8", "int16", "int32", "int64", "float32", "float64"])
+@pytest.mark.parametrize("more", [-1, 0, 1, 12345])
+def test_shared_arrays_around_the_size_that_reads_them_once(gpu, q, scratch, dtype, more):
+    # below 48 MiB every reduction reads the array, from there one pass folds it
+    # for all of them (1-byte elements: for three and more)
+    torch, _ = gpu
+    dt = getattr(torch, dtype)
+    n = (48 << 20) // torch.empty(0, dtype=dt).element_size() + more
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    ops = (acpp.PLUS, acpp.MIN, acpp.MAX, acpp.PLUS)
+    for offset in (0, 1):
+        # integer-valued: float sums are exact
+        a, b = (torch.randint(-50, 50, (n + offset,), device="cuda", generator=gen, dtype=torch.int8) for _ in range(2))
+        ad, bd = a.to(dt)[offset:], b.to(dt)[offset:]
+        want = [(x.sum(dtype=torch.int64), x.min(), x.max()) for x in (a[offset:], b[offset:])]
+        for pick in ((0, 0), (0, 1, 0), (0, 0, 0), (1, 1, 0, 0), (0, 1, 1, 1)):
+            ins = [(ad, bd)[i] for i in pick]
+            outs = [torch.zeros(1, dtype=dt, device="cuda") for _ in pick]
+            acpp.reduction_multi(q, scratch, ins, outs, ops[:len(pick)], True)
+            q.wait()
+            scratch.release()
+            for i, op, out in zip(pick, ops, outs):
+                exp = want[i][{acpp.PLUS: 0, acpp.MIN: 1, acpp.MAX: 2}[op]]
+                assert out[0] == exp.to(dt), (pick, op, offset)
