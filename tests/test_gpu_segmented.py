@@ -486,3 +486,19 @@ def test_runs_of_empty_segments_cost_what_spread_ones_cost(gpu, q, scratch, kind
             samples.append(a.elapsed_time(b))
         times.append(min(samples))
     assert times[1] < 5 * times[0], times
+
+
+@pytest.mark.parametrize("wg", [64, 128, 192, 512, 960, 1024])
+@pytest.mark.parametrize("n", [(1 << 20) - 1, 1 << 20, 4_000_001])
+def test_segmented_scan_with_a_width_alone(gpu, q, scratch, wg, n):
+    # the rows then follow the width: the default tile's size, up to 8 rows
+    torch, _ = gpu
+    rng = np.random.default_rng(wg)
+    off = np.concatenate([[0], np.sort(rng.integers(0, n, 3000)), [n]]).astype(np.uint64)
+    xi = exact_ints(torch, n, wg)
+    xh = host(xi).astype(np.int64)
+    for dt in (torch.int32, torch.float64):
+        yd = torch.zeros(n, dtype=dt, device="cuda")
+        acpp.segmented_inclusive_scan(q, scratch, xi.to(dt), yd, dev(torch, off), config={"work_group_size": wg})
+        q.wait()
+        assert np.array_equal(host(yd).astype(np.int64), O.segmented_inclusive_scan(xh, off)), dt
