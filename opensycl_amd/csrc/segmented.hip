@@ -322,6 +322,14 @@ struct tile_starts {
   }
 
   __device__ __forceinline__ void search(uint32_t count) {
+    if (b1 - b0 <= 2) {  // a few rounds of the whole wave each
+      bound = count;
+      for (uint32_t k = 0; k <= b1 - b0; ++k) {
+        const uint32_t x = static_cast<uint32_t>(wave_lower_bound(starts, count, base + (b0 + k) * 64ull));
+        if ((threadIdx.x & 63) == k) bound = x;
+      }
+      return;
+    }
     const uint64_t key = base + (b0 + (threadIdx.x & 63)) * 64ull;
     uint32_t l = 0, h = count;
     while (l < h) {
@@ -344,15 +352,35 @@ struct tile_starts {
       const uint32_t last = wave::read_lane(bound, static_cast<int>(b - b0) + 1);
       if (last <= first) continue;
       const uint32_t e = b * 64 + (threadIdx.x & 63);
-      uint32_t l = first, h = last;
-      while (l < h) {
-        const uint32_t mid = l + (h - l) / 2;
-        if (starts[mid] <= base + e)
-          l = mid + 1;
-        else
-          h = mid;
+      // Runs: from one start to the next other one by searches of the whole
+      // wave, up to four of them; all starts of the block by lane if more.
+      uint32_t pos = first, at = 0;
+      bool found = false;
+      if (last - first > 64) {
+        for (int hop = 0; hop < 4 && pos < last; ++hop) {
+          const uint64_t key = starts[pos];
+          const uint32_t rest = static_cast<uint32_t>(
+              wave_partition_point(last - pos, [&](uint64_t i) { return starts[pos + i] <= key; }));
+          pos += rest ? rest : 1;
+          if (base + e == key) {
+            found = e < in_range;
+            at = pos - 1;
+          }
+        }
       }
-      f(e, l - 1, e < in_range && l > first && starts[l - 1] == base + e);
+      if (pos < last) {
+        uint32_t l = first, h = last;
+        while (l < h) {
+          const uint32_t mid = l + (h - l) / 2;
+          if (starts[mid] <= base + e)
+            l = mid + 1;
+          else
+            h = mid;
+        }
+        at = l - 1;
+        found = e < in_range && l > first && starts[l - 1] == base + e;
+      }
+      f(e, at, found);
     }
   }
 
@@ -516,7 +544,21 @@ __global__ __launch_bounds__(256) void head_bitmap_kernel(const uint64_t *__rest
   for (uint64_t i = i0 + tid; i < i1; i += 256) mark(offsets[i]);
   __syncthreads();
   if (s_deep) {
-    if (tid < 32) {
+    // From the word's first start to its next other one, by searches of a whole
+    // wave (a binary search by bit: 18 us for a run of 200,000), unless there
+    // are more than four.
+    if (tid < 64) {
+      uint64_t pos = wave_lower_bound(offsets, i0, base);
+      for (int hop = 0; hop < 4 && pos < i0; ++hop) {
+        const uint64_t key = offsets[pos];
+        const uint64_t rest = wave_partition_point(i0 - pos, [&](uint64_t i) { return offsets[pos + i] <= key; });
+        pos += rest ? rest : 1;
+        if (tid == 0 && key >= base && key - base < 32 && key < total) atomicOr(&s_words[0], 1u << (key - base));
+      }
+      if (tid == 0) s_start[0] = pos;
+    }
+    __syncthreads();
+    if (s_start[0] < i0 && tid < 32) {
       const uint64_t key = base + tid;
       uint64_t lo = 0, hi = i0;
       while (lo < hi) {

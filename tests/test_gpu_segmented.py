@@ -456,6 +456,28 @@ def test_runs_of_empty_segments_tile_sizes(gpu, q, scratch, cfg):
     assert np.array_equal(host(out).astype(np.int64), O.segmented_reduce(xh, off, np.int64(3)))
 
 
+@pytest.mark.parametrize("starts", [[40], [0, 63], [1, 31, 32], [0, 1, 33, 63], [2, 3, 31, 32, 62], list(range(64))])
+def test_runs_of_empty_segments_in_one_block(gpu, q, scratch, starts):
+    # as many distinct starts as are found one after the other, and more, in 64
+    # elements: at the input's front, inside a tile, and in front of its end
+    torch, _ = gpu
+    for n in (64, 5000, 70016, 1 << 20):
+        for block in sorted({0, (n // 3) & ~63, n - 64}):
+            for spare in ([], np.arange(0, n, 3)):
+                pos = np.concatenate([np.repeat(block + np.array(starts), 20000), spare, [0, n]])
+                off = np.sort(pos).astype(np.uint64)
+                xi = exact_ints(torch, n, block)
+                xh = host(xi).astype(np.int64)
+                yd = torch.zeros_like(xi)
+                out = torch.full((len(off) - 1,), -7, dtype=xi.dtype, device="cuda")
+                acpp.segmented_inclusive_scan(q, scratch, xi, yd, dev(torch, off))
+                acpp.segmented_reduce(q, scratch, xi, dev(torch, off), out, 3)
+                q.wait()
+                assert np.array_equal(host(yd).astype(np.int64), O.segmented_inclusive_scan(xh, off)), (n, block)
+                assert np.array_equal(host(out).astype(np.int64), O.segmented_reduce(xh, off, np.int64(3))), (n, block)
+                scratch.release()
+
+
 @pytest.mark.parametrize("kind", ["scan", "reduce"])
 @pytest.mark.parametrize("n", [1 << 20, 1 << 23])
 def test_runs_of_empty_segments_cost_what_spread_ones_cost(gpu, q, scratch, kind, n):
