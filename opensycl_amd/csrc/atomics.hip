@@ -808,12 +808,15 @@ acpp_status strided(acpp_allocation_group *g, hipStream_t stream, const T *value
     const uint64_t strips = ceil_div(used_columns, 1ull << p.width_log2);
     const uint64_t band_rows = wg >> p.width_log2;
     // One group per CU, but as many as keep its loads going where the groups
-    // are narrower than the default (26M int64 max into 200 slots, 64 wide: 123
-    // us with one, 51 us with eight; int32 sums flush more than they gain).
+    // are narrower than the default: 576 work-items and six groups, 128
+    // work-items where the cache holds the input and the flushes count more
+    // (int32 into 67 slots: 100M 192 wide 122 us with one group, 76 with two, 72
+    // with three, 26M 23, 28 and 32; 47M 64 wide 124 us with one, 67 with two,
+    // 62 with six, 72 with eight.  int64: 47M 192 wide 113 us with one, 69 with
+    // three, 8M 18 and 30).
     const bool groups_given = cfg && cfg->groups_per_cu;
     const uint32_t per_cu = groups_given ? cfg->groups_per_cu
-                            : sizeof(T) == 8 ? std::max(1u, 512u / wg)
-                                             : std::max(1u, 128u / wg);
+                                         : std::max(1u, large ? std::min(6u, 576u / wg) : 128u / wg);
     const uint64_t cap_groups = static_cast<uint64_t>(cus) * per_cu;
     const uint64_t wanted = std::min(cap_groups, std::max<uint64_t>(1, ceil_div(p.gm.nvec, static_cast<uint64_t>(wg) * 4)));
     const uint64_t bands = std::max<uint64_t>(1, ceil_div(rows, band_rows));

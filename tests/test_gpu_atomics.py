@@ -432,7 +432,9 @@ def test_histogram_flushes_in_many_rounds(gpu, q, scratch, num_bins, wg):
 @pytest.mark.parametrize("dtype, num_slots, wg, n, groups", [
     (np.float64, 35982, 0, 2_000_000, 564),   # 282 strips on 256 CUs: two groups each
     (np.float64, 35982, 0, 100_000, 71),      # a row and a bit, in wider strips
-    (np.int64, 200, 64, 8_000_000, 2040),     # eight narrow groups a CU
+    (np.int64, 200, 64, 8_000_000, 510),      # two narrow groups a CU
+    (np.int64, 200, 64, 24_000_000, 1530),    # six: the cache does not hold the input
+    (np.int32, 4096, 192, 42_000_000, 768),
     (np.int32, 200, 64, 8_000_000, 504),
     (np.int64, 200, 512, 8_000_000, 250),
 ])
