@@ -297,6 +297,7 @@ def segmented_leg(acpp, q, cache, per_segment=True):
         plan = acpp.SegmentedPlan.inclusive_scan(g, xs, ys, off)
         plan.launch(q)
         graph_avg, graph_min = timed(q, lambda: plan.launch(q), 10)
+        log("segmented scan: plan timed")
 
         with acpp.AllocationGroup(cache, 0) as g2:
             def direct2():
@@ -304,6 +305,7 @@ def segmented_leg(acpp, q, cache, per_segment=True):
             direct2()
             g2.release()
             direct_avg, _ = timed(q, direct2, 10, release=g2.release)
+        log("segmented scan: direct call timed")
 
         def per_segment_s():
             st = bench_lib.acpp_bench_per_segment_inclusive_scan_i64(
@@ -313,6 +315,7 @@ def segmented_leg(acpp, q, cache, per_segment=True):
         if per_segment:
             per_segment_s()
             per_avg, _ = timed(q, per_segment_s, 2)
+            log("segmented scan: one call per segment timed")
         else:
             per_avg = float("nan")
         plan.launch(q)
@@ -343,6 +346,7 @@ def segmented_leg(acpp, q, cache, per_segment=True):
         if per_segment:
             per_segment_r()
             per_avg, _ = timed(q, per_segment_r, 2)
+            log("segmented reduction: plan and one call per segment timed")
         else:
             per_avg = float("nan")
         plan.launch(q)
@@ -355,6 +359,7 @@ def segmented_leg(acpp, q, cache, per_segment=True):
         abs64.index_add_(0, seg_id, xf.double().abs())
         err = ((rs.double() - exact64).abs() / abs64.clamp_min(1e-30)).max().item()
         err_ref = ((rref.double() - exact64).abs() / abs64.clamp_min(1e-30)).max().item() if per_segment else None
+        log("segmented reduction: checked against fp64 sums")
         b_red = 4 * T + 8 * (S + 1) + 4 * S
         out["reduce_f32"] = {
             "batched_graph_us": round(graph_avg, 1), "batched_graph_min_us": round(graph_min, 1),
